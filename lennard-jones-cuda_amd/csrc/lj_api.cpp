@@ -60,7 +60,11 @@ void drop_graph(lj_ctx* c)
 }
 
 // rows of one of the two block-row buffers
-size_t blk_rows(const lj_ctx* c) { return (size_t)std::max(c->nblk, step_rows(c->cfg.N)); }
+size_t blk_rows(const lj_ctx* c)
+{
+  const int small = c->small_T ? (c->cfg.N + c->small_T - 1) / c->small_T : 0;
+  return (size_t)std::max({c->nblk, step_rows(c->cfg.N), small});
+}
 
 // b: which of the two buffers of per-workgroup totals (the step's force pass)
 // and of block rows (its integrator kernels) the step fills
@@ -94,7 +98,27 @@ StepArgs step_args(lj_ctx* c, double dt, int b = 0)
   a.ew = c->step_ew ? c->step_ew + (size_t)b * 2 * c->plan3.step_wgs() : nullptr;
   a.nitems = c->step_ew ? c->plan3.step_wgs() : 0;
   a.nrow = is_fp64(c) ? c->nblk : step_rows(c->cfg.N);
+  if (c->small_T) {
+    // one-launch steps: EVN alternates between the two coordinate buffers, TVN
+    // (whose coordinates a launch of their own writes) keeps to one
+    const bool swap = b && c->cfg.canonical == LJ_EVN;
+    a.q = swap ? c->q2 : c->q;
+    a.qn = swap ? c->q : c->q2;
+    a.ew = nullptr;
+    a.nitems = 0;
+    a.nrow = (c->cfg.N + c->small_T - 1) / c->small_T;
+    a.keep_w = !c->plan3.n3;  // w reads 0 after a step of the pair-once sizes
+  }
   return a;
+}
+
+// whether an environment switch picks the force pass of the time step
+bool force_pass_chosen()
+{
+  for (const char* e : {"LJ_PAIR_ONCE", "LJ_PAIR_ONCE_SPLIT", "LJ_PAIR_ONCE_WAVES",
+                        "LJ_PAIR_ONCE_COMP", "LJ_FORCE_SPLIT"})
+    if (std::getenv(e)) return true;
+  return false;
 }
 
 void refresh_scalars(lj_ctx* c)
@@ -165,6 +189,38 @@ int enqueue_force(lj_ctx* c, hipStream_t st, const float4* d_pos)
   return LJ_OK;
 }
 
+// the RDF pass of a sampled step, over the positions its force pass sees
+// (drifted, before the boundary conditions), as CalculateForces bins them
+// inside Integrate
+int enqueue_step_rdf(lj_ctx* c, hipStream_t st)
+{
+  if (c->smp_rdf == LJ_SAMPLE_RDF_OFF) return LJ_OK;
+  if (c->smp_rdf == LJ_SAMPLE_RDF_LAST) LJ_HIP(launch_fill_u64(st, c->rdf_step, c->smp_args.nbins));
+  LJ_HIP(launch_rdf(st, c->smp_args));
+  return LJ_OK;
+}
+
+// One step of a run in the one-launch form (lj_small.hip): the force pass and
+// the integrator are one kernel (EVN) or two (TVN), and the first kernel of
+// each step also computes the previous step's observables.
+int enqueue_small_step(lj_ctx* c, hipStream_t st, double dt, bool first, bool last, int b)
+{
+  const StepArgs a = step_args(c, dt, b);
+  if (first) LJ_HIP(launch_small_drift(st, a));
+  LJ_TRY(enqueue_step_rdf(c, st));
+  const StepArgs prev = step_args(c, dt, b ^ 1);
+  const StepArgs* fin = first ? nullptr : &prev;
+  if (c->cfg.canonical == LJ_EVN) {
+    LJ_HIP(launch_small_evn(st, c->small_T, a, c->ps.C1, !last, fin));
+  } else {
+    LJ_HIP(launch_small_tvn(st, c->small_T, a, c->ps.C1, fin));
+    LJ_HIP(launch_tvn_b(st, a, !last, true));
+  }
+  if (last) LJ_HIP(launch_small_finalize(st, a));
+  if (c->smp_fl) LJ_HIP(launch_fl_sample(st, c->fl, c->pos, c->vel, c->cfg.N, nullptr, nullptr, 0));
+  return LJ_OK;
+}
+
 // One step of a run of steps captured together.  The first step starts with
 // the drift; each later one finds it done by the previous step's last kernel
 // (drift_next).  With the pair-once pass the observables of a step are
@@ -177,6 +233,7 @@ int enqueue_force(lj_ctx* c, hipStream_t st, const float4* d_pos)
 int enqueue_step_part(lj_ctx* c, hipStream_t st, double dt, bool first, bool last, int b)
 {
   if (is_fp64(c)) return enqueue_step64(c, st, dt);
+  if (c->small_T) return enqueue_small_step(c, st, dt, first, last, b);
   const StepArgs a = step_args(c, dt, b);
   const bool comp = c->cfg.precision == LJ_PREC_COMPENSATED;
   const bool fused_fin = a.nitems > 0;  // the pair-once time-step pass
@@ -195,12 +252,7 @@ int enqueue_step_part(lj_ctx* c, hipStream_t st, double dt, bool first, bool las
   } else {
     LJ_HIP(launch_force(st, fplan(c), c->ps, c->q, c->pos, c->fpart, c->apart, comp, false, ew));
   }
-  if (c->smp_rdf != LJ_SAMPLE_RDF_OFF) {
-    // the positions the force pass saw (drifted, before the boundary
-    // conditions), as CalculateForces bins them inside Integrate
-    if (c->smp_rdf == LJ_SAMPLE_RDF_LAST) LJ_HIP(launch_fill_u64(st, c->rdf_step, c->smp_args.nbins));
-    LJ_HIP(launch_rdf(st, c->smp_args));
-  }
+  LJ_TRY(enqueue_step_rdf(c, st));
   const StepArgs prev = step_args(c, dt, b ^ 1);
   const StepArgs* fin = fused_fin && !first ? &prev : nullptr;
   if (c->cfg.canonical == LJ_EVN) {
@@ -362,6 +414,7 @@ int lj_destroy(lj_ctx* c)
   dev_free(c->force);
   dev_free(c->tF);
   dev_free(c->q);
+  dev_free(c->q2);
   dev_free(c->fpart);
   dev_free(c->apart);
   dev_free(c->blk);
@@ -429,6 +482,8 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
     else if (cfg->precision == LJ_PREC_COMPENSATED && n3_comp_enabled())
       c->plan3 = make_n3_plan(cfg->N, true);
   }
+  // the one-launch step unless an explicit choice of force pass asks for it
+  if (cfg->jslices == 0 && !is_fp64(c) && !force_pass_chosen()) c->small_T = small_tile(cfg->N);
   const size_t npart = (size_t)std::max(c->plan.S, c->plan3.S) * c->plan.Npad;
   const int N = cfg->N;
   c->nblk = (N + kBlock - 1) / kBlock;
@@ -443,6 +498,7 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
   A(dev_alloc(&c->force, N));
   A(dev_alloc(&c->tF, N));
   A(dev_alloc(&c->q, N));
+  if (c->small_T) A(dev_alloc(&c->q2, N));
   A(dev_alloc(&c->fpart, npart));
   A(dev_alloc(&c->apart, npart));
   if (c->plan3.n3) {

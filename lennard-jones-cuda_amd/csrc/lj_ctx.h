@@ -22,6 +22,8 @@ struct lj_ctx {
   float4* force = nullptr;
   float4* tF = nullptr;
   uint4* q = nullptr;
+  uint4* q2 = nullptr;  // one-launch steps: the other coordinate buffer
+  int small_T = 0;      // particles per workgroup of the one-launch step (0: off)
   float4* fpart = nullptr;
   float* apart = nullptr;
   double* blk = nullptr;

@@ -387,6 +387,14 @@ __device__ __forceinline__ void step_observables(const StepArgs& a, int nrow, bo
 {
   constexpr int NT = 64 * NW;
   double v[3] = {0., 0., 0.};
+  // the fields that are carried over go out ahead of the sums
+  lj_obs* o = a.obs;
+  lj_obs old = {};
+  int64_t base = 0;
+  if (threadIdx.x == 0) {
+    old = *o;
+    if (advance) base = *a.hist_base;
+  }
   // unrolled so that each thread's loads are in flight together (this block
   // runs beside the particle blocks of an integrator kernel and should not
   // outlast them)
@@ -404,35 +412,35 @@ __device__ __forceinline__ void step_observables(const StepArgs& a, int nrow, bo
     }
   block_allsum<3, NW>(v);
   if (threadIdx.x != 0) return;
-  lj_obs* o = a.obs;
   const int N = a.N;
   const double K = v[0] / 2.;
   const double T = 2. * K / 3. / N;
-  if (force_terms) {
-    o->V = 2. * a.eps * v[1];
-    o->W = 12. * a.eps * v[2];
-  }
-  const double Pvir = o->W / 3.;
+  const double V = force_terms ? 2. * a.eps * v[1] : old.V;
+  const double W = force_terms ? 12. * a.eps * v[2] : old.W;
+  const double Pvir = W / 3.;
   const double P = (Pvir + N * T) / (N / a.rho);
+  const double U = K + V;
+  o->V = V;
+  o->W = W;
   o->K = K;
   o->T = T;
   o->P = P;
-  o->U = K + o->V;
+  o->U = U;
   o->Pshear = 0.;
-  o->av_iters += 1;
-  o->av_U_tot += o->U;
-  o->av_p_tot += P;
-  o->av_T_tot += T;
+  o->av_iters = old.av_iters + 1;
+  o->av_U_tot = old.av_U_tot + U;
+  o->av_p_tot = old.av_p_tot + P;
+  o->av_T_tot = old.av_T_tot + T;
   if (advance) {
-    o->t += a.dt;
-    const int64_t k = o->step - *a.hist_base;
-    o->step += 1;
+    o->t = old.t + a.dt;
+    const int64_t k = old.step - base;
+    o->step = old.step + 1;
     if (a.hist && k >= 0 && k < a.hist_cap) {
       double* h = a.hist + 5 * k;
-      h[0] = o->U;
+      h[0] = U;
       h[1] = T;
       h[2] = K;
-      h[3] = o->V;
+      h[3] = V;
       h[4] = P;
     }
   }

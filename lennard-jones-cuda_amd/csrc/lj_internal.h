@@ -135,6 +135,10 @@ struct StepArgs {
   // block rows of the step's sums (K2, TV2, E, B): one per kRowParticles
   // particles in the FP32 step kernels, one per kBlock in the FP64 ones
   int nrow;
+  // one-launch steps of small boxes (lj_small.hip): the coordinates of the
+  // next step's force pass, and whether Force.w receives e_i (else 0)
+  uint4* qn;
+  int keep_w;
 };
 // steps per replay of the multi-step graphs (single box and batch): each graph
 // launch costs about 8 us of idle device time between replays, against none
@@ -152,9 +156,23 @@ hipError_t launch_drift(hipStream_t st, const StepArgs& a);
 hipError_t launch_kick_evn(hipStream_t st, const StepArgs& a, bool drift_next = false,
                            const StepArgs* fin = nullptr);
 hipError_t launch_tvn_a(hipStream_t st, const StepArgs& a, const StepArgs* fin = nullptr);
-hipError_t launch_tvn_b(hipStream_t st, const StepArgs& a, bool drift_next = false);
+// float_q: the next step's coordinates of a box without images go to a.q too
+hipError_t launch_tvn_b(hipStream_t st, const StepArgs& a, bool drift_next = false,
+                        bool float_q = false);
 // observables of the step; advance t/step, write history
 hipError_t launch_finalize_step(hipStream_t st, const StepArgs& a);
+// One-launch steps of small boxes (lj_small.hip): T particles per workgroup and
+// block row; 0 where the step runs the separate force pass and kernels
+int small_tile(int N);
+// the drift that starts a run, coordinates (fixed point or float bits) into a.q
+hipError_t launch_small_drift(hipStream_t st, const StepArgs& a);
+// force pass from a.q and kick; drift_next: also the next drift, into a.qn;
+// fin: observables of the run's previous step
+hipError_t launch_small_evn(hipStream_t st, int T, const StepArgs& a, float C1, bool drift_next,
+                            const StepArgs* fin);
+// force pass from a.q and the half-step velocities (launch_tvn_b follows)
+hipError_t launch_small_tvn(hipStream_t st, int T, const StepArgs& a, float C1, const StepArgs* fin);
+hipError_t launch_small_finalize(hipStream_t st, const StepArgs& a);
 // observables of the current state (no time advance): K from vel, V/W from blk
 hipError_t launch_params(hipStream_t st, const StepArgs& a, int include_force_terms);
 hipError_t launch_set_hist_base(hipStream_t st, lj_obs* obs, int64_t* base);

@@ -345,7 +345,9 @@ __global__ __launch_bounds__(kSumBlock) void k_tvn_a(StepArgs a, StepArgs fin)
 
 // one particle per thread; each wave (kRowParticles particles) writes the K2
 // field of its block row
-template <bool DRIFT, bool MAKEQ>
+// MAKEQ: 1 the periodic fixed-point copy, 2 the bits of the float coordinates
+// (one-launch steps of small boxes)
+template <bool DRIFT, int MAKEQ>
 __global__ __launch_bounds__(kBlock) void k_tvn_b(StepArgs a)
 {
 #pragma clang fp contract(off)
@@ -379,8 +381,10 @@ __global__ __launch_bounds__(kBlock) void k_tvn_b(StepArgs a)
       drift_one<LJ_TVN>(p, v, tfn, f, dt);
       a.tF[i] = tfn;
       a.pos[i] = p;
-      if constexpr (MAKEQ)
+      if constexpr (MAKEQ == 1)
         a.q[i] = make_uint4(fixq(p.x, a.qscale), fixq(p.y, a.qscale), fixq(p.z, a.qscale), 0u);
+      if constexpr (MAKEQ == 2)
+        a.q[i] = make_uint4(__float_as_uint(p.x), __float_as_uint(p.y), __float_as_uint(p.z), 0u);
     }
   }
 #pragma unroll
@@ -1078,12 +1082,13 @@ hipError_t launch_tvn_a(hipStream_t st, const StepArgs& a, const StepArgs* fin)
   return hipGetLastError();
 }
 
-hipError_t launch_tvn_b(hipStream_t st, const StepArgs& a, bool drift_next)
+hipError_t launch_tvn_b(hipStream_t st, const StepArgs& a, bool drift_next, bool float_q)
 {
   const dim3 g(nblocks(a.N)), b(kBlock);
-  if (!drift_next) hipLaunchKernelGGL((k_tvn_b<false, false>), g, b, 0, st, a);
-  else if (a.bc == LJ_BC_PERIODIC) hipLaunchKernelGGL((k_tvn_b<true, true>), g, b, 0, st, a);
-  else hipLaunchKernelGGL((k_tvn_b<true, false>), g, b, 0, st, a);
+  if (!drift_next) hipLaunchKernelGGL((k_tvn_b<false, 0>), g, b, 0, st, a);
+  else if (a.bc == LJ_BC_PERIODIC) hipLaunchKernelGGL((k_tvn_b<true, 1>), g, b, 0, st, a);
+  else if (float_q) hipLaunchKernelGGL((k_tvn_b<true, 2>), g, b, 0, st, a);
+  else hipLaunchKernelGGL((k_tvn_b<true, 0>), g, b, 0, st, a);
   return hipGetLastError();
 }
 
