@@ -216,7 +216,7 @@ int enqueue_small_step(lj_ctx* c, hipStream_t st, double dt, bool first, bool la
     LJ_HIP(launch_small_tvn(st, c->small_T, a, c->ps.C1, fin));
     LJ_HIP(launch_tvn_b(st, a, !last, true));
   }
-  if (last) LJ_HIP(launch_small_finalize(st, a));
+  if (last) LJ_HIP(launch_finalize_step(st, a));
   if (c->smp_fl) LJ_HIP(launch_fl_sample(st, c->fl, c->pos, c->vel, c->cfg.N, nullptr, nullptr, 0));
   return LJ_OK;
 }

@@ -4,7 +4,7 @@
 // over workgroups that never straddle two boxes, so every per-box reduction
 // stays a fixed-order FP64 sum.  Physics per box is the single-box step of
 // lj_kernels.hip (reference MDSystem.cpp:438-583, MDSystem.cu:21-138).
-#include "lj_device.h"
+#include "lj_small.h"
 
 namespace lj {
 
@@ -109,6 +109,13 @@ __global__ __launch_bounds__(kBlock) void k_batch_prep_q(BatchArgs a)
   a.q[p.gi] = make_uint4(fixq(x.x, qs), fixq(x.y, qs), fixq(x.z, qs), 0u);
 }
 
+// the drifted coordinates as the next force pass reads them
+__device__ __forceinline__ void batch_make_q(const BatchArgs& a, const PIdx& pp, const float4& p)
+{
+  if (a.bc == LJ_BC_PERIODIC) a.q[pp.gi] = small_q<true>(p, a.box[pp.b].qscale);
+  else if (a.ntiles) a.q[pp.gi] = small_q<false>(p, 0.);
+}
+
 template <int CANON>
 __global__ __launch_bounds__(kBlock) void k_batch_drift(BatchArgs a)
 {
@@ -124,10 +131,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_drift(BatchArgs a)
   if constexpr (CANON == LJ_EVN) a.vel[i] = v;
   else a.tF[i] = tf;
   a.pos[i] = p;
-  if (a.bc == LJ_BC_PERIODIC) {
-    const double qs = a.box[pp.b].qscale;
-    a.q[i] = make_uint4(fixq(p.x, qs), fixq(p.y, qs), fixq(p.z, qs), 0u);
-  }
+  batch_make_q(a, pp, p);
 }
 
 // the next step's drift of one particle at the end of a kick kernel (the
@@ -142,10 +146,7 @@ __device__ __forceinline__ void batch_drift_next(const BatchArgs& a, const PIdx&
   if constexpr (CANON == LJ_EVN) a.vel[pp.gi] = v;
   else a.tF[pp.gi] = tf;
   a.pos[pp.gi] = p;
-  if (a.bc == LJ_BC_PERIODIC) {
-    const double qs = a.box[pp.b].qscale;
-    a.q[pp.gi] = make_uint4(fixq(p.x, qs), fixq(p.y, qs), fixq(p.z, qs), 0u);
-  }
+  batch_make_q(a, pp, p);
 }
 
 __device__ __forceinline__ Partial box_slices(const BatchArgs& a, const BoxParam& bp, int i)
@@ -263,8 +264,11 @@ __global__ __launch_bounds__(kBlock) void k_batch_tvn_b(BatchArgs a)
     if constexpr (DRIFT) batch_drift_next<LJ_TVN>(a, pp, p, v, a.force[i]);
   }
   __syncthreads();
+  // row k of the box: its k-th block here (one-launch steps hold more rows, the
+  // others' K2 and NSUB fields zeroed by their first kernel)
   const int fld[2] = {BLK_K2, BLK_NSUB};
-  block_sum_store<2>(v2, a.blk + (size_t)blockIdx.x * kBlkFields, fld);
+  const int row = bp.blk0 + a.pblock[blockIdx.x].y / kBlock;
+  block_sum_store<2>(v2, a.blk + (size_t)row * kBlkFields, fld);
 }
 
 __global__ __launch_bounds__(kBlock) void k_batch_reduce_forces(BatchArgs a)
@@ -297,11 +301,10 @@ __global__ __launch_bounds__(kBlock) void k_batch_kinetic(BatchArgs a)
   block_sum_store<2>(v2, a.blk + (size_t)blockIdx.x * kBlkFields, fld);
 }
 
-// one workgroup per box: observables (MDSystem.cpp:325-359) and, when
+// kBlock threads per box: observables (MDSystem.cpp:325-359) and, when
 // advancing, the accumulated fluctuation statistics of the box
-__global__ __launch_bounds__(kBlock) void k_batch_finalize(BatchArgs a, int advance)
+__device__ __forceinline__ void batch_observables(const BatchArgs& a, int b, int advance)
 {
-  const int b = blockIdx.x;
   const BoxParam& bp = a.box[b];
   double v[4] = {0., 0., 0., 0.};
   const double* rows = a.blk + (size_t)bp.blk0 * kBlkFields;
@@ -362,6 +365,155 @@ __global__ __launch_bounds__(kBlock) void k_batch_finalize(BatchArgs a, int adva
     st[ST_N3] += n * n * n;
     st[ST_N4] += n * n * n * n;
   }
+}
+
+__global__ __launch_bounds__(kBlock) void k_batch_finalize(BatchArgs a, int advance)
+{
+  batch_observables(a, blockIdx.x, advance);
+}
+
+// ---- one-launch steps (lj_small.h): the workgroup that computes the whole
+// force on kBatchTile particles of a box also runs their integrator.  FIN: the
+// first nboxes workgroups finalise the run's previous step.  They serve every
+// batch whose tuning was not set: an ensemble of a few small boxes had one wave
+// per 64 particles and slice, each meeting up to 512 j one after another (16
+// boxes of 400: 131 us per EVN step, 9.4 us here; 64 of 1000: 173 / 53; 100 of
+// 3000: 534 / 462; the 512-box ensemble 1542 / 1530), which is why the launch is
+// bound by the pairs' issue slots only from about 1e8 pairs on.  Tiles of 16:
+// 8 and 4 re-read the box for fewer pairs each (16 of 400: 11.8 and 16.3). ----
+
+template <bool PERIODIC, bool DRIFT, bool FIN>
+__global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(8))) void
+k_batch_small_evn(BatchArgs a, BatchArgs fin)
+{
+#pragma clang fp contract(off)
+  constexpr int T = kBatchTile;
+  __shared__ SmallLds<T> lds;
+  if constexpr (FIN) {
+    if ((int)blockIdx.x < fin.nboxes) {
+      // by the threads of k_batch_finalize: the same bits
+      if (threadIdx.x < kBlock) batch_observables(fin, blockIdx.x, 1);
+      return;
+    }
+  }
+  const int2 tile = a.tiles[blockIdx.x - (FIN ? a.nboxes : 0)];
+  const BoxParam& bp = a.box[tile.x];
+  const int i = tile.y + threadIdx.x, gi = bp.off + i;
+  const bool lead = threadIdx.x < T && i < bp.N;
+  float4 v = {}, p = {};
+  if (lead) {
+    v = a.vel[gi];
+    p = a.pos[gi];
+  }
+  const Partial s = small_forces<PERIODIC, T>(lds, a.q + bp.off, bp.N, tile.y, bp.C1);
+  if (threadIdx.x >= 64) return;
+  double v4[4] = {0., 0., 0., 0.};
+  if (lead) {
+    const double e = 0.5 * (s.b - s.a);
+    const float fx = (float)(bp.FS * s.fx), fy = (float)(bp.FS * s.fy), fz = (float)(bp.FS * s.fz);
+    a.force[gi] = make_float4(fx, fy, fz, (float)e);
+    const double dt = a.dt;
+    v.x = (float)(v.x + dt * fx / 2.);  // MDSystem.cpp:460-462
+    v.y = (float)(v.y + dt * fy / 2.);
+    v.z = (float)(v.z + dt * fz / 2.);
+    apply_bc_one(p, v, a.bc, bp.L);
+    if (!DRIFT && PERIODIC) a.pos[gi] = p;
+    v4[0] = kin2(v);
+    v4[1] = e;
+    v4[2] = s.b;
+    v4[3] = inside(p, bp);
+    if constexpr (DRIFT) {
+      float4 tf;
+      drift_one<LJ_EVN>(p, v, tf, make_float4(fx, fy, fz, 0.f), dt);
+      a.pos[gi] = p;
+      a.qn[gi] = small_q<PERIODIC>(p, bp.qscale);
+    }
+    a.vel[gi] = v;
+  }
+  small_row_sum<4, T>(v4);
+  if (threadIdx.x == 0) {
+    double* r = a.blk + (size_t)(bp.blk0 + tile.y / T) * kBlkFields;
+    r[BLK_K2] = v4[0];
+    r[BLK_E] = v4[1];
+    r[BLK_B] = v4[2];
+    r[BLK_NSUB] = v4[3];
+  }
+}
+
+template <bool PERIODIC, bool FIN>
+__global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(8))) void
+k_batch_small_tvn(BatchArgs a, BatchArgs fin)
+{
+#pragma clang fp contract(off)
+  constexpr int T = kBatchTile;
+  __shared__ SmallLds<T> lds;
+  if constexpr (FIN) {
+    if ((int)blockIdx.x < fin.nboxes) {
+      // by the threads of k_batch_finalize: the same bits
+      if (threadIdx.x < kBlock) batch_observables(fin, blockIdx.x, 1);
+      return;
+    }
+  }
+  const int2 tile = a.tiles[blockIdx.x - (FIN ? a.nboxes : 0)];
+  const BoxParam& bp = a.box[tile.x];
+  const int i = tile.y + threadIdx.x, gi = bp.off + i;
+  const bool lead = threadIdx.x < T && i < bp.N;
+  float4 v = {}, tf = {};
+  if (lead) {
+    v = a.vel[gi];
+    tf = a.tF[gi];
+  }
+  const Partial s = small_forces<PERIODIC, T>(lds, a.q + bp.off, bp.N, tile.y, bp.C1);
+  if (threadIdx.x >= 64) return;
+  double v3[3] = {0., 0., 0.};
+  if (lead) {
+    const double e = 0.5 * (s.b - s.a);
+    const float fx = (float)(bp.FS * s.fx), fy = (float)(bp.FS * s.fy), fz = (float)(bp.FS * s.fz);
+    a.force[gi] = make_float4(fx, fy, fz, (float)e);
+    tf.x += 0.5f * fx;  // MDSystem.cpp:486-488
+    tf.y += 0.5f * fy;
+    tf.z += 0.5f * fz;
+    a.tF[gi] = tf;
+    const double dt = a.dt;
+    float4 tv;
+    tv.x = (float)(v.x + dt * tf.x / 2.);  // MDSystem.cpp:493-495
+    tv.y = (float)(v.y + dt * tf.y / 2.);
+    tv.z = (float)(v.z + dt * tf.z / 2.);
+    tv.w = 0.f;
+    v3[0] = kin2(tv);
+    v3[1] = e;
+    v3[2] = s.b;
+  }
+  small_row_sum<3, T>(v3);
+  if (threadIdx.x == 0) {
+    double* r = a.blk + (size_t)(bp.blk0 + tile.y / T) * kBlkFields;
+    r[BLK_K2] = 0.;
+    r[BLK_TV2] = v3[0];
+    r[BLK_E] = v3[1];
+    r[BLK_B] = v3[2];
+    r[BLK_NSUB] = 0.;
+  }
+}
+
+template <bool PERIODIC>
+void batch_small_evn_t(hipStream_t st, const BatchArgs& a, bool drift_next, const BatchArgs* fin)
+{
+  const dim3 g(a.ntiles + (fin ? a.nboxes : 0)), b(kSmallThreads);
+  if (drift_next) {
+    if (fin) hipLaunchKernelGGL((k_batch_small_evn<PERIODIC, true, true>), g, b, 0, st, a, *fin);
+    else hipLaunchKernelGGL((k_batch_small_evn<PERIODIC, true, false>), g, b, 0, st, a, a);
+  } else {
+    if (fin) hipLaunchKernelGGL((k_batch_small_evn<PERIODIC, false, true>), g, b, 0, st, a, *fin);
+    else hipLaunchKernelGGL((k_batch_small_evn<PERIODIC, false, false>), g, b, 0, st, a, a);
+  }
+}
+
+template <bool PERIODIC>
+void batch_small_tvn_t(hipStream_t st, const BatchArgs& a, const BatchArgs* fin)
+{
+  const dim3 g(a.ntiles + (fin ? a.nboxes : 0)), b(kSmallThreads);
+  if (fin) hipLaunchKernelGGL((k_batch_small_tvn<PERIODIC, true>), g, b, 0, st, a, *fin);
+  else hipLaunchKernelGGL((k_batch_small_tvn<PERIODIC, false>), g, b, 0, st, a, a);
 }
 
 __global__ void k_batch_set_hist_base(const lj_obs* obs, int64_t* base, int nboxes)
@@ -451,6 +603,21 @@ hipError_t launch_batch_tvn_b(hipStream_t st, const BatchArgs& a, bool drift_nex
 hipError_t launch_batch_finalize(hipStream_t st, const BatchArgs& a, int advance)
 {
   hipLaunchKernelGGL(k_batch_finalize, dim3(a.nboxes), dim3(kBlock), 0, st, a, advance);
+  return hipGetLastError();
+}
+
+hipError_t launch_batch_small_evn(hipStream_t st, const BatchArgs& a, bool drift_next,
+                                  const BatchArgs* fin)
+{
+  if (a.bc == LJ_BC_PERIODIC) batch_small_evn_t<true>(st, a, drift_next, fin);
+  else batch_small_evn_t<false>(st, a, drift_next, fin);
+  return hipGetLastError();
+}
+
+hipError_t launch_batch_small_tvn(hipStream_t st, const BatchArgs& a, const BatchArgs* fin)
+{
+  if (a.bc == LJ_BC_PERIODIC) batch_small_tvn_t<true>(st, a, fin);
+  else batch_small_tvn_t<false>(st, a, fin);
   return hipGetLastError();
 }
 

@@ -37,6 +37,15 @@ struct lj_batch {
   float* apart = nullptr;
   size_t part_cap = 0;
   double* blk = nullptr;
+  // one-launch steps (until a tuning is set): the other coordinate buffer, the
+  // tiles, the boxes with the tiles' rows, and two buffers of block rows that
+  // the steps alternate between
+  bool tuned = false;
+  uint4* q2 = nullptr;
+  BoxParam* box_s = nullptr;
+  int2* tiles = nullptr;
+  double* blk_s = nullptr;
+  int ntiles = 0;
   lj_obs* obs = nullptr;
   double* stats = nullptr;
   BoxParam* box = nullptr;
@@ -120,6 +129,48 @@ BatchArgs bargs(lj_batch* b, double dt, bool lean = false)
   a.hist_base = b->hist_base;
   a.hist_cap = b->hist_cap;
   return a;
+}
+
+// a one-launch step; par: its parity in the run
+BatchArgs small_args(lj_batch* b, double dt, int par)
+{
+  BatchArgs a = bargs(b, dt);
+  const bool swap = par && b->canonical == LJ_EVN;
+  a.q = swap ? b->q2 : b->q;
+  a.qn = swap ? b->q : b->q2;
+  a.box = b->box_s;
+  a.blk = b->blk_s + (size_t)par * b->ntiles * kBlkFields;
+  a.ntiles = b->ntiles;
+  a.tiles = b->tiles;
+  return a;
+}
+
+// tables of the one-launch steps, from the boxes' parameters
+int build_small(lj_batch* b, const std::vector<BoxParam>& bp)
+{
+  if (b->tuned) return LJ_OK;
+  const int T = kBatchTile;
+  std::vector<BoxParam> bs = bp;
+  std::vector<int2> tiles;
+  for (int k = 0; k < b->nboxes; ++k) {
+    bs[k].blk0 = (int)tiles.size();
+    bs[k].nblk = (b->N[k] + T - 1) / T;
+    for (int t = 0; t < bs[k].nblk; ++t) tiles.push_back(make_int2(k, t * T));
+  }
+  // the boxes' rows stay in box order; the tiles with the longest chains first
+  std::stable_sort(tiles.begin(), tiles.end(),
+                   [&](const int2& x, const int2& y) { return b->N[x.x] > b->N[y.x]; });
+  b->ntiles = (int)tiles.size();
+  if (!b->q2) LJ_TRY(dev_alloc(&b->q2, b->Ntot));
+  if (!b->box_s) LJ_TRY(dev_alloc(&b->box_s, b->nboxes));
+  if (!b->tiles) LJ_TRY(dev_alloc(&b->tiles, tiles.size()));
+  if (!b->blk_s) LJ_TRY(dev_alloc(&b->blk_s, (size_t)2 * tiles.size() * kBlkFields));
+  LJ_HIP(hipMemcpyAsync(b->box_s, bs.data(), sizeof(BoxParam) * bs.size(), hipMemcpyHostToDevice,
+                        b->stream));
+  LJ_HIP(hipMemcpyAsync(b->tiles, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice,
+                        b->stream));
+  LJ_HIP(hipStreamSynchronize(b->stream));
+  return LJ_OK;
 }
 
 // (re)build the per-box tables and the work items for the current tuning
@@ -222,6 +273,7 @@ int build_tables(lj_batch* b)
   LJ_HIP(hipMemcpyAsync(b->items, items.data(), sizeof(BatchItem) * items.size(),
                         hipMemcpyHostToDevice, b->stream));
   LJ_HIP(hipStreamSynchronize(b->stream));
+  LJ_TRY(build_small(b, bp));
   b->hbox = bp;
   b->nblocks = (int)pblock.size();
   b->nitems = (int)items.size();
@@ -232,8 +284,23 @@ int build_tables(lj_batch* b)
 // one step of a run captured together: the first starts with the drift, each
 // later one finds it done by the previous step's kick kernel (drift_next), with
 // the same arithmetic, so a run gives the bits of single steps
-int enqueue_batch_step(lj_batch* b, hipStream_t st, double dt, bool first = true, bool last = true)
+int enqueue_batch_step(lj_batch* b, hipStream_t st, double dt, bool first = true, bool last = true,
+                       int par = 0)
 {
+  if (!b->tuned) {
+    const BatchArgs a = small_args(b, dt, par), prev = small_args(b, dt, par ^ 1);
+    if (first) LJ_HIP(launch_batch_drift(st, a));
+    if (b->canonical == LJ_EVN) {
+      LJ_HIP(launch_batch_small_evn(st, a, !last, first ? nullptr : &prev));
+    } else {
+      LJ_HIP(launch_batch_small_tvn(st, a, first ? nullptr : &prev));
+      LJ_HIP(launch_batch_tvn_b(st, a, !last));
+    }
+    if (last) LJ_HIP(launch_batch_finalize(st, a, 1));
+    if (b->smp_fl)
+      LJ_HIP(launch_fl_sample(st, b->fl, b->pos, b->vel, 0, b->box, b->pblock, b->nblocks));
+    return LJ_OK;
+  }
   const BatchArgs a = bargs(b, dt, true);
   if (first) LJ_HIP(launch_batch_drift(st, a));
   LJ_HIP(launch_batch_force(st, a, b->boundary == LJ_BC_PERIODIC, false));
@@ -258,7 +325,7 @@ int capture_batch_steps(lj_batch* b, double dt, int steps, hipGraph_t* graph, hi
   // step fused into their kick kernels)
   const bool alone = b->smp_fl != 0;
   for (int k = 0; k < steps && rc == LJ_OK; ++k)
-    rc = enqueue_batch_step(b, st, dt, alone || k == 0, alone || k == steps - 1);
+    rc = enqueue_batch_step(b, st, dt, alone || k == 0, alone || k == steps - 1, k & 1);
   hipGraph_t g = nullptr;
   hipError_t ee = hipStreamEndCapture(st, &g);
   if (rc != LJ_OK) {
@@ -389,6 +456,10 @@ int lj_batch_destroy(lj_batch* b)
   dev_free(b->force);
   dev_free(b->tF);
   dev_free(b->q);
+  dev_free(b->q2);
+  dev_free(b->box_s);
+  dev_free(b->tiles);
+  dev_free(b->blk_s);
   dev_free(b->fpart);
   dev_free(b->apart);
   dev_free(b->blk);
@@ -506,6 +577,7 @@ int lj_batch_set_tuning(lj_batch* b, const lj_batch_tuning* t)
       t->blocks_per_cu < 0 || t->blocks_per_cu > 64 || (t->pair_once != 0 && t->pair_once != 1))
     return fail(LJ_ERR_ARG, "lj_batch_set_tuning: ipl in {1,2}, jchunk in [8, 2^20], blocks_per_cu in [0, 64], pair_once in {0,1}");
   b->tune = *t;
+  b->tuned = true;
   return build_tables(b);
 }
 

@@ -172,7 +172,6 @@ hipError_t launch_small_evn(hipStream_t st, int T, const StepArgs& a, float C1, 
                             const StepArgs* fin);
 // force pass from a.q and the half-step velocities (launch_tvn_b follows)
 hipError_t launch_small_tvn(hipStream_t st, int T, const StepArgs& a, float C1, const StepArgs* fin);
-hipError_t launch_small_finalize(hipStream_t st, const StepArgs& a);
 // observables of the current state (no time advance): K from vel, V/W from blk
 hipError_t launch_params(hipStream_t st, const StepArgs& a, int include_force_terms);
 hipError_t launch_set_hist_base(hipStream_t st, lj_obs* obs, int64_t* base);
@@ -278,6 +277,8 @@ struct BoxParam {
 // with the pair-once decomposition (box, group g, group h).
 constexpr int kPairOnceGroup = 256;  // group size of the batched pair-once pass
 
+constexpr int kBatchTile = 16;  // particles per workgroup of the one-launch steps
+
 struct BatchItem {
   int box, i0, s;
   int e;  // pair-once: the item's slot in the per-box runs of (E, W) totals
@@ -320,6 +321,12 @@ struct BatchArgs {
   double* hist;
   const int64_t* hist_base;
   int hist_cap;
+  // one-launch steps (ntiles > 0): tiles (box, first particle) of kBatchTile
+  // particles, a block row each (box holds the rows); coordinates (fixed point
+  // or float bits) in q, those of the next step go to qn
+  int ntiles;
+  const int2* tiles;
+  uint4* qn;
 };
 hipError_t launch_batch_drift(hipStream_t st, const BatchArgs& a);
 hipError_t launch_batch_force(hipStream_t st, const BatchArgs& a, bool periodic, bool ties);
@@ -329,6 +336,12 @@ hipError_t launch_batch_kick_evn(hipStream_t st, const BatchArgs& a, bool drift_
 hipError_t launch_batch_tvn_a(hipStream_t st, const BatchArgs& a);
 hipError_t launch_batch_tvn_b(hipStream_t st, const BatchArgs& a, bool drift_next = false);
 hipError_t launch_batch_finalize(hipStream_t st, const BatchArgs& a, int advance);
+// one-launch steps: force pass and kick (EVN), or force pass and half-step
+// velocities (TVN, launch_batch_tvn_b follows); fin: the finaliser of the run's
+// previous step as extra workgroups
+hipError_t launch_batch_small_evn(hipStream_t st, const BatchArgs& a, bool drift_next,
+                                  const BatchArgs* fin);
+hipError_t launch_batch_small_tvn(hipStream_t st, const BatchArgs& a, const BatchArgs* fin);
 hipError_t launch_batch_prep_q(hipStream_t st, const BatchArgs& a);
 hipError_t launch_batch_reduce_forces(hipStream_t st, const BatchArgs& a);
 hipError_t launch_batch_kinetic(hipStream_t st, const BatchArgs& a);

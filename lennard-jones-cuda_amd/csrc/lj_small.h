@@ -18,7 +18,6 @@ namespace dev {
 // phases, twice the sums to reduce and a few spills (N = 2048, T = 8, EVN step:
 // 8.75 against 7.67 us; four per lane 13 us and more).
 constexpr int kSmallThreads = 1024;
-constexpr int kSmallWaves = kSmallThreads / 64;
 
 template <int T>
 struct SmallGeo {

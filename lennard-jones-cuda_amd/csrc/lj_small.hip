@@ -6,10 +6,10 @@
 // A step of a small box is a chain of latencies: at N = 400 its 80,000 pairs
 // are 0.05 us of the device's FP32 rate, an empty kernel in a chain of graph
 // nodes takes 1.8 us, and the force pass, kick and finaliser took 11.0 us.
-// Here the step is 4.6 us: the launch, one load of all coordinates, the pairs
+// Here the step is 4.3 us: the launch, one load of all coordinates, the pairs
 // of a lane, two passes through LDS and the stores.  From about N = 1500 on the
-// pair loop is visible, and at N = 4096 it is 9.4 us of the 14.2, which is the
-// issue time of its 22 slots per ordered pair.
+// pair loop is visible, and at N = 4096 it is 9.4 us of the 14, which is the issue
+// time of its 22 slots per ordered pair.
 #include "lj_small.h"
 
 namespace lj {
@@ -44,7 +44,8 @@ __global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(8
   __shared__ SmallLds<T> lds;
   if constexpr (FIN) {
     if (blockIdx.x == 0) {
-      step_observables<kSmallWaves>(fin, fin.nrow, true, true);
+      // by the threads of the stand-alone finaliser: the same bits
+      if (threadIdx.x < kBlock) step_observables<kWaves>(fin, fin.nrow, true, true);
       return;
     }
   }
@@ -99,7 +100,8 @@ __global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(8
   __shared__ SmallLds<T> lds;
   if constexpr (FIN) {
     if (blockIdx.x == 0) {
-      step_observables<kSmallWaves>(fin, fin.nrow, true, true);
+      // by the threads of the stand-alone finaliser: the same bits
+      if (threadIdx.x < kBlock) step_observables<kWaves>(fin, fin.nrow, true, true);
       return;
     }
   }
@@ -140,11 +142,6 @@ __global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(8
     r[BLK_E] = v3[1];
     r[BLK_B] = v3[2];
   }
-}
-
-__global__ __launch_bounds__(kSmallThreads) void k_small_finalize(StepArgs a)
-{
-  step_observables<kSmallWaves>(a, a.nrow, true, true);
 }
 
 template <bool PERIODIC, int T>
@@ -229,12 +226,6 @@ hipError_t launch_small_tvn(hipStream_t st, int T, const StepArgs& a, float C1, 
   } while (0)
   LJ_SMALL_T(LJ_CALL)
 #undef LJ_CALL
-  return hipGetLastError();
-}
-
-hipError_t launch_small_finalize(hipStream_t st, const StepArgs& a)
-{
-  hipLaunchKernelGGL(k_small_finalize, dim3(1), dim3(kSmallThreads), 0, st, a);
   return hipGetLastError();
 }
 

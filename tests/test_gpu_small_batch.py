@@ -1,0 +1,49 @@
+"""The one-launch time steps of a batch whose tuning was not set, at the edges
+of their tiles (16 particles) and LDS chunks (2048): box sizes 1 to 4097 in one
+batch, against the same boxes run one by one through the separate kernels of
+the sliced tuning, and in any split of the run."""
+import numpy as np
+import pytest
+
+import ljamd
+from helpers import rel, xyz
+
+pytestmark = pytest.mark.gpu
+
+N = np.array([2, 15, 16, 17, 64, 400, 2047, 2048, 2049, 4097], np.int32)
+RHO = np.array([0.02, 0.1, 0.2, 0.3, 0.4, 0.05, 0.5, 0.85, 0.6, 0.7])
+T0 = np.linspace(0.8, 2.0, N.size)
+
+
+@pytest.mark.parametrize("bc", [ljamd.BC_PERIODIC, ljamd.BC_WALL, ljamd.BC_NONE])
+@pytest.mark.parametrize("canon", [ljamd.EVN, ljamd.TVN])
+def test_small_batch_edges(canon, bc):
+    # tolerances: those of the single-box comparison of test_gpu_batch.py
+    steps = 20
+    print(f"\n[case] small batch canon={canon} bc={bc}", flush=True)
+    out = []
+    for chunks, tuning in (([steps], None), ([7, 13], None), ([steps], (1, 512, 8, 0))):
+        with ljamd.LJBatch(N, RHO, T0, canonical=canon, boundary=bc, seed=31) as b:
+            if tuning:
+                b.set_tuning(*tuning)
+            h = np.concatenate([b.integrate_hist(0.004, c) for c in chunks])
+            obs = b.observables()
+            f = [b.get_array(ljamd.ARRAY_FORCE, box=k) for k in range(N.size)]
+            p = [b.get_array(ljamd.ARRAY_POS, box=k) for k in range(N.size)]
+            v = [b.get_array(ljamd.ARRAY_VEL, box=k) for k in range(N.size)]
+            st = b.stats()
+            b.compute_forces()
+            full = b.observables()
+        out.append((h, obs, p, v, f, st, full))
+    a, split, sliced = out
+    for x, y in zip((a[0], a[5], *a[2], *a[3], *a[4]), (split[0], split[5], *split[2], *split[3], *split[4])):
+        assert np.array_equal(x, y)
+    assert np.all(a[5][:, 0] == steps) and np.array_equal(a[5][:, 9], sliced[5][:, 9])
+    for k in range(N.size):
+        assert np.max(np.abs(a[0][:, k, 0] - sliced[0][:, k, 0])) / N[k] <= 2e-5, k
+        assert np.max(np.abs(xyz(a[2][k]) - xyz(sliced[2][k]))) <= 4e-5, k
+        assert np.max(np.abs(xyz(a[3][k]) - xyz(sliced[3][k]))) <= 1e-3, k
+        assert abs(a[1][k]["V"] - a[6][k]["V"]) <= 1e-6 * max(abs(a[6][k]["V"]), N[k]), k
+        assert abs(a[1][k]["W"] - a[6][k]["W"]) <= 1e-5 * max(abs(a[6][k]["W"]), N[k]), k
+        e = np.sum(a[4][k].reshape(-1, 4)[:, 3].astype(np.float64)) * 2.0
+        assert rel(e, a[1][k]["V"]) <= 1e-5 or abs(e) < 1e-5, k
