@@ -45,6 +45,30 @@ struct AdjStep {
   double* rowacc = nullptr;
 };
 
+// One-launch steps of the FP64-state trajectory and of the reverse sweep (boxes
+// that have a small_tile): T particles per workgroup and block row.
+// q holds fixed-point coordinates, or the bits of the floats in an open box.
+struct DStep {
+  const uint4* q = nullptr;  // coordinates of this step's force pass
+  uint4* qn = nullptr;       // of the next one
+  double4 *x = nullptr, *v = nullptr, *f = nullptr;
+  double4 *slot_x = nullptr, *slot_v = nullptr;  // as launch_dkick's
+  double* blk = nullptr;  // rows of 8 doubles: e, b, |v|^2
+  double* acc = nullptr;  // as launch_dfinal's (fin and the last step)
+  int N = 0, nrow = 0;
+  double dt = 0., FS = 0., qs = 0., eps = 1., vol = 1.;
+  float C1 = 1.f;
+};
+// forces from a.q and kick, then (drift_next) the next step's drift; fin: the
+// run's previous step, whose observables one extra workgroup adds to acc
+hipError_t launch_small_dstep(hipStream_t st, int T, const DStep& a, bool drift_next,
+                              const DStep* fin);
+// the reverse sweep's pass at the coordinates q with vector z and its whole
+// update; zn / step.q receive the next state's vector and coordinates
+hipError_t launch_small_adj(hipStream_t st, int T, const PairScalars& ps, int N, const uint4* q,
+                            const float4* z, float4* zn, double* blk, const AdjStep& step);
+hipError_t launch_adj_narrow(hipStream_t st, const double4* dx0, int N, float4* out);
+
 // the pair pass's geometry for N particles (slices of the j range)
 ForcePlan adj_force_plan(int N);
 hipError_t launch_adj_pass(hipStream_t st, const ForcePlan& pl, const PairScalars& ps,
@@ -63,6 +87,7 @@ hipError_t launch_adj_zero2(hipStream_t st, double* g);
 // FP64-state trajectory of the differentiable path
 hipError_t launch_dstate_init(hipStream_t st, const float4* pos, const float4* vel, int N,
                               double4* xd, double4* vd);
+// xf == nullptr: without images, the bits of the float coordinates into q
 hipError_t launch_dprep(hipStream_t st, const double4* xd, int N, double qs, uint4* q, float4* xf);
 hipError_t launch_ddrift(hipStream_t st, double4* xd, double4* vd, const double4* fd, int N,
                          double dt, double qs, uint4* q, float4* xf);

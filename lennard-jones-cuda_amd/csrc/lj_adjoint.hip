@@ -19,7 +19,7 @@
 #include <cstdlib>
 
 #include "lj_adjoint.h"
-#include "lj_device.h"
+#include "lj_small.h"
 
 namespace lj {
 
@@ -314,6 +314,19 @@ __device__ __forceinline__ unsigned fixqd(double x, double qs)
   return (unsigned)(long long)__builtin_rint(x * qs);
 }
 
+// internal coordinates of a double position: fixed point (qs > 0), or its
+// float rounding, to xf or as bits to q where there is no xf
+__device__ __forceinline__ void put_coords(const double4& x, double qs, uint4* q, float4* xf, int i)
+{
+  if (qs > 0.) {
+    q[i] = make_uint4(fixqd(x.x, qs), fixqd(x.y, qs), fixqd(x.z, qs), 0u);
+    return;
+  }
+  const float4 p = make_float4((float)x.x, (float)x.y, (float)x.z, 0.f);
+  if (xf) xf[i] = p;
+  else q[i] = small_q<false>(p, 0.);
+}
+
 // what the reverse sweep's update of particle i reads besides the pass's sums
 struct AdjPre {
   double4 u, lv, vp, xn;
@@ -391,11 +404,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_reduce(const float4* __restrict_
     v[3] = s;
     v[4] = F.x * zi.x + F.y * zi.y + F.z * zi.z;
     if (step.next_x) {  // the next pass's coordinates (k_dprep)
-      const double4 x = pre.xn;
-      if (step.qs > 0.)
-        step.q[i] = make_uint4(fixqd(x.x, step.qs), fixqd(x.y, step.qs), fixqd(x.z, step.qs), 0u);
-      else
-        step.xf[i] = make_float4((float)x.x, (float)x.y, (float)x.z, 0.f);
+      put_coords(pre.xn, step.qs, step.q, step.xf, i);
     }
     if (step.mode == 1) {
       adj_update_one(i, H, F, G, step, pre, z);
@@ -521,9 +530,7 @@ __global__ __launch_bounds__(kBlock) void k_dprep(const double4* __restrict__ xd
 {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= N) return;
-  const double4 x = xd[i];
-  if (qs > 0.) q[i] = make_uint4(fixqd(x.x, qs), fixqd(x.y, qs), fixqd(x.z, qs), 0u);
-  else xf[i] = make_float4((float)x.x, (float)x.y, (float)x.z, 0.f);
+  put_coords(xd[i], qs, q, xf, i);
 }
 
 // x += dt v + dt^2/2 f;  v += dt/2 f  (double), then internal coordinates
@@ -545,8 +552,7 @@ __global__ __launch_bounds__(kBlock) void k_ddrift(double4* __restrict__ xd, dou
   v.z += h * f.z;
   xd[i] = x;
   vd[i] = v;
-  if (qs > 0.) q[i] = make_uint4(fixqd(x.x, qs), fixqd(x.y, qs), fixqd(x.z, qs), 0u);
-  else xf[i] = make_float4((float)x.x, (float)x.y, (float)x.z, 0.f);
+  put_coords(x, qs, q, xf, i);
 }
 
 // f = FS * sum of slices (double); kick (dt != 0): v += dt/2 f; block partials
@@ -588,9 +594,8 @@ __global__ __launch_bounds__(kBlock) void k_dkick(const float4* __restrict__ fpa
 
 // E = 2 eps sum e, W = 12 eps sum b, P = (W/3 + sum v^2 / 3) / vol;
 // acc[0] += E, acc[1] += P (accumulate != 0), acc[2] = E, acc[3] = P
-__global__ __launch_bounds__(kBlock) void k_dfinal(const double* __restrict__ blk, int nblk,
-                                                   double eps, double vol, int accumulate,
-                                                   double* __restrict__ acc)
+__device__ __forceinline__ void dfinal_block(const double* __restrict__ blk, int nblk, double eps,
+                                             double vol, int accumulate, double* __restrict__ acc)
 {
   double v[3] = {0., 0., 0.};
   for (int r = threadIdx.x; r < nblk; r += kBlock)
@@ -606,6 +611,190 @@ __global__ __launch_bounds__(kBlock) void k_dfinal(const double* __restrict__ bl
   }
   acc[2] = E;
   acc[3] = P;
+}
+
+__global__ __launch_bounds__(kBlock) void k_dfinal(const double* __restrict__ blk, int nblk,
+                                                   double eps, double vol, int accumulate,
+                                                   double* __restrict__ acc)
+{
+  dfinal_block(blk, nblk, eps, vol, accumulate, acc);
+}
+
+// ---- one-launch steps (lj_small.h): the workgroup that computes the whole
+// force, or the whole adjoint pass, on T particles also runs their update.
+// A step was four dependent launches of 2 to 5 us each (drift, force pass, slice
+// sums and kick, observables: 13.9 us at N = 2048), a state of the reverse sweep
+// two (9.0 us pass, 4.8 us sums). ----
+
+template <bool PERIODIC, int T, bool DRIFT, bool FIN>
+__global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(8))) void
+k_small_dstep(DStep a, DStep fin)
+{
+  __shared__ SmallLds<T> lds;
+  if constexpr (FIN) {
+    if (blockIdx.x == 0) {
+      if (threadIdx.x < kBlock) dfinal_block(fin.blk, fin.nrow, fin.eps, fin.vol, 1, fin.acc);
+      return;
+    }
+  }
+  const int row = (int)blockIdx.x - (FIN ? 1 : 0);
+  const int i = row * T + threadIdx.x;
+  const bool lead = threadIdx.x < T && i < a.N;
+  const Partial s = small_forces<PERIODIC, T>(lds, a.q, a.N, row * T, a.C1);
+  if (threadIdx.x >= 64) return;
+  double v3[3] = {0., 0., 0.};
+  if (lead) {
+    double4 x = a.x[i], v = a.v[i];
+    const double4 f = make_double4(a.FS * s.fx, a.FS * s.fy, a.FS * s.fz, 0.5 * (s.b - s.a));
+    a.f[i] = f;
+    const double h = 0.5 * a.dt;
+    v.x += h * f.x;
+    v.y += h * f.y;
+    v.z += h * f.z;
+    if (a.slot_x) {
+      a.slot_x[i] = x;
+      a.slot_v[i] = v;
+    }
+    v3[0] = f.w;
+    v3[1] = s.b;
+    v3[2] = v.x * v.x + v.y * v.y + v.z * v.z;
+    if constexpr (DRIFT) {  // k_ddrift
+      const double h2 = 0.5 * a.dt * a.dt;
+      x.x += a.dt * v.x + h2 * f.x;
+      x.y += a.dt * v.y + h2 * f.y;
+      x.z += a.dt * v.z + h2 * f.z;
+      v.x += h * f.x;
+      v.y += h * f.y;
+      v.z += h * f.z;
+      a.x[i] = x;
+      put_coords(x, a.qs, a.qn, nullptr, i);
+    }
+    a.v[i] = v;
+  }
+  small_row_sum<3, T>(v3);
+  if (threadIdx.x == 0) {
+    double* r = a.blk + (size_t)row * 8;
+    r[0] = v3[0];
+    r[1] = v3[1];
+    r[2] = v3[2];
+  }
+}
+
+template <int T>
+union SmallAdjLds {
+  struct {
+    uint4 q[SmallGeo<T>::CH];
+    float4 z[SmallGeo<T>::CH];
+  } j;
+  double red[12][SmallGeo<T>::E][T];
+};
+
+// mode 1: the update of u, lambda and z to state m - 1 (block partials added
+// to the rows of step.rowacc); mode 2: dL/dx0 (rows of blk).  One workgroup per
+// CU: its 46 VALU per pair and twelve sums need more than 64 registers.
+template <bool PERIODIC, int T>
+__global__ __launch_bounds__(kSmallThreads) void k_small_adj(const uint4* __restrict__ q,
+                                                             const float4* __restrict__ z,
+                                                             float4* __restrict__ zn, int N,
+                                                             float C1, float K2, AdjScales sc,
+                                                             double* __restrict__ blk, AdjStep step)
+{
+  using G = SmallGeo<T>;
+  __shared__ SmallAdjLds<T> lds;
+  const int tid = threadIdx.x, ph = tid / T, i0 = blockIdx.x * T, i = i0 + tid % T;
+  const int ic = min(i, N - 1);
+  const AdjI<PERIODIC> I = adj_lane<PERIODIC>(small_pos<PERIODIC>(q[ic]), z[ic]);
+  double t[12] = {};
+  for (int c0 = 0; c0 < N; c0 += G::CH) {
+    const int n = min(G::CH, N - c0);
+    if (c0 > 0) __syncthreads();
+#pragma unroll
+    for (int k = 0; k < G::CH; k += kSmallThreads)
+      if (k + tid < n) {
+        lds.j.q[k + tid] = q[c0 + k + tid];
+        lds.j.z[k + tid] = z[c0 + k + tid];
+      }
+    __syncthreads();
+    AdjAcc a;
+    adj_zero(a);
+    // rows of P particles, as in small_forces
+    const int rows = n / G::P;
+    const int self = i0 >= c0 && i0 < c0 + G::CH ? (i0 - c0) / G::P : -1;
+    const auto open = [&](int k0, int k1) {
+#pragma unroll 2
+      for (int k = k0; k < k1; ++k) {
+        const int j = k * G::P + ph;
+        adj_pair<PERIODIC, false>(I, small_pos<PERIODIC>(lds.j.q[j]), lds.j.z[j], 0, 0, C1, K2, a);
+      }
+    };
+    const auto guarded = [&](int k) {
+      const int j = k * G::P + ph, jc = min(j, n - 1);
+      adj_pair<PERIODIC, true>(I, small_pos<PERIODIC>(lds.j.q[jc]), lds.j.z[jc], i,
+                               j < n ? c0 + j : i, C1, K2, a);
+    };
+    if (self >= 0 && self < rows) {
+      open(0, self);
+      guarded(self);
+      open(self + 1, rows);
+    } else {
+      open(0, rows);
+    }
+    if (rows * G::P < n) guarded(rows);
+    adj_unmirror<PERIODIC>(I, a);
+    const float v[12] = {a.hx, a.hy, a.hz, a.a, a.fx, a.fy, a.fz, a.c, a.gx, a.gy, a.gz, a.s};
+#pragma unroll
+    for (int k = 0; k < 12; ++k) t[k] += v[k];
+  }
+  small_reduce<12, T>(t, lds.red);
+  if (tid >= 64) return;
+  double v[5] = {0., 0., 0., 0., 0.};
+  if (tid < T && i < N) {
+    AdjPre pre{};
+    adj_preload(i, step, pre);
+    const float4 zi = z[i];
+    const double a = t[3], c = t[7], s = t[11];
+    const double4 F = make_double4(sc.f * t[4], sc.f * t[5], sc.f * t[6], c - a);
+    const double4 H = make_double4(sc.h * t[0], sc.h * t[1], sc.h * t[2], 0.);
+    const double4 W = make_double4(sc.g * t[8], sc.g * t[9], sc.g * t[10], 0.);
+    v[0] = c - a;
+    v[1] = 2. * c - a;
+    v[2] = 24. * c - 6. * a;
+    v[3] = s;
+    v[4] = F.x * zi.x + F.y * zi.y + F.z * zi.z;
+    if (step.next_x) put_coords(pre.xn, step.qs, step.q, nullptr, i);
+    if (step.mode == 1)
+      adj_update_one(i, H, F, W, step, pre, zn);
+    else
+      step.dx0[i] = make_double4(pre.u.x + H.x, pre.u.y + H.y, pre.u.z + H.z, 0.);
+  }
+  small_row_sum<5, T>(v);
+  if (tid == 0) {
+    double* r = (step.rowacc ? step.rowacc : blk) + (size_t)blockIdx.x * 8;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) r[k] = step.rowacc ? r[k] + v[k] : v[k];
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_adj_narrow(const double4* __restrict__ d, int N,
+                                                       float4* __restrict__ out)
+{
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= N) return;
+  const double4 x = d[i];
+  out[i] = make_float4((float)x.x, (float)x.y, (float)x.z, 0.f);
+}
+
+template <bool PERIODIC, int T>
+void small_dstep_t(hipStream_t st, const DStep& a, bool drift_next, const DStep* fin)
+{
+  const dim3 g(a.nrow + (fin ? 1 : 0)), b(kSmallThreads);
+  if (drift_next) {
+    if (fin) hipLaunchKernelGGL((k_small_dstep<PERIODIC, T, true, true>), g, b, 0, st, a, *fin);
+    else hipLaunchKernelGGL((k_small_dstep<PERIODIC, T, true, false>), g, b, 0, st, a, a);
+  } else {
+    if (fin) hipLaunchKernelGGL((k_small_dstep<PERIODIC, T, false, true>), g, b, 0, st, a, *fin);
+    else hipLaunchKernelGGL((k_small_dstep<PERIODIC, T, false, false>), g, b, 0, st, a, a);
+  }
 }
 
 __global__ void k_dzero4(double* acc)
@@ -692,6 +881,51 @@ hipError_t launch_adj_pass(hipStream_t st, const ForcePlan& pl, const PairScalar
   else
     hipLaunchKernelGGL(k_adj_pass<false>, grid, dim3(kBlock), 0, st, q, posf, z, part, pl.N, pl.Npad,
                        pl.jchunk, ps.C1, K2);
+  return hipGetLastError();
+}
+
+hipError_t launch_small_dstep(hipStream_t st, int T, const DStep& a, bool drift_next,
+                              const DStep* fin)
+{
+  const bool per = a.qs > 0.;
+#define LJ_CALL(K)                                                    \
+  per ? small_dstep_t<true, K>(st, a, drift_next, fin)                \
+      : small_dstep_t<false, K>(st, a, drift_next, fin)
+  switch (T) {
+    case 4: LJ_CALL(4); break;
+    case 8: LJ_CALL(8); break;
+    case 16: LJ_CALL(16); break;
+    default: return hipErrorInvalidValue;
+  }
+#undef LJ_CALL
+  return hipGetLastError();
+}
+
+hipError_t launch_small_adj(hipStream_t st, int T, const PairScalars& ps, int N, const uint4* q,
+                            const float4* z, float4* zn, double* blk, const AdjStep& step)
+{
+  const double u = ps.periodic ? ps.L / 4294967296.0 : 1.0;
+  const float K2 = (float)(2. * u * u / (ps.sigma * ps.sigma));
+  const AdjScales sc = make_adj_scales(ps);
+  const dim3 g((N + T - 1) / T), b(kSmallThreads);
+#define LJ_CALL(K)                                                                               \
+  if (ps.periodic)                                                                               \
+    hipLaunchKernelGGL((k_small_adj<true, K>), g, b, 0, st, q, z, zn, N, ps.C1, K2, sc, blk, step); \
+  else                                                                                           \
+    hipLaunchKernelGGL((k_small_adj<false, K>), g, b, 0, st, q, z, zn, N, ps.C1, K2, sc, blk, step)
+  switch (T) {
+    case 4: LJ_CALL(4); break;
+    case 8: LJ_CALL(8); break;
+    case 16: LJ_CALL(16); break;
+    default: return hipErrorInvalidValue;
+  }
+#undef LJ_CALL
+  return hipGetLastError();
+}
+
+hipError_t launch_adj_narrow(hipStream_t st, const double4* dx0, int N, float4* out)
+{
+  hipLaunchKernelGGL(k_adj_narrow, dim3(nb(N)), dim3(kBlock), 0, st, dx0, N, out);
   return hipGetLastError();
 }
 

@@ -21,6 +21,7 @@
 // Hessian-vector product per stored state, and
 //   dL/dtheta = sum_m (dF/dtheta(x_m))^T z_m + direct terms.
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <vector>
 
@@ -32,17 +33,21 @@ using namespace lj;
 
 struct AdjState {
   int N = 0, nblk = 0;
+  int T = 0;     // particles per workgroup of the one-launch steps (0: off)
+  int rows = 0;  // block rows held: nblk, or the one-launch steps'
   int seg_cap = 0, ck_cap = 0;
   ForcePlan plan;  // pair pass geometry (adj_force_plan)
   float4* part = nullptr;
   float4* z = nullptr;
+  float4* z2 = nullptr;  // one-launch sweep: the next state's vector
   double4 *hz = nullptr, *f = nullptr, *gw = nullptr, *u = nullptr, *lv = nullptr, *dx0 = nullptr;
   double* blk = nullptr;
   double* rowacc = nullptr;  // block partials added over the reverse sweep's states
   double* scal = nullptr;
   double* theta = nullptr;
   double* acc = nullptr;                                // {sum E, sum P, E, P}
-  double4 *xd = nullptr, *vd = nullptr, *fd = nullptr;  // FP64 working state
+  double4 *xd = nullptr, *vd = nullptr, *fd = nullptr;  // FP64 working state (one block)
+  float4* dxf = nullptr;                                // dL/dx0 in float
   float4* xf = nullptr;                                 // float coordinates (open box)
   double4* ck = nullptr;   // checkpoints [ncheck][3][N] (x, v, f)
   double4* seg = nullptr;  // segment states [k+1][2][N] (x, v)
@@ -56,6 +61,7 @@ struct AdjState {
   hipGraph_t graph_k = nullptr, graph_seg = nullptr;
   hipGraphExec_t gexec_k = nullptr, gexec_seg = nullptr;
   int g_k = 0;
+  std::vector<hipEvent_t> ev;  // of a gradient's timing: four, then two per segment
 };
 
 namespace {
@@ -80,6 +86,14 @@ void adj_drop_graph(AdjState* a)
   adj_drop_kgraphs(a);
 }
 
+// whether an environment switch picks the adjoint pass
+bool adj_pass_chosen()
+{
+  for (const char* e : {"LJ_ADJ_SPLIT", "LJ_ADJ_SPLIT_WAVES", "LJ_ADJ_SLICES"})
+    if (std::getenv(e)) return true;
+  return false;
+}
+
 int adj_ensure(lj_ctx* c, int ncheck, int seg)
 {
   AdjState*& a = c->adj;
@@ -90,21 +104,25 @@ int adj_ensure(lj_ctx* c, int ncheck, int seg)
     const int N = a->N;
     a->plan = adj_force_plan(N);
     LJ_TRY(dev_alloc(&a->part, (size_t)3 * a->plan.S * a->plan.Npad));
+    if (c->small_T && !adj_pass_chosen()) a->T = c->small_T;
+    a->rows = a->T ? std::max(a->nblk, (N + a->T - 1) / a->T) : a->nblk;
     LJ_TRY(dev_alloc(&a->z, N));
+    if (a->T) LJ_TRY(dev_alloc(&a->z2, N));
     LJ_TRY(dev_alloc(&a->hz, N));
     LJ_TRY(dev_alloc(&a->f, N));
     LJ_TRY(dev_alloc(&a->gw, N));
     LJ_TRY(dev_alloc(&a->u, N));
     LJ_TRY(dev_alloc(&a->lv, N));
     LJ_TRY(dev_alloc(&a->dx0, N));
-    LJ_TRY(dev_alloc(&a->blk, (size_t)a->nblk * 8));
-    LJ_TRY(dev_alloc(&a->rowacc, (size_t)a->nblk * 8));
+    LJ_TRY(dev_alloc(&a->blk, (size_t)2 * a->rows * 8));  // two buffers
+    LJ_TRY(dev_alloc(&a->rowacc, (size_t)a->rows * 8));
     LJ_TRY(dev_alloc(&a->scal, kAdjScalars));
     LJ_TRY(dev_alloc(&a->theta, 2));
     LJ_TRY(dev_alloc(&a->acc, 4));
-    LJ_TRY(dev_alloc(&a->xd, N));
-    LJ_TRY(dev_alloc(&a->vd, N));
-    LJ_TRY(dev_alloc(&a->fd, N));
+    LJ_TRY(dev_alloc(&a->xd, (size_t)3 * N));
+    a->vd = a->xd + N;
+    a->fd = a->xd + 2 * N;
+    LJ_TRY(dev_alloc(&a->dxf, N));
     LJ_TRY(dev_alloc(&a->xf, N));
   }
   if (ncheck > a->ck_cap) {
@@ -125,9 +143,11 @@ int adj_ensure(lj_ctx* c, int ncheck, int seg)
   return LJ_OK;
 }
 
-int dcopy(lj_ctx* c, double4* dst, const double4* src)
+// k arrays of N from src to dst
+int dcopy(lj_ctx* c, double4* dst, const double4* src, int k)
 {
-  LJ_HIP(hipMemcpyAsync(dst, src, sizeof(double4) * c->cfg.N, hipMemcpyDeviceToDevice, c->stream));
+  LJ_HIP(hipMemcpyAsync(dst, src, sizeof(double4) * k * c->cfg.N, hipMemcpyDeviceToDevice,
+                        c->stream));
   return LJ_OK;
 }
 
@@ -240,6 +260,48 @@ int check_traj_args(lj_ctx* c, double dt, int nsteps)
   return LJ_OK;
 }
 
+// Steps [m0, m1) of the trajectory from its state m0 as one-launch steps: step m
+// reads the coordinates in buffer m & 1 and leaves the next ones in the other.
+// observe: their observables go to acc, each step's by an extra workgroup of the
+// next step (the trajectory's last one, m1 == M, by a launch of its own, left to
+// the caller).  slot0 >= 0: state m goes to segment slot m - slot0.
+// Plain launches: at one launch per step the host keeps ahead of the device.
+int enqueue_small_dsteps(lj_ctx* c, double dt, int m0, int m1, bool observe, int slot0)
+{
+  AdjState* a = c->adj;
+  const int N = c->cfg.N;
+  hipStream_t st = c->stream;
+  const auto step = [&](int m) {
+    DStep d;
+    d.q = m & 1 ? c->q2 : c->q;
+    d.qn = m & 1 ? c->q : c->q2;
+    d.x = a->xd;
+    d.v = a->vd;
+    d.f = a->fd;
+    if (slot0 >= 0) {
+      d.slot_x = a->seg + (size_t)2 * (m + 1 - slot0) * N;
+      d.slot_v = d.slot_x + N;
+    }
+    d.blk = a->blk + (size_t)(m & 1) * a->rows * 8;
+    d.acc = a->acc;
+    d.N = N;
+    d.nrow = (N + a->T - 1) / a->T;
+    d.dt = dt;
+    d.FS = c->ps.FS;
+    d.qs = qscale_of(c);
+    d.eps = c->cfg.eps;
+    d.vol = std::pow(c->L, 3.);
+    d.C1 = c->ps.C1;
+    return d;
+  };
+  LJ_HIP(launch_ddrift(st, a->xd, a->vd, a->fd, N, dt, qscale_of(c), m0 & 1 ? c->q2 : c->q, nullptr));
+  for (int m = m0; m < m1; ++m) {
+    const DStep prev = step(m - 1);
+    LJ_HIP(launch_small_dstep(st, a->T, step(m), m + 1 < m1, observe && m > 0 ? &prev : nullptr));
+  }
+  return LJ_OK;
+}
+
 // forward from the context state (converted to FP64): forces at x0, M steps,
 // checkpoints every k steps (k <= 0: none); out3 = {L, mean E, mean P}
 int forward(lj_ctx* c, double dt, int M, int k, double pt, double wp, double* out3)
@@ -250,29 +312,35 @@ int forward(lj_ctx* c, double dt, int M, int k, double pt, double wp, double* ou
   LJ_HIP(launch_dstate_init(st, c->pos, c->vel, N, a->xd, a->vd));
   LJ_TRY(dforces(c, st, a->xd));
   LJ_HIP(launch_dzero4(st, a->acc));
-  LJ_TRY(ensure_dgraph(c, dt));
-  if (k > 1 && a->seg_cap >= k + 1) LJ_TRY(ensure_kgraphs(c, dt, k));
-  if (k > 0) {
-    LJ_TRY(dcopy(c, a->ck, a->xd));
-    LJ_TRY(dcopy(c, a->ck + N, a->vd));
-    LJ_TRY(dcopy(c, a->ck + 2 * N, a->fd));
+  if (k > 0) LJ_TRY(dcopy(c, a->ck, a->xd, 3));
+  if (a->T) {
+    // the last checkpoint interval also leaves its states in the segment's slots
+    const int tail = k > 0 ? (M - 1) / k * k : M;
+    for (int m = 0; m < M;) {
+      const int e = k > 0 ? std::min(M, m + k) : M;
+      LJ_TRY(enqueue_small_dsteps(c, dt, m, e, true, m >= tail ? m : -1));
+      m = e;
+      if (k > 0 && m < M) LJ_TRY(dcopy(c, a->ck + (size_t)3 * (m / k) * N, a->xd, 3));
+    }
+  } else {
+    LJ_TRY(ensure_dgraph(c, dt));
+    if (k > 1 && a->seg_cap >= k + 1) LJ_TRY(ensure_kgraphs(c, dt, k));
+    // whole checkpoint intervals replay the k-step graph, the rest single steps
+    const bool runs = k > 1 && a->gexec_k && a->g_k == k;
+    for (int m = 0; m < M;) {
+      if (runs && m % k == 0 && m + k <= M) {
+        LJ_HIP(hipGraphLaunch(a->gexec_k, st));
+        m += k;
+      } else {
+        LJ_HIP(hipGraphLaunch(a->gexec, st));
+        m += 1;
+      }
+      if (k > 0 && m % k == 0 && m < M) LJ_TRY(dcopy(c, a->ck + (size_t)3 * (m / k) * N, a->xd, 3));
+    }
   }
-  // whole checkpoint intervals replay the k-step graph, the rest single steps
-  const bool runs = k > 1 && a->gexec_k && a->g_k == k;
-  for (int m = 0; m < M;) {
-    if (runs && m % k == 0 && m + k <= M) {
-      LJ_HIP(hipGraphLaunch(a->gexec_k, st));
-      m += k;
-    } else {
-      LJ_HIP(hipGraphLaunch(a->gexec, st));
-      m += 1;
-    }
-    if (k > 0 && m % k == 0 && m < M) {
-      double4* slot = a->ck + (size_t)3 * (m / k) * N;
-      LJ_TRY(dcopy(c, slot, a->xd));
-      LJ_TRY(dcopy(c, slot + N, a->vd));
-      LJ_TRY(dcopy(c, slot + 2 * N, a->fd));
-    }
+  if (a->T) {  // the last step's observables
+    const double* blk = a->blk + (size_t)((M - 1) & 1) * a->rows * 8;
+    LJ_HIP(launch_dfinal(st, blk, (N + a->T - 1) / a->T, c->cfg.eps, std::pow(c->L, 3.), 1, a->acc));
   }
   double acc[4];
   LJ_HIP(hipMemcpyAsync(acc, a->acc, sizeof(acc), hipMemcpyDeviceToHost, st));
@@ -309,6 +377,9 @@ void adj_free(lj_ctx* c)
   adj_drop_graph(a);
   dev_free(a->part);
   dev_free(a->z);
+  dev_free(a->z2);
+  dev_free(a->dxf);
+  for (hipEvent_t e : a->ev) (void)hipEventDestroy(e);
   dev_free(a->hz);
   dev_free(a->f);
   dev_free(a->gw);
@@ -321,8 +392,6 @@ void adj_free(lj_ctx* c)
   dev_free(a->theta);
   dev_free(a->acc);
   dev_free(a->xd);
-  dev_free(a->vd);
-  dev_free(a->fd);
   dev_free(a->xf);
   dev_free(a->ck);
   dev_free(a->seg);
@@ -419,15 +488,18 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
   AdjState* a = c->adj;
   const int N = c->cfg.N;
   hipStream_t st = c->stream;
-  hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-  for (auto& e : ev) LJ_HIP(hipEventCreate(&e));
+  while (a->ev.size() < (size_t)4 + 2 * ncheck) {
+    hipEvent_t e = nullptr;
+    LJ_HIP(hipEventCreate(&e));
+    a->ev.push_back(e);
+  }
+  const std::vector<hipEvent_t>& ev = a->ev;
   int rc = LJ_OK;
   auto check = [&](hipError_t e) {
     if (e != hipSuccess && rc == LJ_OK)
       rc = fail(LJ_ERR_DEVICE, "lj_trajectory_grad: %s", hipGetErrorString(e));
     return rc == LJ_OK;
   };
-  float recompute_ms = 0.f;
   if (check(hipEventRecord(ev[0], st)) && (rc = forward(c, dt, M, k, p_target, w_p, out3)) == LJ_OK &&
       check(hipEventRecord(ev[1], st))) {
     const double vol = std::pow(c->L, 3.);
@@ -439,36 +511,40 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
     // the block partials of the states m >= 1 add up in rowacc; one finaliser
     // turns their total into the eps / sigma terms at the end of the sweep
     check(launch_fill_u64(st, reinterpret_cast<unsigned long long*>(a->rowacc),
-                          (int)((size_t)a->nblk * 8)));
+                          (int)((size_t)a->rows * 8)));
+    const int nrow = a->T ? (N + a->T - 1) / a->T : a->nblk;
     bool first = true;
     bool prepped = false;  // the next pass's coordinates prepared by the last reduction
+    int par = 0;           // one-launch sweep: the buffers of the current coordinates and z
     for (int cseg = ncheck - 1; cseg >= 0 && rc == LJ_OK; --cseg) {
       const int s0 = cseg * k, s1 = std::min(M, s0 + k);
-      // recompute the segment's states s0..s1 from its checkpoint
-      if (!check(hipEventRecord(ev[2], st))) break;
+      // recompute the segment's states s0+1..s1 from its checkpoint (the
+      // one-launch forward run left those of the last segment)
+      if (!check(hipEventRecord(ev[4 + 2 * cseg], st))) break;
       const double4* ckp = a->ck + (size_t)3 * cseg * N;
-      if ((rc = dcopy(c, a->xd, ckp)) || (rc = dcopy(c, a->vd, ckp + N)) || (rc = dcopy(c, a->fd, ckp + 2 * N)))
-        break;
-      if ((rc = dcopy(c, a->seg, a->xd)) || (rc = dcopy(c, a->seg + N, a->vd))) break;
-      if (s1 - s0 == k && a->gexec_seg && a->g_k == k) {
-        check(hipGraphLaunch(a->gexec_seg, st));  // k steps, each state into its slot
-      } else {
-        for (int m = s0 + 1; m <= s1 && rc == LJ_OK; ++m) {
-          if (!check(hipGraphLaunch(a->gexec, st))) break;
-          double4* slot = a->seg + (size_t)2 * (m - s0) * N;
-          if ((rc = dcopy(c, slot, a->xd)) || (rc = dcopy(c, slot + N, a->vd))) break;
+      if (!(a->T && cseg == ncheck - 1)) {
+        if ((rc = dcopy(c, a->xd, ckp, 3))) break;
+        if (a->T) {
+          rc = enqueue_small_dsteps(c, dt, s0, s1, false, s0);
+        } else if (s1 - s0 == k && a->gexec_seg && a->g_k == k) {
+          check(hipGraphLaunch(a->gexec_seg, st));  // k steps, each state into its slot
+        } else {
+          for (int m = s0 + 1; m <= s1 && rc == LJ_OK; ++m) {
+            if (!check(hipGraphLaunch(a->gexec, st))) break;
+            rc = dcopy(c, a->seg + (size_t)2 * (m - s0) * N, a->xd, 2);
+          }
         }
       }
-      if (rc || !check(hipEventRecord(ev[3], st)) || !check(hipEventSynchronize(ev[3]))) break;
-      float ms = 0.f;
-      if (!check(hipEventElapsedTime(&ms, ev[2], ev[3]))) break;
-      recompute_ms += ms;
+      if (rc || !check(hipEventRecord(ev[5 + 2 * cseg], st))) break;
+      // state m of the segment: positions, then velocities
+      const auto state = [&](int m) { return m == s0 ? ckp : a->seg + (size_t)2 * (m - s0) * N; };
       // reverse over m = s1 .. s0+1 (and m = 0 in the first segment)
       const int mlow = cseg == 0 ? 0 : s0 + 1;
       for (int m = s1; m >= mlow && rc == LJ_OK; --m) {
-        const double4* xm = a->seg + (size_t)2 * (m - s0) * N;
+        const double4* xm = state(m);
+        float4* z = par ? a->z2 : a->z;
         if (first) {
-          if (!check(launch_adj_init(st, xm + N, N, gv, dt, a->u, a->lv, a->z))) break;
+          if (!check(launch_adj_init(st, xm + N, N, gv, dt, a->u, a->lv, z))) break;
           first = false;
         }
         // the pass, then (fused into its reduction and finaliser) the update of
@@ -481,7 +557,7 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
         step.gv = gv;
         step.dt = dt;
         step.last = m - 1 == 0;
-        step.vel_prev = (m - 1 >= 1) ? a->seg + (size_t)2 * (m - 1 - s0) * N + N : nullptr;
+        step.vel_prev = (m - 1 >= 1) ? state(m - 1) + N : nullptr;
         step.u = a->u;
         step.lv = a->lv;
         step.dx0 = a->dx0;
@@ -492,12 +568,23 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
         // the next state of this segment (the next segment's are recomputed
         // first, which overwrites the coordinates)
         if (m - 1 >= mlow) {
-          step.next_x = a->seg + (size_t)2 * (m - 1 - s0) * N;
+          step.next_x = state(m - 1);
           step.qs = qscale_of(c);
-          step.q = c->q;
+          step.q = a->T && !par ? c->q2 : c->q;
           step.xf = a->xf;
         }
-        if ((rc = adj_pass_d(c, xm, !prepped, st, step)) != LJ_OK) break;
+        if (a->T) {
+          uint4* q = par ? c->q2 : c->q;
+          if (!prepped && !check(launch_dprep(st, xm, N, qscale_of(c), q, nullptr))) break;
+          if (!check(launch_small_adj(st, a->T, c->ps, N, q, z, par ? a->z : a->z2, a->blk, step)))
+            break;
+          if (!step.rowacc &&
+              !check(launch_adj_finalize(st, a->blk, nrow, make_adj_scales(c->ps), a->scal, step)))
+            break;
+          par ^= 1;
+        } else if ((rc = adj_pass_d(c, xm, !prepped, st, step)) != LJ_OK) {
+          break;
+        }
         prepped = step.next_x != nullptr;
       }
       prepped = false;
@@ -509,29 +596,25 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
       fin.cw = cw;
       fin.direct = 1;
       fin.g = a->theta;
-      check(launch_adj_finalize(st, a->rowacc, a->nblk, make_adj_scales(c->ps), a->scal, fin));
+      check(launch_adj_finalize(st, a->rowacc, nrow, make_adj_scales(c->ps), a->scal, fin));
     }
   }
   if (rc == LJ_OK && check(hipEventRecord(ev[3], st)) &&
       check(hipMemcpyAsync(grad_eps_sigma, a->theta, 2 * sizeof(double), hipMemcpyDeviceToHost, st))) {
     if (dx0_host4 || d_dx0_4) {
-      std::vector<double4> h(N);
-      std::vector<float> hf((size_t)4 * N);
-      if (check(hipMemcpyAsync(h.data(), a->dx0, sizeof(double4) * N, hipMemcpyDeviceToHost, st)) &&
-          check(hipStreamSynchronize(st))) {
-        for (int i = 0; i < N; ++i) {
-          hf[4 * i] = (float)h[i].x;
-          hf[4 * i + 1] = (float)h[i].y;
-          hf[4 * i + 2] = (float)h[i].z;
-          hf[4 * i + 3] = 0.f;
-        }
-        if (dx0_host4) std::memcpy(dx0_host4, hf.data(), sizeof(float) * 4 * N);
-        if (d_dx0_4)
-          check(hipMemcpyAsync(d_dx0_4, hf.data(), sizeof(float) * 4 * N, hipMemcpyHostToDevice, st));
-      }
+      check(launch_adj_narrow(st, a->dx0, N, a->dxf));
+      if (dx0_host4)
+        check(hipMemcpyAsync(dx0_host4, a->dxf, sizeof(float4) * N, hipMemcpyDeviceToHost, st));
+      if (d_dx0_4)
+        check(hipMemcpyAsync(d_dx0_4, a->dxf, sizeof(float4) * N, hipMemcpyDeviceToDevice, st));
     }
     if (check(hipStreamSynchronize(st)) && times_ms3) {
-      float f_ms = 0.f, all_ms = 0.f;
+      float f_ms = 0.f, all_ms = 0.f, recompute_ms = 0.f;
+      for (int g = 0; g < ncheck; ++g) {
+        float ms = 0.f;
+        check(hipEventElapsedTime(&ms, ev[4 + 2 * g], ev[5 + 2 * g]));
+        recompute_ms += ms;
+      }
       check(hipEventElapsedTime(&f_ms, ev[0], ev[1]));
       check(hipEventElapsedTime(&all_ms, ev[1], ev[3]));
       times_ms3[0] = f_ms;
@@ -539,8 +622,6 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
       times_ms3[2] = all_ms - recompute_ms;
     }
   }
-  for (auto& e : ev)
-    if (e) (void)hipEventDestroy(e);
   return rc;
 }
 

@@ -59,6 +59,40 @@ __device__ __forceinline__ PosT<PERIODIC> small_pos(const uint4& v)
   return p;
 }
 
+// Totals of NV sums over the workgroup's lanes of each particle, left in every
+// lane of wave 0 (lane % T: the particle); the other waves leave with undefined
+// sums and no barrier follows.  The lanes' other LDS data is done with.
+template <int NV, int T>
+__device__ __forceinline__ void small_reduce(double (&d)[NV],
+                                             double (*red)[SmallGeo<T>::E][T])
+{
+  using G = SmallGeo<T>;
+  const int tid = threadIdx.x;
+  // the phases of a row of 16 lanes, then the rows through LDS
+#pragma unroll
+  for (int c = 0; c < NV; ++c) {
+    if constexpr (T <= 8) d[c] += row_ror<8>(d[c]);
+    if constexpr (T <= 4) d[c] += row_ror<4>(d[c]);
+  }
+  __syncthreads();
+  if (tid % 16 < T)
+#pragma unroll
+    for (int c = 0; c < NV; ++c) red[c][tid / 16][tid % T] = d[c];
+  __syncthreads();
+  if (tid >= 64) return;
+  constexpr int EG = G::E * T / 64;  // rows per lane
+#pragma unroll
+  for (int c = 0; c < NV; ++c) d[c] = 0.;
+#pragma unroll
+  for (int e = 0; e < EG; ++e)
+#pragma unroll
+    for (int c = 0; c < NV; ++c) d[c] += red[c][(tid / T) * EG + e][tid % T];
+#pragma unroll
+  for (int o = T; o < 64; o <<= 1)
+#pragma unroll
+    for (int c = 0; c < NV; ++c) d[c] += __shfl_xor(d[c], o, 64);
+}
+
 // Sums over all j of the pairs of particle i0 + lane % T, returned in every
 // lane of wave 0 (the other waves return with undefined sums; no barrier
 // follows).  i0 is a multiple of T; q holds the box's N particles.
@@ -108,35 +142,8 @@ __device__ __forceinline__ Partial small_forces(SmallLds<T>& lds, const uint4* _
     d[3] += a.a;
     d[4] += a.b;
   }
-  // the phases of a row of 16 lanes, then the rows through LDS
-#pragma unroll
-  for (int c = 0; c < 5; ++c) {
-    if constexpr (T <= 8) d[c] += row_ror<8>(d[c]);
-    if constexpr (T <= 4) d[c] += row_ror<4>(d[c]);
-  }
-  __syncthreads();
-  if (tid % 16 < T)
-#pragma unroll
-    for (int c = 0; c < 5; ++c) lds.red[c][tid / 16][tid % T] = d[c];
-  __syncthreads();
-  Partial p{0., 0., 0., 0., 0.};
-  if (tid >= 64) return p;
-  constexpr int EG = G::E * T / 64;  // rows per lane
-  double s[5] = {0., 0., 0., 0., 0.};
-#pragma unroll
-  for (int e = 0; e < EG; ++e)
-#pragma unroll
-    for (int c = 0; c < 5; ++c) s[c] += lds.red[c][(tid / T) * EG + e][tid % T];
-#pragma unroll
-  for (int o = T; o < 64; o <<= 1)
-#pragma unroll
-    for (int c = 0; c < 5; ++c) s[c] += __shfl_xor(s[c], o, 64);
-  p.fx = s[0];
-  p.fy = s[1];
-  p.fz = s[2];
-  p.a = s[3];
-  p.b = s[4];
-  return p;
+  small_reduce<5, T>(d, lds.red);
+  return Partial{d[0], d[1], d[2], d[3], d[4]};
 }
 
 // totals of NV values over the T lead lanes of wave 0 (the others hold zeros)

@@ -1,4 +1,4 @@
-"""The one-launch time step of small boxes (N <= 4096 without an explicit choice
+"""The one-launch time step and trajectory gradient of small boxes (N <= 4096 without an explicit choice
 of force pass) at the edges of its tiles: box sizes around the particle counts
 at which its tile (4, 8, 16 particles per workgroup) and its LDS chunk (2048
 particles) change, against the reference CPU path restated in the oracle."""
@@ -7,7 +7,7 @@ import pytest
 
 import ljamd
 from helpers import perturbed_state, xyz
-from oracle_lib import OracleSystem
+from oracle_lib import OracleSystem, traj_grad_fp64
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +49,26 @@ def test_small_step_edges(N, canon, bc):
         # the step's V and W are those of a separate evaluation at its positions
         assert abs(obs["V"] - full["V"]) <= 2e-6 * N * scale
         assert abs(obs["W"] - full["W"]) <= 1e-5 * max(abs(full["W"]), N * scale)
+
+
+@pytest.mark.parametrize("bc", [ljamd.BC_PERIODIC, ljamd.BC_NONE])
+@pytest.mark.parametrize("N,M,k", [(2, 6, 4), (17, 5, 5), (1025, 6, 4), (2049, 4, 1), (4096, 4, 3)])
+def test_small_gradient_edges(N, M, k, bc):
+    """Forward, recompute and reverse sweep in one-launch steps (the last
+    checkpoint interval whole, partial, one step long and the only one) against
+    the FP64 adjoint, with the tolerances of test_gpu_adjoint.py."""
+    rho, dt = (0.1 if N < 64 else 0.6), 0.004
+    L, pos, vel = perturbed_state(N, rho, 1.0, seed=67)
+    print(f"\n[case] small gradient N={N} M={M} k={k} bc={bc}", flush=True)
+    with ljamd.LJSystem(N, rho, 1.0, boundary=bc) as s:
+        s.set_state(pos, vel)
+        loss = s.trajectory_loss(dt, M)
+        out, g2, dx0, _ = s.trajectory_grad(dt, M, k)
+        again = s.trajectory_grad(dt, M, M)
+    assert np.array_equal(out, loss)
+    assert np.array_equal(g2, again[1]) and np.array_equal(dx0, again[2])
+    ref, ref_g2, ref_dx = traj_grad_fp64(xyz(pos), xyz(vel), L, int(bc == ljamd.BC_PERIODIC), 1.0, 1.0,
+                                         dt, M)
+    assert abs(out[0] - ref[0]) <= 1e-5 * abs(ref[0])
+    assert np.all(np.abs(g2 - ref_g2) <= 1e-4 * np.abs(ref_g2) + 1e-6)
+    assert np.linalg.norm(dx0[:, :3] - ref_dx) <= 1e-4 * np.linalg.norm(ref_dx) + 1e-6
