@@ -78,7 +78,7 @@ StepArgs step_args(lj_ctx* c, double dt, int b = 0)
   a.q = c->q;
   a.fpart = c->fpart;
   a.apart = c->apart;
-  a.blk = c->blk + (is_fp64(c) ? 0 : (size_t)b * blk_rows(c) * kBlkFields);
+  a.blk = c->blk + (size_t)b * blk_rows(c) * kBlkFields;
   a.obs = c->obs;
   a.hist = c->hist;
   a.hist_base = c->hist_base;
@@ -97,7 +97,7 @@ StepArgs step_args(lj_ctx* c, double dt, int b = 0)
   a.Npad = fplan(c).Npad;
   a.ew = c->step_ew ? c->step_ew + (size_t)b * 2 * c->plan3.step_wgs() : nullptr;
   a.nitems = c->step_ew ? c->plan3.step_wgs() : 0;
-  a.nrow = is_fp64(c) ? c->nblk : step_rows(c->cfg.N);
+  a.nrow = step_rows(c->cfg.N);
   if (c->small_T) {
     // one-launch steps: EVN alternates between the two coordinate buffers, TVN
     // (whose coordinates a launch of their own writes) keeps to one
@@ -127,7 +127,8 @@ void refresh_scalars(lj_ctx* c)
                             false);
 }
 
-Step64 step64_args(lj_ctx* c, double dt)
+// b: the block-row buffer the step fills, as for step_args
+Step64 step64_args(lj_ctx* c, double dt, int b = 0)
 {
   Step64 a{};
   a.x = c->xd;
@@ -138,11 +139,13 @@ Step64 step64_args(lj_ctx* c, double dt)
   a.vel = c->vel;
   a.force = c->force;
   a.part = c->part64;
-  a.apart = c->apart64;
-  a.blk = c->blk;
+  a.wt = c->wt64;
+  a.nwt = force64_totals(c->plan64);
+  a.blk = c->blk + (size_t)b * blk_rows(c) * kBlkFields;
+  a.nrow = step_rows(c->cfg.N);
   a.N = c->cfg.N;
-  a.S = c->plan.S;
-  a.Npad = c->plan.Npad;
+  a.S = c->plan64.S;
+  a.Npad = c->plan64.Npad;
   a.bc = c->cfg.boundary;
   a.dt = dt;
   a.L = c->L;
@@ -158,23 +161,26 @@ double4* state64(lj_ctx* c, int type)
 
 hipError_t enqueue_force64(lj_ctx* c, hipStream_t st)
 {
-  return launch_force64(st, c->plan, c->xd, c->cfg.boundary == LJ_BC_PERIODIC, c->L,
-                        c->cfg.sigma, c->part64, c->apart64);
+  return launch_force64(st, c->plan64, c->xd, c->cfg.boundary == LJ_BC_PERIODIC, c->L,
+                        c->cfg.sigma, c->part64, c->wt64);
 }
 
-// the FP64 step: MDSystem.cpp:442-510 in double
-int enqueue_step64(lj_ctx* c, hipStream_t st, double dt)
+// one FP64 step of a run (MDSystem.cpp:442-510 in double), fused across steps
+// as enqueue_step_part's
+int enqueue_step64(lj_ctx* c, hipStream_t st, double dt, bool first, bool last, int b)
 {
-  const Step64 a = step64_args(c, dt);
-  LJ_HIP(launch_drift64(st, a, c->cfg.canonical));
+  const Step64 a = step64_args(c, dt, b);
+  if (first) LJ_HIP(launch_drift64(st, a, c->cfg.canonical));
   LJ_HIP(enqueue_force64(c, st));
+  const StepArgs prev = step_args(c, dt, b ^ 1);
+  const StepArgs* fin = first ? nullptr : &prev;
   if (c->cfg.canonical == LJ_EVN) {
-    LJ_HIP(launch_kick64(st, a));
+    LJ_HIP(launch_kick64(st, a, !last, fin));
   } else {
-    LJ_HIP(launch_tvn64_a(st, a));
-    LJ_HIP(launch_tvn64_b(st, a));
+    LJ_HIP(launch_tvn64_a(st, a, fin));
+    LJ_HIP(launch_tvn64_b(st, a, !last));
   }
-  LJ_HIP(launch_finalize_step(st, step_args(c, dt)));
+  if (last) LJ_HIP(launch_finalize_step(st, step_args(c, dt, b)));
   // the float mirrors the step kernels wrote are the sampled state
   if (c->smp_fl) LJ_HIP(launch_fl_sample(st, c->fl, c->pos, c->vel, c->cfg.N, nullptr, nullptr, 0));
   return LJ_OK;
@@ -232,7 +238,7 @@ int enqueue_small_step(lj_ctx* c, hipStream_t st, double dt, bool first, bool la
 // so a run gives the bits of single steps.
 int enqueue_step_part(lj_ctx* c, hipStream_t st, double dt, bool first, bool last, int b)
 {
-  if (is_fp64(c)) return enqueue_step64(c, st, dt);
+  if (is_fp64(c)) return enqueue_step64(c, st, dt, first, last, b);
   if (c->small_T) return enqueue_small_step(c, st, dt, first, last, b);
   const StepArgs a = step_args(c, dt, b);
   const bool comp = c->cfg.precision == LJ_PREC_COMPENSATED;
@@ -361,7 +367,8 @@ int compute_forces_internal(lj_ctx* c)
     LJ_TRY(enqueue_force(c, st, c->pos));
     LJ_HIP(launch_reduce_forces(st, fplan(c), c->ps, c->fpart, c->apart, c->force, c->blk));
   }
-  LJ_HIP(launch_finalize_forces(st, c->blk, c->nblk, c->cfg.eps, c->ev, nullptr));
+  LJ_HIP(launch_finalize_forces(st, c->blk, is_fp64(c) ? step_rows(c->cfg.N) : c->nblk, c->cfg.eps,
+                                c->ev, nullptr));
   // V and W into the observables block (CalculateForces sets V and P, MDSystem.cpp:257-309)
   LJ_HIP(launch_store_vw(st, c->ev, c->obs));
   return LJ_OK;
@@ -437,7 +444,7 @@ int lj_destroy(lj_ctx* c)
   dev_free(c->fd);
   dev_free(c->tfd);
   dev_free(c->part64);
-  dev_free(c->apart64);
+  dev_free(c->wt64);
   fl_free(c->fl);
   dev_free(c->rdf_step);
   dev_free(c->step_tab);
@@ -482,6 +489,7 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
     else if (cfg->precision == LJ_PREC_COMPENSATED && n3_comp_enabled())
       c->plan3 = make_n3_plan(cfg->N, true);
   }
+  if (is_fp64(c)) c->plan64 = make_plan64(cfg->N, cfg->jslices);
   // the one-launch step unless an explicit choice of force pass asks for it
   if (cfg->jslices == 0 && !is_fp64(c) && !force_pass_chosen()) c->small_T = small_tile(cfg->N);
   const size_t npart = (size_t)std::max(c->plan.S, c->plan3.S) * c->plan.Npad;
@@ -501,11 +509,12 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
   if (c->small_T) A(dev_alloc(&c->q2, N));
   A(dev_alloc(&c->fpart, npart));
   A(dev_alloc(&c->apart, npart));
-  if (c->plan3.n3) {
+  ForcePlan& pn = is_fp64(c) ? c->plan64 : c->plan3;
+  if (pn.n3) {
     // the full variant's items, then the time step's
-    std::vector<int2> it((size_t)c->plan3.nitems + c->plan3.nitems_step);
-    n3_items(c->plan3.ng, it.data());
-    n3_step_items(c->plan3, it.data() + c->plan3.nitems);
+    std::vector<int2> it((size_t)pn.nitems + pn.nitems_step);
+    n3_items(pn.ng, it.data());
+    n3_step_items(pn, it.data() + pn.nitems);
     A(dev_alloc(&c->n3items, it.size()));
     // copies on the context's stream: a null-stream copy can break another
     // thread's stream capture
@@ -514,9 +523,9 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
                         c->stream) != hipSuccess ||
          hipStreamSynchronize(c->stream) != hipSuccess))
       A(fail(LJ_ERR_DEVICE, "item table upload failed"));
-    c->plan3.items = c->n3items;
-    c->plan3.items_step = c->n3items + c->plan3.nitems;
-    A(dev_alloc(&c->step_ew, (size_t)4 * c->plan3.step_wgs()));  // two buffers
+    pn.items = c->n3items;
+    pn.items_step = c->n3items + pn.nitems;
+    if (!is_fp64(c)) A(dev_alloc(&c->step_ew, (size_t)4 * pn.step_wgs()));  // two buffers
   }
   // rows: nblk for the per-block kernels, step_rows(N) >= nblk for the step
   A(dev_alloc(&c->blk, 2 * blk_rows(c) * kBlkFields));
@@ -528,8 +537,8 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
     A(dev_alloc(&c->vd, N));
     A(dev_alloc(&c->fd, N));
     A(dev_alloc(&c->tfd, N));
-    A(dev_alloc(&c->part64, (size_t)c->plan.S * c->plan.Npad));
-    A(dev_alloc(&c->apart64, (size_t)c->plan.S * c->plan.Npad));
+    A(dev_alloc(&c->part64, (size_t)c->plan64.S * c->plan64.Npad));
+    A(dev_alloc(&c->wt64, force64_totals(c->plan64)));
   }
   if (rc == LJ_OK && hipEventCreate(&c->e0) != hipSuccess) A(fail(LJ_ERR_DEVICE, "hipEventCreate"));
   if (rc == LJ_OK && hipEventCreate(&c->e1) != hipSuccess) A(fail(LJ_ERR_DEVICE, "hipEventCreate"));
@@ -1142,7 +1151,7 @@ int lj_time_force_kernel(lj_ctx* c, int reps, double* us)
 int lj_force_plan_info(lj_ctx* c, int* pair_once, int* nslots)
 {
   if (!c) return fail(LJ_ERR_ARG, "null context");
-  const ForcePlan& pl = is_fp64(c) ? c->plan : fplan(c);
+  const ForcePlan& pl = is_fp64(c) ? c->plan64 : fplan(c);
   if (pair_once) *pair_once = pl.n3;
   if (nslots) *nslots = pl.S;
   return LJ_OK;

@@ -13,7 +13,8 @@ struct lj_ctx {
   double L = 0.;
   hipStream_t stream = nullptr;
   lj::ForcePlan plan;   // sliced force pass (also the adjoint pass geometry)
-  lj::ForcePlan plan3;  // pair-once force pass, when enabled (FP32 mode, large N)
+  lj::ForcePlan plan3;  // pair-once force pass, when enabled (FP32 modes, large N)
+  lj::ForcePlan plan64;  // force pass of the FP64 mode
   int2* n3items = nullptr;
   double* step_ew = nullptr;  // per-workgroup (E, W) of the step's pair-once pass
   lj::PairScalars ps;
@@ -72,7 +73,7 @@ struct lj_ctx {
   double4* fd = nullptr;
   double4* tfd = nullptr;
   double4* part64 = nullptr;
-  double* apart64 = nullptr;
+  double* wt64 = nullptr;  // the force pass's totals of the virial
   // fluctuation counters (lj_fl_*)
   lj::FlSampler fl;
   // sampling inside the step graphs (lj_set_step_sampling)

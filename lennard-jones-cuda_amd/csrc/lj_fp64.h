@@ -14,21 +14,30 @@ struct Step64 {
   float4* pos;       // FP32 mirrors of the state at the boundary
   float4* vel;
   float4* force;
-  const double4* part;  // slice partials (fx, fy, fz, b)
-  const double* apart;  // slice partials a
-  double* blk;
+  const double4* part;  // partial entries (fx, fy, fz, m), e_i = -sum m / 2
+  const double* wt;     // the force pass's nwt totals of w (virial)
+  int nwt;
+  double* blk;          // nrow rows, one per kRowParticles particles
+  int nrow;
   int N, S, Npad, bc;
   double dt, L, T0, FS;
 };
 
+// plan of the pass: pair-once (n3 != 0; items: the ng (ng + 1) / 2 group pairs
+// of n3_items) or sliced
+ForcePlan make_plan64(int N, int jslices);
+// totals of w that a pass of this plan writes
+int force64_totals(const ForcePlan& pl);
 hipError_t launch_force64(hipStream_t st, const ForcePlan& pl, const double4* x, bool periodic,
-                          double L, double sigma, double4* part, double* apart);
-// slice sums -> f, FP32 force mirror, block partials (E, B)
+                          double L, double sigma, double4* part, double* wt);
+// partial sums -> f, FP32 force mirror, block partials (E, B)
 hipError_t launch_reduce64(hipStream_t st, const Step64& a);
 hipError_t launch_drift64(hipStream_t st, const Step64& a, int canonical);
-hipError_t launch_kick64(hipStream_t st, const Step64& a);
-hipError_t launch_tvn64_a(hipStream_t st, const Step64& a);
-hipError_t launch_tvn64_b(hipStream_t st, const Step64& a);
+// drift_next: also the next step's drift (no FP32 mirrors of this state then);
+// fin: one extra block computes the observables of the run's previous step
+hipError_t launch_kick64(hipStream_t st, const Step64& a, bool drift_next, const StepArgs* fin);
+hipError_t launch_tvn64_a(hipStream_t st, const Step64& a, const StepArgs* fin);
+hipError_t launch_tvn64_b(hipStream_t st, const Step64& a, bool drift_next);
 // float4 -> double4 (state upload through the FP32 arrays) and back
 hipError_t launch_widen(hipStream_t st, const float4* src, double4* dst, int N);
 hipError_t launch_narrow(hipStream_t st, const double4* src, float4* dst, int N);

@@ -155,3 +155,48 @@ def test_precision_workload_modes_full_size():
         assert fe <= 2.5e-6 and dE <= 1.2e-6 and dP <= 3.5e-5
     # the compensated per-particle sums are the more accurate ones
     assert errs["compensated"] <= errs["fp32"]
+
+
+@pytest.mark.parametrize("bc", [ljamd.BC_PERIODIC, ljamd.BC_WALL, ljamd.BC_NONE])
+@pytest.mark.parametrize("N,pair_once", [(4096, False), (4097, True), (4353, True), (16384, True),
+                                         (16641, True)])
+def test_forces_fp64_pair_once(N, pair_once, bc):
+    """Every pair once from N = 4097 on: a last group of one particle (4097,
+    split items; 16641, whole items), of one particle over a whole group (4353)
+    and none; forces, per-particle energies, E and W as test_forces_fp64, and V
+    and W of a step against an evaluation at its positions."""
+    rho = 0.7
+    L, pos, vel = perturbed_state(N, rho, 1.0, seed=71)
+    x = xyz(pos) + np.random.default_rng(3).uniform(-1e-3, 1e-3, (N, 3))
+    print(f"\n[case] fp64 pair-once N={N} bc={bc}", flush=True)
+    with ljamd.LJSystem(N, rho, 1.0, boundary=bc, eps=1.3, sigma=0.9, precision=ljamd.PREC_FP64) as s:
+        assert s.force_plan()[0] == pair_once
+        s.set_array_f64(ljamd.ARRAY_POS, _x4(x))
+        s.set_array(ljamd.ARRAY_VEL, vel)
+        obs = s.CalculateForces()
+        f = s.get_array_f64(ljamd.ARRAY_FORCE).reshape(N, 4)
+        s.Integrate(0.004, 9)
+        step = s.observables()
+        full = s.CalculateForces()
+    F, ew, E, W = forces_fp64d(x, L, bc == ljamd.BC_PERIODIC, 1.3, 0.9)
+    assert np.linalg.norm(f[:, :3] - F) <= 1e-12 * np.linalg.norm(F)
+    assert abs(obs["V"] - E) <= 1e-12 * abs(E) and abs(obs["W"] - W) <= 1e-11 * abs(W)
+    assert np.max(np.abs(f[:, 3] - ew[:, 0])) <= 1e-12 * np.max(np.abs(ew[:, 0]))
+    assert abs(step["V"] - full["V"]) <= 1e-12 * abs(full["V"])
+    assert abs(step["W"] - full["W"]) <= 1e-11 * abs(full["W"])
+
+
+@pytest.mark.parametrize("canon,bc", [(ljamd.EVN, ljamd.BC_WALL), (ljamd.TVN, ljamd.BC_PERIODIC)])
+@pytest.mark.parametrize("N", [700, 4097])
+def test_fp64_runs_split_anywhere(N, canon, bc):
+    # 41 steps as 32 + 8 + 1, 9 + 32 and 7 + 13 + 21: the same bits
+    outs = []
+    for chunks in ([41], [9, 32], [7, 13, 21]):
+        with ljamd.LJSystem(N, 0.6, 1.0, canonical=canon, boundary=bc, seed=8,
+                            precision=ljamd.PREC_FP64) as s:
+            h = np.concatenate([s.Integrate(0.004, c) for c in chunks])
+            outs.append((h, s.get_array_f64(ljamd.ARRAY_POS), s.get_array_f64(ljamd.ARRAY_VEL),
+                         s.get_array_f64(ljamd.ARRAY_FORCE), s.pos, s.vel, s.force))
+    for o in outs[1:]:
+        for a, b in zip(outs[0], o):
+            assert np.array_equal(a, b)
