@@ -151,7 +151,33 @@ Step64 step64_args(lj_ctx* c, double dt, int b = 0)
   a.L = c->L;
   a.T0 = c->cfg.T0;
   a.FS = 24. * c->cfg.eps / (c->cfg.sigma * c->cfg.sigma);
+  a.sigma = c->cfg.sigma;
   return a;
+}
+
+// one FP64 step of a run in the one-launch form (see enqueue_small_step)
+int enqueue_small_step64(lj_ctx* c, hipStream_t st, double dt, bool first, bool last, int b)
+{
+  Step64 a = step64_args(c, dt, b);
+  const StepArgs s = step_args(c, dt, b), prev = step_args(c, dt, b ^ 1);
+  const StepArgs* fin = first ? nullptr : &prev;
+  a.nrow = s.nrow;
+  if (first) {
+    a.xn = b ? c->xs2 : c->xs;
+    LJ_HIP(launch_small_drift64(st, a, c->cfg.canonical));
+  }
+  if (c->cfg.canonical == LJ_EVN) {
+    a.xs = b ? c->xs2 : c->xs;
+    a.xn = b ? c->xs : c->xs2;
+    LJ_HIP(launch_small64_evn(st, c->small_T, a, !last, fin));
+  } else {
+    a.xs = a.x;  // which only the second launch writes
+    LJ_HIP(launch_small64_tvn(st, c->small_T, a, fin));
+    LJ_HIP(launch_tvn64_b(st, a, !last));
+  }
+  if (last) LJ_HIP(launch_finalize_step(st, s));
+  if (c->smp_fl) LJ_HIP(launch_fl_sample(st, c->fl, c->pos, c->vel, c->cfg.N, nullptr, nullptr, 0));
+  return LJ_OK;
 }
 
 double4* state64(lj_ctx* c, int type)
@@ -169,6 +195,7 @@ hipError_t enqueue_force64(lj_ctx* c, hipStream_t st)
 // as enqueue_step_part's
 int enqueue_step64(lj_ctx* c, hipStream_t st, double dt, bool first, bool last, int b)
 {
+  if (c->small_T) return enqueue_small_step64(c, st, dt, first, last, b);
   const Step64 a = step64_args(c, dt, b);
   if (first) LJ_HIP(launch_drift64(st, a, c->cfg.canonical));
   LJ_HIP(enqueue_force64(c, st));
@@ -443,6 +470,8 @@ int lj_destroy(lj_ctx* c)
   dev_free(c->vd);
   dev_free(c->fd);
   dev_free(c->tfd);
+  dev_free(c->xs);
+  dev_free(c->xs2);
   dev_free(c->part64);
   dev_free(c->wt64);
   fl_free(c->fl);
@@ -491,7 +520,7 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
   }
   if (is_fp64(c)) c->plan64 = make_plan64(cfg->N, cfg->jslices);
   // the one-launch step unless an explicit choice of force pass asks for it
-  if (cfg->jslices == 0 && !is_fp64(c) && !force_pass_chosen()) c->small_T = small_tile(cfg->N);
+  if (cfg->jslices == 0 && !force_pass_chosen()) c->small_T = small_tile(cfg->N);
   const size_t npart = (size_t)std::max(c->plan.S, c->plan3.S) * c->plan.Npad;
   const int N = cfg->N;
   c->nblk = (N + kBlock - 1) / kBlock;
@@ -537,6 +566,10 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
     A(dev_alloc(&c->vd, N));
     A(dev_alloc(&c->fd, N));
     A(dev_alloc(&c->tfd, N));
+    if (c->small_T) {
+      A(dev_alloc(&c->xs, N));
+      A(dev_alloc(&c->xs2, N));
+    }
     A(dev_alloc(&c->part64, (size_t)c->plan64.S * c->plan64.Npad));
     A(dev_alloc(&c->wt64, force64_totals(c->plan64)));
   }

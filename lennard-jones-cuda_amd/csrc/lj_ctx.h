@@ -72,6 +72,8 @@ struct lj_ctx {
   double4* vd = nullptr;
   double4* fd = nullptr;
   double4* tfd = nullptr;
+  double4* xs = nullptr;   // one-launch steps: the force pass's coordinates,
+  double4* xs2 = nullptr;  // this step's and the next one's
   double4* part64 = nullptr;
   double* wt64 = nullptr;  // the force pass's totals of the virial
   // fluctuation counters (lj_fl_*)

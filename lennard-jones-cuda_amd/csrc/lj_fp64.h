@@ -21,6 +21,10 @@ struct Step64 {
   int nrow;
   int N, S, Npad, bc;
   double dt, L, T0, FS;
+  // one-launch steps: coordinates of this step's force pass and of the next
+  const double4* xs;
+  double4* xn;
+  double sigma;
 };
 
 // plan of the pass: pair-once (n3 != 0; items: the ng (ng + 1) / 2 group pairs
@@ -38,6 +42,14 @@ hipError_t launch_drift64(hipStream_t st, const Step64& a, int canonical);
 hipError_t launch_kick64(hipStream_t st, const Step64& a, bool drift_next, const StepArgs* fin);
 hipError_t launch_tvn64_a(hipStream_t st, const Step64& a, const StepArgs* fin);
 hipError_t launch_tvn64_b(hipStream_t st, const Step64& a, bool drift_next);
+// One-launch steps (T = small_tile(N) particles per workgroup and block row): the
+// drift that starts a run also fills a.xn; force pass from a.xs and kick
+// (drift_next: the next drift, into a.xn); force pass from a.xs and half-step
+// velocities (launch_tvn64_b follows)
+hipError_t launch_small_drift64(hipStream_t st, const Step64& a, int canonical);
+hipError_t launch_small64_evn(hipStream_t st, int T, const Step64& a, bool drift_next,
+                              const StepArgs* fin);
+hipError_t launch_small64_tvn(hipStream_t st, int T, const Step64& a, const StepArgs* fin);
 // float4 -> double4 (state upload through the FP32 arrays) and back
 hipError_t launch_widen(hipStream_t st, const float4* src, double4* dst, int N);
 hipError_t launch_narrow(hipStream_t st, const double4* src, float4* dst, int N);

@@ -10,8 +10,8 @@
 // i-tiles x j-slices, j streamed through SGPRs by uniform scalar loads); minimum
 // image dx -= L rint(dx / L) in double; self pair excluded by index
 // (MDSystem.cpp:267).  Partial entries are summed per particle in fixed order.
-#include "lj_device.h"
 #include "lj_fp64.h"
+#include "lj_small.h"
 
 namespace lj {
 
@@ -557,6 +557,183 @@ __global__ __launch_bounds__(kBlock) void k_tvn64_b(Step64 a)
   if ((threadIdx.x & 63) == 0 && row < a.nrow) a.blk[(size_t)row * kBlkFields + BLK_K2] = k2;
 }
 
+// ---- one-launch steps (lj_small.h) in double: N <= 4096 ----
+
+template <int T>
+union Small64Lds {
+  double x[3][SmallGeo<T>::CH];
+  double red[5][SmallGeo<T>::E][T];
+};
+
+// (fx, fy, fz, m, b) of particle i0 + lane % T in wave 0, as small_forces
+template <bool PERIODIC, int T>
+__device__ __forceinline__ void small_forces64(Small64Lds<T>& lds, const double4* __restrict__ xs,
+                                               int N, int i0, double L, double s2, double (&d)[5])
+{
+  using G = SmallGeo<T>;
+  const int tid = threadIdx.x, ph = tid / T, i = i0 + tid % T;
+  const double4 xi = xs[min(i, N - 1)];
+  const double invL = 1. / L;
+  Acc64 a{0., 0., 0., 0., 0.};
+  for (int c0 = 0; c0 < N; c0 += G::CH) {
+    const int n = min(G::CH, N - c0);
+    if (c0 > 0) __syncthreads();
+#pragma unroll
+    for (int t = 0; t < G::CH; t += kSmallThreads)
+      if (t + tid < n) {
+        const double4 p = xs[c0 + t + tid];
+        lds.x[0][t + tid] = p.x;
+        lds.x[1][t + tid] = p.y;
+        lds.x[2][t + tid] = p.z;
+      }
+    __syncthreads();
+    const int rows = n / G::P;
+    const int self = i0 >= c0 && i0 < c0 + G::CH ? (i0 - c0) / G::P : -1;
+    const auto one = [&](auto guard, int j, bool ok) {
+      double dx, dy, dz, sc, ir6, w;
+      terms64<PERIODIC, decltype(guard)::value>(xi.x, xi.y, xi.z, lds.x[0][j], lds.x[1][j], lds.x[2][j],
+                                                L, invL, s2, ok, dx, dy, dz, sc, ir6, w);
+      add64(a, dx, dy, dz, sc, ir6, w);
+    };
+    const auto open = [&](int k0, int k1) {
+#pragma unroll 2
+      for (int k = k0; k < k1; ++k) one(std::false_type{}, k * G::P + ph, true);
+    };
+    const auto guarded = [&](int k) {
+      const int j = k * G::P + ph;
+      one(std::true_type{}, min(j, n - 1), j < n && c0 + j != i);
+    };
+    if (self >= 0 && self < rows) {
+      open(0, self);
+      guarded(self);
+      open(self + 1, rows);
+    } else {
+      open(0, rows);
+    }
+    if (rows * G::P < n) guarded(rows);
+  }
+  d[0] = a.fx;
+  d[1] = a.fy;
+  d[2] = a.fz;
+  d[3] = a.a - a.b;
+  d[4] = a.b;
+  small_reduce<5, T>(d, lds.red);
+}
+
+template <int CANON>
+__global__ __launch_bounds__(kBlock) void k_small_drift64(Step64 a)
+{
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= a.N) return;
+  drift64<CANON>(a, i, a.x[i], a.v[i], a.f[i]);
+  a.xn[i] = a.x[i];
+}
+
+template <bool PERIODIC, int T, bool DRIFT, bool FIN>
+__global__ __launch_bounds__(kSmallThreads) void k_small64_evn(Step64 a, StepArgs fin)
+{
+#pragma clang fp contract(off)
+  __shared__ Small64Lds<T> lds;
+  if constexpr (FIN) {
+    if (blockIdx.x == 0) {
+      if (threadIdx.x < kBlock) step_observables<kWaves>(fin, fin.nrow, true, true);
+      return;
+    }
+  }
+  const int row = (int)blockIdx.x - (FIN ? 1 : 0);
+  const int i = row * T + threadIdx.x;
+  const bool lead = threadIdx.x < T && i < a.N;
+  double s[5];
+  small_forces64<PERIODIC, T>(lds, a.xs, a.N, row * T, a.L, a.sigma * a.sigma, s);
+  if (threadIdx.x >= 64) return;
+  double v3[3] = {0., 0., 0.};
+  if (lead) {
+    double4 v = a.v[i], x = a.x[i];
+    const double4 f = finish_force(a, i, Sum64{s[0], s[1], s[2], s[3]});
+    const double dt = a.dt;
+    v.x += dt * f.x / 2.;
+    v.y += dt * f.y / 2.;
+    v.z += dt * f.z / 2.;
+    bc64(x, v, a.bc, a.L);
+    v3[0] = sq3(v);
+    v3[1] = f.w;
+    v3[2] = s[4];
+    end_step64<DRIFT, LJ_EVN>(a, i, x, v, f);
+    if constexpr (DRIFT) a.xn[i] = a.x[i];
+  }
+  small_row_sum<3, T>(v3);
+  if (threadIdx.x == 0) {
+    double* r = a.blk + (size_t)row * kBlkFields;
+    r[BLK_K2] = v3[0];
+    r[BLK_E] = v3[1];
+    r[BLK_B] = v3[2];
+  }
+}
+
+template <bool PERIODIC, int T, bool FIN>
+__global__ __launch_bounds__(kSmallThreads) void k_small64_tvn(Step64 a, StepArgs fin)
+{
+#pragma clang fp contract(off)
+  __shared__ Small64Lds<T> lds;
+  if constexpr (FIN) {
+    if (blockIdx.x == 0) {
+      if (threadIdx.x < kBlock) step_observables<kWaves>(fin, fin.nrow, true, true);
+      return;
+    }
+  }
+  const int row = (int)blockIdx.x - (FIN ? 1 : 0);
+  const int i = row * T + threadIdx.x;
+  const bool lead = threadIdx.x < T && i < a.N;
+  double s[5];
+  small_forces64<PERIODIC, T>(lds, a.xs, a.N, row * T, a.L, a.sigma * a.sigma, s);
+  if (threadIdx.x >= 64) return;
+  double v3[3] = {0., 0., 0.};
+  if (lead) {
+    const double4 v = a.v[i];
+    double4 tf = a.tf[i];
+    const double4 f = finish_force(a, i, Sum64{s[0], s[1], s[2], s[3]});
+    tf.x += 0.5 * f.x;
+    tf.y += 0.5 * f.y;
+    tf.z += 0.5 * f.z;
+    a.tf[i] = tf;
+    const double dt = a.dt;
+    const double4 tv = make_double4(v.x + dt * tf.x / 2., v.y + dt * tf.y / 2., v.z + dt * tf.z / 2., 0.);
+    v3[0] = sq3(tv);
+    v3[1] = f.w;
+    v3[2] = s[4];
+  }
+  small_row_sum<3, T>(v3);
+  if (threadIdx.x == 0) {
+    double* r = a.blk + (size_t)row * kBlkFields;
+    r[BLK_K2] = 0.;  // k_tvn64_b writes the first rows' totals
+    r[BLK_TV2] = v3[0];
+    r[BLK_E] = v3[1];
+    r[BLK_B] = v3[2];
+  }
+}
+
+template <bool PERIODIC, int T>
+void small64_evn_t(hipStream_t st, const Step64& a, bool drift_next, const StepArgs* fin)
+{
+  const dim3 g(a.nrow + (fin ? 1 : 0)), b(kSmallThreads);
+  const StepArgs none{};
+  if (drift_next) {
+    if (fin) hipLaunchKernelGGL((k_small64_evn<PERIODIC, T, true, true>), g, b, 0, st, a, *fin);
+    else hipLaunchKernelGGL((k_small64_evn<PERIODIC, T, true, false>), g, b, 0, st, a, none);
+  } else {
+    if (fin) hipLaunchKernelGGL((k_small64_evn<PERIODIC, T, false, true>), g, b, 0, st, a, *fin);
+    else hipLaunchKernelGGL((k_small64_evn<PERIODIC, T, false, false>), g, b, 0, st, a, none);
+  }
+}
+
+template <bool PERIODIC, int T>
+void small64_tvn_t(hipStream_t st, const Step64& a, const StepArgs* fin)
+{
+  const dim3 g(a.nrow + (fin ? 1 : 0)), b(kSmallThreads);
+  if (fin) hipLaunchKernelGGL((k_small64_tvn<PERIODIC, T, true>), g, b, 0, st, a, *fin);
+  else hipLaunchKernelGGL((k_small64_tvn<PERIODIC, T, false>), g, b, 0, st, a, StepArgs{});
+}
+
 __global__ __launch_bounds__(kBlock) void k_widen(const float4* __restrict__ s, double4* __restrict__ d, int N)
 {
   const int i = blockIdx.x * kBlock + threadIdx.x;
@@ -729,6 +906,45 @@ hipError_t launch_tvn64_b(hipStream_t st, const Step64& a, bool drift_next)
   else hipLaunchKernelGGL(k_tvn64_b<false>, dim3(nb(a.N)), dim3(kBlock), 0, st, a);
   return hipGetLastError();
 }
+
+hipError_t launch_small_drift64(hipStream_t st, const Step64& a, int canonical)
+{
+  if (canonical == LJ_EVN)
+    hipLaunchKernelGGL(k_small_drift64<LJ_EVN>, dim3(nb(a.N)), dim3(kBlock), 0, st, a);
+  else
+    hipLaunchKernelGGL(k_small_drift64<LJ_TVN>, dim3(nb(a.N)), dim3(kBlock), 0, st, a);
+  return hipGetLastError();
+}
+
+#define LJ_SMALL_T(CALL)                  \
+  switch (T) {                            \
+    case 4: CALL(4); break;               \
+    case 8: CALL(8); break;               \
+    case 16: CALL(16); break;             \
+    default: return hipErrorInvalidValue; \
+  }
+
+hipError_t launch_small64_evn(hipStream_t st, int T, const Step64& a, bool drift_next,
+                              const StepArgs* fin)
+{
+#define LJ_CALL(K)                                                              \
+  a.bc == LJ_BC_PERIODIC ? small64_evn_t<true, K>(st, a, drift_next, fin)       \
+                         : small64_evn_t<false, K>(st, a, drift_next, fin)
+  LJ_SMALL_T(LJ_CALL)
+#undef LJ_CALL
+  return hipGetLastError();
+}
+
+hipError_t launch_small64_tvn(hipStream_t st, int T, const Step64& a, const StepArgs* fin)
+{
+#define LJ_CALL(K)                                                  \
+  a.bc == LJ_BC_PERIODIC ? small64_tvn_t<true, K>(st, a, fin)       \
+                         : small64_tvn_t<false, K>(st, a, fin)
+  LJ_SMALL_T(LJ_CALL)
+#undef LJ_CALL
+  return hipGetLastError();
+}
+#undef LJ_SMALL_T
 
 hipError_t launch_widen(hipStream_t st, const float4* src, double4* dst, int N)
 {

@@ -200,3 +200,26 @@ def test_fp64_runs_split_anywhere(N, canon, bc):
     for o in outs[1:]:
         for a, b in zip(outs[0], o):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("canon,bc", [(ljamd.EVN, ljamd.BC_WALL), (ljamd.EVN, ljamd.BC_PERIODIC),
+                                      (ljamd.TVN, ljamd.BC_PERIODIC), (ljamd.TVN, ljamd.BC_NONE)])
+@pytest.mark.parametrize("N", [2, 17, 1024, 1025, 2049, 4095, 4096])
+def test_small_step_fp64_edges(N, canon, bc):
+    """The one-launch FP64 steps at the edges of their tiles and LDS chunks,
+    with the tolerances of test_trajectory_fp64."""
+    rho, T0, dt, n = (0.05 if N < 64 else 0.5), 1.0, 0.002, 10
+    L, pos, vel = perturbed_state(N, rho, T0, seed=73)
+    print(f"\n[case] fp64 small N={N} canon={canon} bc={bc}", flush=True)
+    with ljamd.LJSystem(N, rho, T0, canonical=canon, boundary=bc, precision=ljamd.PREC_FP64) as s:
+        s.set_state(pos, vel)
+        s.CalculateForces()
+        hist = s.Integrate(dt, n)
+        x = s.get_array_f64(ljamd.ARRAY_POS).reshape(N, 4)[:, :3]
+        v = s.get_array_f64(ljamd.ARRAY_VEL).reshape(N, 4)[:, :3]
+        p32 = s.pos.reshape(N, 4)[:, :3]
+    xo, vo, _, obs = fp64_steps(xyz(pos), xyz(vel), L, bc, canon, T0, dt, n)
+    assert np.max(np.abs(x - xo)) <= 1e-9 and np.max(np.abs(v - vo)) <= 1e-8
+    assert np.max(np.abs(hist[:, 3] - obs[:, 0])) <= 1e-10 * np.max(np.abs(obs[:, 0]))
+    assert np.max(np.abs(hist[:, 2] - obs[:, 1])) <= 1e-10 * np.max(np.abs(obs[:, 1]))
+    assert np.array_equal(p32, x.astype(np.float32))
