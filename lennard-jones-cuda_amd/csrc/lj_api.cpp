@@ -1210,6 +1210,11 @@ int lj_forces_device(lj_ctx* c, const float* d_pos4, float* d_force4, double* d_
 
 namespace {
 
+struct CompatResult {
+  unsigned long long rdf[256];
+  float pressure;
+};
+
 struct CompatScratch {
   int device = -1;
   hipStream_t st = nullptr;
@@ -1223,6 +1228,7 @@ struct CompatScratch {
   float* pressure = nullptr;
   float* rdf_tab = nullptr;  // bin thresholds of the GPU rule for tab_dr2
   float tab_dr2 = 0.f, tab_last = 0.f;
+  CompatResult* host = nullptr;  // pinned: a call's results on their way out
 };
 
 std::mutex g_compat_mu;
@@ -1247,6 +1253,7 @@ void compat_release(CompatScratch& s)
   dev_free(s.rdf);
   dev_free(s.pressure);
   dev_free(s.rdf_tab);
+  if (s.host) (void)hipHostFree(s.host);
   if (s.st) (void)hipStreamDestroy(s.st);
   s = CompatScratch();
 }
@@ -1277,6 +1284,12 @@ int compat_scratch(int N, const ForcePlan& pl, CompatScratch** out)
   if (!s.rdf) LJ_TRY(dev_alloc(&s.rdf, 256));
   if (!s.rdf_tab) LJ_TRY(dev_alloc(&s.rdf_tab, 257));
   if (!s.pressure) LJ_TRY(dev_alloc(&s.pressure, 1));
+  if (!s.host) {
+    void* h = nullptr;
+    if (hipHostMalloc(&h, sizeof(CompatResult), hipHostMallocDefault) != hipSuccess)
+      return fail(LJ_ERR_ALLOC, "calculateNForces: pinned memory");
+    s.host = static_cast<CompatResult*>(h);
+  }
   *out = &s;
   return LJ_OK;
 }
@@ -1299,6 +1312,8 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
   LJ_HIP(launch_force(st, pl, ps, s->q, p, s->fpart, s->apart, false, true));
   LJ_HIP(launch_reduce_forces(st, pl, ps, s->fpart, s->apart, reinterpret_cast<float4*>(Force), s->blk));
   LJ_HIP(launch_finalize_forces(st, s->blk, (N + kBlock - 1) / kBlock, 1., nullptr, s->pressure));
+  CompatResult& r = *s->host;
+  RdfArgs a{};
   if (host_RDF) {
     LJ_HIP(launch_fill_u64(st, s->rdf, 256));
     if (s->tab_dr2 != host_dr2) {
@@ -1309,7 +1324,6 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
       s->tab_dr2 = host_dr2;
       s->tab_last = tab[255];
     }
-    RdfArgs a{};
     a.pos = p;
     a.N = N;
     a.periodic = Lperiodic != 0;
@@ -1322,15 +1336,13 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
     a.end = s->tab_last;
     a.hist = s->rdf;
     LJ_HIP(launch_rdf(st, a));
+    LJ_HIP(hipMemcpyAsync(r.rdf, s->rdf, sizeof(r.rdf), hipMemcpyDeviceToHost, st));
   }
-  float pr = 0.f;
-  unsigned long long h[256];
-  LJ_HIP(hipMemcpyAsync(&pr, s->pressure, sizeof(float), hipMemcpyDeviceToHost, st));
-  if (host_RDF) LJ_HIP(hipMemcpyAsync(h, s->rdf, sizeof(h), hipMemcpyDeviceToHost, st));
+  LJ_HIP(hipMemcpyAsync(&r.pressure, s->pressure, sizeof(float), hipMemcpyDeviceToHost, st));
   LJ_HIP(hipStreamSynchronize(st));
-  if (host_pressure) *host_pressure = pr;
+  if (host_pressure) *host_pressure = r.pressure;
   if (host_RDF)
-    for (int b = 0; b < 256; ++b) host_RDF[b] = (int)h[b];
+    for (int b = 0; b < 256; ++b) host_RDF[b] = (int)r.rdf[b];
   return LJ_OK;
 }
 

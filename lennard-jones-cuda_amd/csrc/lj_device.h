@@ -72,22 +72,71 @@ __device__ __forceinline__ float mi_fixed(unsigned qi, unsigned qj)
   return f;
 }
 
-// GUARD: 0 no exclusion, 1 self by index (i == j), 2 pairs with r2 <= thr
-template <bool PERIODIC, int GUARD, bool TIES = false>
-__device__ __forceinline__ void pair(const PosT<PERIODIC>& pi, const PosT<PERIODIC>& pj, int i,
-                                     int j, float C1, float thr, Acc& c)
+// The same rule for a lane's own particle without a compare and select per
+// axis: axis a of the lane is mirrored (s_a = -1) when qi_a < 2^31, so that the
+// separation in the lane's frame is one xor-add, (qj_a ^ m_a) + o_a, and an exact
+// half-box separation converts to -2^31 there, i.e. to -L/2 when qi > qj and to
+// +L/2 when qi < qj.  Every other separation is the exact negation of the
+// unmirrored one, so sums taken in the frame are s_a times the unmirrored sums
+// bit for bit.  (The sliced pass with ties and a check of every pair took 175 us
+// at N = 16384 with the compare and select.)
+struct MirPos {
+  unsigned mx, my, mz, ox, oy, oz;
+};
+
+__device__ __forceinline__ MirPos mirror(const PosT<true>& p)
 {
-  float dx, dy, dz;
+  MirPos r;
+  const bool fx = p.x < 0x80000000u, fy = p.y < 0x80000000u, fz = p.z < 0x80000000u;
+  r.mx = fx ? 0u : ~0u;
+  r.my = fy ? 0u : ~0u;
+  r.mz = fz ? 0u : ~0u;
+  r.ox = fx ? 0u - p.x : p.x + 1u;
+  r.oy = fy ? 0u - p.y : p.y + 1u;
+  r.oz = fz ? 0u - p.z : p.z + 1u;
+  return r;
+}
+
+__device__ __forceinline__ void unmirror(const MirPos& m, Acc& c)
+{
+  c.fx = m.mx ? c.fx : -c.fx;
+  c.fy = m.my ? c.fy : -c.fy;
+  c.fz = m.mz ? c.fz : -c.fz;
+}
+
+// separation of the lane's particle and j in the lane's frame
+template <bool PERIODIC>
+__device__ __forceinline__ void sep(const PosT<PERIODIC>& pi, const PosT<PERIODIC>& pj, float& dx,
+                                    float& dy, float& dz)
+{
   if constexpr (PERIODIC) {
-    dx = mi_fixed<TIES>(pi.x, pj.x);
-    dy = mi_fixed<TIES>(pi.y, pj.y);
-    dz = mi_fixed<TIES>(pi.z, pj.z);
+    dx = mi_fixed<false>(pi.x, pj.x);
+    dy = mi_fixed<false>(pi.y, pj.y);
+    dz = mi_fixed<false>(pi.z, pj.z);
   } else {
     dx = pi.x - pj.x;
     dy = pi.y - pj.y;
     dz = pi.z - pj.z;
   }
-  float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+}
+
+__device__ __forceinline__ void sep(const MirPos& m, const PosT<true>& pj, float& dx, float& dy,
+                                    float& dz)
+{
+  dx = (float)(int)((pj.x ^ m.mx) + m.ox);
+  dy = (float)(int)((pj.y ^ m.my) + m.oy);
+  dz = (float)(int)((pj.z ^ m.mz) + m.oz);
+}
+
+// pi: PosT (no tie rule) or MirPos.  GUARD: 0 no exclusion, 1 self by index
+// (i == j), 2 pairs with r2 <= thr (or not comparable).  Returns r2.
+template <int GUARD, class PI, class PJ>
+__device__ __forceinline__ float pair(const PI& pi, const PJ& pj, int i, int j, float C1, float thr,
+                                      Acc& c)
+{
+  float dx, dy, dz;
+  sep(pi, pj, dx, dy, dz);
+  const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
   float ir2 = __builtin_amdgcn_rcpf(r2) * C1;  // (sigma/r)^2
   if constexpr (GUARD == 1) ir2 = (i == j) ? 0.f : ir2;
   if constexpr (GUARD == 2) ir2 = (r2 > thr) ? ir2 : 0.f;
@@ -99,6 +148,62 @@ __device__ __forceinline__ void pair(const PosT<PERIODIC>& pi, const PosT<PERIOD
   c.fz = __builtin_fmaf(dz, s, c.fz);
   c.a += ir6;
   c.b += w;
+  return r2;
+}
+
+template <bool PERIODIC, bool TIES>
+struct LaneI {
+  PosT<PERIODIC> p;
+  __device__ __forceinline__ void set(const PosT<PERIODIC>& x) { p = x; }
+  __device__ __forceinline__ void common_frame(Acc&) const {}
+};
+template <>
+struct LaneI<true, true> {
+  MirPos p;
+  __device__ __forceinline__ void set(const PosT<true>& x) { p = mirror(x); }
+  __device__ __forceinline__ void common_frame(Acc& c) const { unmirror(p, c); }
+};
+
+// the sums t of one block of j, [b0, b1), at most kJB of them.  GUARD 2 looks
+// for a pair to exclude by the block's least r2 (half an instruction per pair,
+// against two for a compare and select in each) and by sums that are not
+// numbers, and only then takes the block again pair by pair: the same sums.
+template <bool PERIODIC, int GUARD, int IPL, class I>
+__device__ __forceinline__ void j_block(const uint4* __restrict__ q, const float4* __restrict__ pf,
+                                        int b0, int b1, const I (&li)[IPL], const int (&ii)[IPL],
+                                        float C1, float thr, Acc (&t)[IPL])
+{
+#pragma unroll
+  for (int k = 0; k < IPL; ++k) acc_zero(t[k]);
+  if constexpr (GUARD == 2) {
+    float least = __builtin_inff();
+#pragma unroll 8
+    for (int j = b0; j < b1; ++j) {
+      const PosT<PERIODIC> pj = load_pos<PERIODIC>(q, pf, j);
+#pragma unroll
+      for (int k = 0; k < IPL; ++k)
+        least = __builtin_fminf(least, pair<0>(li[k].p, pj, ii[k], j, C1, thr, t[k]));
+    }
+    bool bad = !(least > thr);
+#pragma unroll
+    for (int k = 0; k < IPL; ++k) bad |= t[k].a != t[k].a || t[k].b != t[k].b;
+    if (!__any(bad)) return;
+#pragma unroll
+    for (int k = 0; k < IPL; ++k) acc_zero(t[k]);
+#pragma unroll 1
+    for (int j = b0; j < b1; ++j) {
+      const PosT<PERIODIC> pj = load_pos<PERIODIC>(q, pf, j);
+#pragma unroll
+      for (int k = 0; k < IPL; ++k) pair<2>(li[k].p, pj, ii[k], j, C1, thr, t[k]);
+    }
+  } else {
+#pragma unroll 8
+    for (int j = b0; j < b1; ++j) {
+      const PosT<PERIODIC> pj = load_pos<PERIODIC>(q, pf, j);
+#pragma unroll
+      for (int k = 0; k < IPL; ++k) pair<GUARD>(li[k].p, pj, ii[k], j, C1, thr, t[k]);
+    }
+  }
 }
 
 template <bool PERIODIC, int GUARD, int IPL, bool COMP, bool TIES = false>
@@ -107,17 +212,15 @@ __device__ __forceinline__ void j_range(const uint4* __restrict__ q, const float
                                         const int (&ii)[IPL], float C1, float thr, Acc (&hi)[IPL],
                                         Acc (&lo)[IPL])
 {
+  LaneI<PERIODIC, TIES> li[IPL];
+#pragma unroll
+  for (int k = 0; k < IPL; ++k) li[k].set(pi[k]);
   for (int b0 = jb; b0 < je; b0 += kJB) {
     const int b1 = min(je, b0 + kJB);
     Acc t[IPL];
+    j_block<PERIODIC, GUARD, IPL>(q, pf, b0, b1, li, ii, C1, thr, t);
 #pragma unroll
-    for (int k = 0; k < IPL; ++k) acc_zero(t[k]);
-#pragma unroll 8
-    for (int j = b0; j < b1; ++j) {
-      const PosT<PERIODIC> pj = load_pos<PERIODIC>(q, pf, j);
-#pragma unroll
-      for (int k = 0; k < IPL; ++k) pair<PERIODIC, GUARD, TIES>(pi[k], pj, ii[k], j, C1, thr, t[k]);
-    }
+    for (int k = 0; k < IPL; ++k) li[k].common_frame(t[k]);
 #pragma unroll
     for (int k = 0; k < IPL; ++k) {
       if constexpr (COMP) {

@@ -121,11 +121,11 @@ __device__ __forceinline__ Partial small_forces(SmallLds<T>& lds, const uint4* _
     const auto open = [&](int k0, int k1) {
 #pragma unroll 4
       for (int k = k0; k < k1; ++k)
-        pair<PERIODIC, 0>(pi, small_pos<PERIODIC>(lds.j[k * G::P + ph]), 0, 0, C1, 0.f, a);
+        pair<0>(pi, small_pos<PERIODIC>(lds.j[k * G::P + ph]), 0, 0, C1, 0.f, a);
     };
     const auto guarded = [&](int k) {
       const int j = k * G::P + ph;
-      pair<PERIODIC, 1>(pi, small_pos<PERIODIC>(lds.j[min(j, n - 1)]), i, j < n ? c0 + j : i, C1,
+      pair<1>(pi, small_pos<PERIODIC>(lds.j[min(j, n - 1)]), i, j < n ? c0 + j : i, C1,
                         0.f, a);
     };
     if (self >= 0 && self < rows) {

@@ -58,3 +58,29 @@ def test_compat_errors_do_not_crash():
     # null device arrays: reported, not a crash
     ljamd.lib().calculateNForces(None, None, None, 10, 1.0, 1, None, 0.1, 256, 1)
     assert b"null" in ljamd.lib().lj_last_error()
+
+
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("N", [2, 33, 1000, 5000])
+def test_excluded_pairs(N, periodic):
+    """Pairs at r^2 <= 1e-6 are left out of the force (MDSystem.cu:37), wherever
+    in a block of 32 j they fall and whatever else the block holds: copies of
+    particles at the same place and 5e-4 away, against FP64 with the same rule."""
+    rho = 0.3 if N > 2 else 0.01
+    L, pos, _ = perturbed_state(N, rho, 1.0, seed=79)
+    p = pos.reshape(N, 4).copy()
+    for a, b, d in ((0, 1, 0.0),) if N == 2 else ((0, 1, 0.0), (2, N - 1, 0.0), (5, 32, 5e-4), (31, 6, 0.0)):
+        p[b] = p[a]
+        p[b, 0] += np.float32(d)
+    print(f"\n[case] excluded pairs N={N} periodic={periodic}", flush=True)
+    arr = ljamd.CompatArrays(N)
+    f, pr, _ = arr.calculate(p.reshape(-1), L, periodic, 0.1)
+    arr.close()
+    F64, _, E, W = forces_fp64(p.reshape(-1), float(np.float32(L)), periodic, skip_r2=1e-6)
+    assert np.all(np.isfinite(f))
+    if N == 2:  # the only pair is left out
+        assert not np.any(F64) and not np.any(f)
+    else:
+        err = force_errors(xyz(f), F64)
+        assert err["global_rel"] <= 2e-6 and err["max_rel_floor"] <= 1e-5, err
+    assert abs(pr - W / 3.0) <= 1e-5 * max(abs(W / 3.0), 1e-3)
