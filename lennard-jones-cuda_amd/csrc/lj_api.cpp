@@ -478,6 +478,7 @@ int lj_destroy(lj_ctx* c)
   dev_free(c->rdf_step);
   dev_free(c->step_tab);
   rdf_cells_free(c->rdf_cells);
+  dev_free(c->rdf_rows);
   if (c->e0) (void)hipEventDestroy(c->e0);
   if (c->e1) (void)hipEventDestroy(c->e1);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -806,7 +807,7 @@ int prepare_rdf(lj_ctx* c, int rule, int nbins, float dr2, double rmax, int accu
   std::vector<float> e(nbins + 1);
   rdf_bin_thresholds(rule, nbins, dr2, rmax, e.data());
   a.end = rule == LJ_RDF_REF_GPU ? e[nbins - 1] : e[nbins];
-  LJ_TRY(attach_rdf_cells(c, a));
+  LJ_TRY(attach_rdf_workspace(c, a));
   if (nbins + 1 > c->edges_cap) {
     LJ_HIP(hipStreamSynchronize(st));
     dev_free(c->edges2);
@@ -1213,6 +1214,7 @@ namespace {
 struct CompatResult {
   unsigned long long rdf[256];
   float pressure;
+  unsigned flagged;  // the cell-list RDF pass counted nothing
 };
 
 struct CompatScratch {
@@ -1228,6 +1230,9 @@ struct CompatScratch {
   float* pressure = nullptr;
   float* rdf_tab = nullptr;  // bin thresholds of the GPU rule for tab_dr2
   float tab_dr2 = 0.f, tab_last = 0.f;
+  RdfCellsWs cells;          // workspace of the cell-list RDF pass
+  unsigned* rows = nullptr;  // and of the all-pairs pass
+  size_t rows_cap = 0;
   CompatResult* host = nullptr;  // pinned: a call's results on their way out
 };
 
@@ -1253,6 +1258,8 @@ void compat_release(CompatScratch& s)
   dev_free(s.rdf);
   dev_free(s.pressure);
   dev_free(s.rdf_tab);
+  rdf_cells_free(s.cells);
+  dev_free(s.rows);
   if (s.host) (void)hipHostFree(s.host);
   if (s.st) (void)hipStreamDestroy(s.st);
   s = CompatScratch();
@@ -1313,6 +1320,7 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
   LJ_HIP(launch_reduce_forces(st, pl, ps, s->fpart, s->apart, reinterpret_cast<float4*>(Force), s->blk));
   LJ_HIP(launch_finalize_forces(st, s->blk, (N + kBlock - 1) / kBlock, 1., nullptr, s->pressure));
   CompatResult& r = *s->host;
+  r.flagged = 0;
   RdfArgs a{};
   if (host_RDF) {
     LJ_HIP(launch_fill_u64(st, s->rdf, 256));
@@ -1335,11 +1343,41 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
     gpu_minimage_thresholds((double)host_L, a.thr);
     a.end = s->tab_last;
     a.hist = s->rdf;
+    // the cell list where it applies (97 against 44 us at N = 16384, rho* = 0.85):
+    // the same counts
+    int reach = 1;
+    const int nc = rdf_cells_grid(a, &reach);
+    if (nc > 0) {
+      bool grown = false;
+      LJ_TRY(rdf_cells_ensure(s->cells, N, nc * nc * nc, a.nbins, st, &grown));
+      a.cells = &s->cells;
+    } else {
+      const size_t need = (size_t)rdf_workgroups(a) * a.nbins;
+      if (need > s->rows_cap) {
+        LJ_HIP(hipStreamSynchronize(st));
+        dev_free(s->rows);
+        s->rows_cap = 0;
+        LJ_TRY(dev_alloc(&s->rows, need));
+        s->rows_cap = need;
+      }
+      a.rows = s->rows;
+      a.rows_cap = s->rows_cap;
+    }
     LJ_HIP(launch_rdf(st, a));
+    if (rdf_uses_cells(a))
+      LJ_HIP(hipMemcpyAsync(&r.flagged, a.cells->result, sizeof(unsigned), hipMemcpyDeviceToHost, st));
     LJ_HIP(hipMemcpyAsync(r.rdf, s->rdf, sizeof(r.rdf), hipMemcpyDeviceToHost, st));
   }
   LJ_HIP(hipMemcpyAsync(&r.pressure, s->pressure, sizeof(float), hipMemcpyDeviceToHost, st));
   LJ_HIP(hipStreamSynchronize(st));
+  if (host_RDF && r.flagged) {
+    // a coordinate beyond [-L, 2 L): the all-pairs pass counts instead
+    LJ_HIP(hipMemsetAsync(a.cells->result, 0, sizeof(unsigned), st));
+    a.cells = nullptr;
+    LJ_HIP(launch_rdf(st, a));
+    LJ_HIP(hipMemcpyAsync(r.rdf, s->rdf, sizeof(r.rdf), hipMemcpyDeviceToHost, st));
+    LJ_HIP(hipStreamSynchronize(st));
+  }
   if (host_pressure) *host_pressure = r.pressure;
   if (host_RDF)
     for (int b = 0; b < 256; ++b) host_RDF[b] = (int)r.rdf[b];

@@ -88,6 +88,8 @@ struct lj_ctx {
   int step_tab_cap = 0;
   int64_t rdf_step_n = 0;              // steps the step histogram holds
   lj::RdfCellsWs rdf_cells;            // workspace of the cell-list RDF pass
+  unsigned* rdf_rows = nullptr;        // and of the all-pairs pass
+  size_t rdf_rows_cap = 0;
   bool sampling() const { return smp_rdf != LJ_SAMPLE_RDF_OFF || smp_fl != 0; }
 };
 
@@ -109,16 +111,35 @@ inline bool is_fp64(const lj_ctx* c) { return c->cfg.precision == LJ_PREC_FP64; 
 double4* state64(lj_ctx* c, int type);
 // plan of the force pass that fills fpart/apart
 inline const ForcePlan& fplan(const lj_ctx* c) { return c->plan3.n3 ? c->plan3 : c->plan; }
-// gives an RDF pass of the context the cell-list workspace where that pass
-// applies (at most 1024 bins; periodic boxes with 3 or more cells per axis,
-// hard-wall boxes with 6 or more), grown first
-inline int attach_rdf_cells(lj_ctx* c, RdfArgs& a)
+// gives an RDF pass of the context the workspace of the cell-list pass where
+// that pass applies, else of the all-pairs pass, grown first
+inline int attach_rdf_workspace(lj_ctx* c, RdfArgs& a)
 {
   a.cells = nullptr;
-  if (a.nbins > 1024) return LJ_OK;
+  a.rows = nullptr;
   int reach = 1;
   const int nc = rdf_cells_grid(a, &reach);
-  if (nc <= 0) return LJ_OK;
+  if (nc <= 0) {
+    const size_t need = (size_t)rdf_workgroups(a) * a.nbins;
+    if (need > c->rdf_rows_cap) {
+      LJ_HIP(hipStreamSynchronize(c->stream));
+      // the steps that sample the RDF, captured or not, hold the old rows
+      drop_graph(c);
+      const bool sampled = c->smp_args.rows != nullptr;
+      dev_free(c->rdf_rows);
+      c->rdf_rows_cap = c->smp_args.rows_cap = 0;
+      c->smp_args.rows = nullptr;  // (atomics instead, should the growth fail)
+      LJ_TRY(dev_alloc(&c->rdf_rows, need));
+      c->rdf_rows_cap = need;
+      if (sampled) {
+        c->smp_args.rows = c->rdf_rows;
+        c->smp_args.rows_cap = need;
+      }
+    }
+    a.rows = c->rdf_rows;
+    a.rows_cap = c->rdf_rows_cap;
+    return LJ_OK;
+  }
   bool grown = false;
   const int rc = rdf_cells_ensure(c->rdf_cells, a.N, nc * nc * nc, a.nbins, c->stream, &grown);
   if (rc != LJ_OK) return rc;

@@ -137,8 +137,8 @@ int lj_set_step_sampling(lj_ctx* c, const lj_step_sampling* s)
     else
       cpu_minimage_thresholds(c->L, a.thr);
     a.end = rule == LJ_RDF_REF_GPU ? e[nbins - 1] : e[nbins];
-    LJ_TRY(attach_rdf_cells(c, a));
     a.sampling = 1;
+    LJ_TRY(attach_rdf_workspace(c, a));
     a.hist = c->rdf_step;
     LJ_HIP(launch_fill_u64(st, c->rdf_step, nbins));
     LJ_HIP(hipStreamSynchronize(st));

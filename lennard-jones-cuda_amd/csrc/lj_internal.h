@@ -217,9 +217,6 @@ struct RdfCellsWs {
 };
 // cells per axis for a periodic range ending at r^2 = end, or 0 (fewer than 3)
 int rdf_cells_per_axis(double L, double end);
-// cells per axis of the periodic layout the pass takes (0: none), and its
-// reach (1 or 2)
-int rdf_cells_layout(double L, double end, int* reach);
 // LJ_OK or a status; st: the owner's stream (its work is waited for, and the
 // new arrays are cleared on it); *grown: whether the arrays were reallocated
 int rdf_cells_ensure(RdfCellsWs& w, int N, int ncell, int nbins, hipStream_t st, bool* grown);
@@ -238,9 +235,15 @@ struct RdfArgs {
   double end;        // the counted range's end, tab[nbins - 1] (REF_GPU) or tab[nbins]
   unsigned long long* hist;
   const RdfCellsWs* cells;  // may be null: no cell-list pass
+  // the all-pairs passes of at most 1024 bins: a histogram per workgroup
+  // (rdf_workgroups x nbins; null or too small: atomics on hist)
+  unsigned* rows;
+  size_t rows_cap;
   int sampling;             // the per-step sampling's pass (its own result word)
 };
 hipError_t launch_rdf(hipStream_t st, const RdfArgs& a);
+// workgroups of the all-pairs pass with at most 1024 bins (0: more bins)
+int rdf_workgroups(const RdfArgs& a);
 hipError_t launch_rdf_cells(hipStream_t st, const RdfArgs& a);
 // cells per axis (0: none) and reach of the cell-list pass for these
 // arguments, periodic or hard-wall

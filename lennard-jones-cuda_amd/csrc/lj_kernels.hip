@@ -485,17 +485,63 @@ __global__ void k_reset_averaging(lj_obs* obs)
 // differences of the two orders are exact negatives, the image shift rounds
 // half away from zero, r^2 squares them), so each unordered pair is binned
 // once and counted twice: the ordered-pair counts of the reference, exactly.
-// Work item (g, h), h >= g, over groups of kBlock particles (grid ng x ng;
-// blocks with h < g exit at once); one i per thread.  SMALL (nbins <=
-// kRdfWaveCopy): one LDS histogram per wave and group h staged in LDS; else one
-// histogram per block and the j particles read from global memory, so that
-// the LDS stays within 64 KiB at the largest nbins.  Bin divisions and the
-// image rounding are table lookups (host-bisected thresholds), with the
-// reference's float/double arithmetic reproduced.  Periodic boxes with SMALL
-// histograms take k_rdf_fx, which decides almost every pair from the
-// fixed-point image with a proven error bound and runs the reference
-// arithmetic only near bin edges; the others take k_rdf.
+// Bin divisions and the image rounding are table lookups (host-bisected
+// thresholds), with the reference's float/double arithmetic reproduced.
+//   Up to kRdfWaveCopy bins: one LDS histogram per wave, j staged in LDS, one i
+// per thread.  Group g of kBlock particles meets the j from its own first
+// particle on, in units of 32; the units of all groups in a row are cut into
+// one run per workgroup (RdfWalk), and each workgroup writes its histogram once
+// (to a row of its own where the caller has rows, k_rdf_rows adds them up; else
+// by atomics).
+// One workgroup per pair of groups left a box of N = 400 to three workgroups
+// that walked 256 j each (36 us against 10), and at N = 16384 its 2080 histograms
+// of 500 bins cost 1e6 atomics on 500 addresses.  Periodic boxes take k_rdf_fx,
+// which decides almost every pair from the fixed-point image with a proven error
+// bound and runs the reference arithmetic only near bin edges; the others
+// k_rdf_wall.
+//   More bins (k_rdf): one workgroup per pair of groups with one histogram, the
+// j particles read from global memory, so that the LDS stays within 64 KiB.
 constexpr int kRdfWaveCopy = 1024;
+constexpr int kRdfUnit = 32;
+constexpr int kGroupUnits = kBlock / kRdfUnit;
+
+// The units [u, u1) of a workgroup.  Group g has nb - kGroupUnits g units, nb =
+// ceil(N / kRdfUnit), so units before group g: first(g).
+struct RdfWalk {
+  long long u, u1;
+  int nb, g;
+  __device__ __forceinline__ long long first(int k) const
+  {
+    return (long long)k * nb - (long long)(kGroupUnits / 2) * k * (k - 1);
+  }
+  __device__ __forceinline__ RdfWalk(int N)
+  {
+    const int wg = blockIdx.x, nwg = gridDim.x;
+    nb = (N + kRdfUnit - 1) / kRdfUnit;
+    const int ng = (N + kBlock - 1) / kBlock;
+    const long long units = first(ng);
+    u = units * wg / nwg;
+    u1 = units * (wg + 1) / nwg;
+    int lo = 0, hi = ng;  // first(lo) <= u < first(hi)
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (first(mid) <= u) lo = mid;
+      else hi = mid;
+    }
+    g = lo;
+  }
+  // the next run of at most kBlock j of one group; false when done
+  __device__ __forceinline__ bool next(int N, int& j0, int& nj)
+  {
+    if (u >= u1) return false;
+    if (u == first(g + 1)) ++g;
+    j0 = g * kBlock + (int)(u - first(g)) * kRdfUnit;
+    const long long e = min(min(u1, first(g + 1)), u + kGroupUnits);
+    nj = min((int)(e - u) * kRdfUnit, N - j0);
+    u = e;
+    return true;
+  }
+};
 
 // The block's counts, one unit per unordered pair (doubled into the ordered
 // counts when flushed), in one LDS histogram per wave, h[wave][bin].  Pairs of
@@ -510,10 +556,12 @@ __device__ __forceinline__ unsigned int* rdf_hist_init(unsigned int* hs, int nbi
   return hs + (int)(threadIdx.x >> 6) * nbins;
 }
 
-// adds the block's counts (with the waves' last-bin registers) to hist
+// the block's counts (with the waves' last-bin registers): stored to its row
+// of rows, or added to hist as ordered pairs where there are no rows
 __device__ __forceinline__ void rdf_flush(const unsigned int* hs, unsigned int* hw, int ncopy,
                                           int nbins, unsigned int last,
-                                          unsigned long long* __restrict__ hist)
+                                          unsigned long long* __restrict__ hist,
+                                          unsigned int* __restrict__ rows = nullptr)
 {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) last += __shfl_xor(last, o, 64);
@@ -522,11 +570,90 @@ __device__ __forceinline__ void rdf_flush(const unsigned int* hs, unsigned int* 
   for (int b = threadIdx.x; b < nbins; b += kBlock) {
     unsigned int c = 0u;
     for (int k = 0; k < ncopy; ++k) c += hs[k * nbins + b];
-    if (c) atomicAdd(&hist[b], 2ull * c);
+    if (rows) rows[(size_t)blockIdx.x * nbins + b] = c;
+    else if (c) atomicAdd(&hist[b], 2ull * c);
   }
 }
 
-template <int RULE, bool PERIODIC, bool SMALL>
+// hist[b] += 2 sum of bin b over the nrow rows: a workgroup takes 64 bins and
+// every kRowParts-th sixteen rows
+constexpr int kRowParts = 16;
+__global__ __launch_bounds__(1024) void k_rdf_rows(const unsigned int* __restrict__ rows, int nrow,
+                                                   int nbins, unsigned long long* __restrict__ hist)
+{
+  __shared__ unsigned long long sh[16][64];
+  const int col = threadIdx.x & 63, part = threadIdx.x >> 6;
+  const int b = blockIdx.x * 64 + col;
+  unsigned long long c = 0ull;
+  if (b < nbins)
+#pragma unroll 8
+    for (int r = blockIdx.y * 16 + part; r < nrow; r += 16 * kRowParts)
+      c += rows[(size_t)r * nbins + b];
+  sh[part][col] = c;
+  __syncthreads();
+  if (part != 0 || b >= nbins) return;
+  for (int k = 1; k < 16; ++k) c += sh[k][col];
+  if (c) atomicAdd(&hist[b], 2ull * c);
+}
+
+// hard walls: the reference arithmetic of rdf_exact_bin without its early
+// returns, 8 pairs at a time (their LDS reads in flight together)
+template <int RULE>
+__global__ __launch_bounds__(kBlock) void k_rdf_wall(const float4* __restrict__ pos, int N, int nbins,
+                                                     const float* __restrict__ tab, float est_scale,
+                                                     unsigned long long* __restrict__ hist,
+                                                     unsigned int* __restrict__ rows)
+{
+  extern __shared__ float4 sh_rdf4[];
+  float4* pj_s = sh_rdf4;  // [kBlock]
+  unsigned int* hs = reinterpret_cast<unsigned int*>(sh_rdf4 + kBlock);
+  float* T = reinterpret_cast<float*>(hs + kWaves * nbins);
+  unsigned int* hw = rdf_hist_init(hs, nbins);
+  for (int b = threadIdx.x; b <= nbins; b += kBlock) T[b] = tab[b];
+  const int tid = threadIdx.x;
+  unsigned int last = 0u;
+  RdfWalk walk(N);
+  int j0, nj;
+  while (walk.next(N, j0, nj)) {
+    const int i = walk.g * kBlock + tid;
+    const float4 pi = pos[min(i, N - 1)];
+    __syncthreads();  // the previous unit is no longer read (first: nothing)
+    if (tid < nj) pj_s[tid] = pos[j0 + tid];
+    __syncthreads();
+    const float Tmax = T[nbins], Tlast = T[nbins - 1];
+    const int jlo = i < N ? i - j0 : nj;  // pairs with a later j
+    const auto run = [&](auto every) {    // every: each lane counts every j
+      constexpr bool EVERY = decltype(every)::value;
+      for (int jb = 0; jb < nj; jb += 8) {
+        constexpr int B = 8;
+        float r2[B];
+        int kk[B];
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+          r2[b] = rdf_wall_r2<RULE>(pi, pj_s[EVERY ? jb + b : min(jb + b, nj - 1)]);
+          const float e = RULE == LJ_RDF_RBINS ? __builtin_amdgcn_sqrtf(r2[b]) * est_scale
+                                               : r2[b] * est_scale;
+          kk[b] = rdf_bin(r2[b], T, nbins, (int)e);
+        }
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+          const int jj = jb + b;
+          // kept: r2 > 1e-6 (GPU rule) or below the last bin's end (the others)
+          const bool keep = RULE == LJ_RDF_REF_GPU ? r2[b] > 1e-6f : r2[b] < Tmax;
+          const bool count = (EVERY || ((jj < nj) & (jj > jlo))) & keep;
+          const bool inlast = r2[b] >= Tlast;
+          last += (count & inlast) ? 1u : 0u;
+          if (count & !inlast) atomicAdd(&hw[kk[b]], 1u);
+        }
+      }
+    };
+    if (j0 >= (walk.g + 1) * kBlock && (nj & 7) == 0) run(std::true_type{});
+    else run(std::false_type{});
+  }
+  rdf_flush(hs, hw, kWaves, nbins, last, hist, rows);
+}
+
+template <int RULE, bool PERIODIC>
 __global__ __launch_bounds__(kBlock) void k_rdf(const float4* __restrict__ pos, int N, double L,
                                                 int nbins, const float* __restrict__ tab,
                                                 float est_scale, float t0, float t1, float t2,
@@ -534,20 +661,14 @@ __global__ __launch_bounds__(kBlock) void k_rdf(const float4* __restrict__ pos, 
 {
   const int g = blockIdx.x, hgrp = blockIdx.y;
   if (hgrp < g) return;  // uniform, before any barrier
-  extern __shared__ float4 sh_rdf4[];
-  float4* pj_s = sh_rdf4;  // [kBlock] when SMALL
-  unsigned int* hs = reinterpret_cast<unsigned int*>(sh_rdf4 + (SMALL ? kBlock : 0));
-  float* T = reinterpret_cast<float*>(hs + (SMALL ? kWaves : 1) * nbins);
-  unsigned int* hw = hs;
-  if constexpr (SMALL) hw = rdf_hist_init(hs, nbins);
-  else
-    for (int b = threadIdx.x; b < nbins; b += kBlock) hs[b] = 0u;
+  extern __shared__ unsigned int sh_rdf[];
+  unsigned int* hs = sh_rdf;
+  float* T = reinterpret_cast<float*>(hs + nbins);
+  for (int b = threadIdx.x; b < nbins; b += kBlock) hs[b] = 0u;
   for (int b = threadIdx.x; b <= nbins; b += kBlock) T[b] = tab[b];
   const int j0 = hgrp * kBlock;
   const int nj = min(kBlock, N - j0);
-  if constexpr (SMALL)
-    if ((int)threadIdx.x < nj) pj_s[threadIdx.x] = pos[j0 + threadIdx.x];
-  const float4* PJ = SMALL ? pj_s : pos + j0;
+  const float4* PJ = pos + j0;
   __syncthreads();
 
   const int i = g * kBlock + threadIdx.x;
@@ -557,43 +678,15 @@ __global__ __launch_bounds__(kBlock) void k_rdf(const float4* __restrict__ pos, 
   const float thr[4] = {t0, t1, t2, t3};
   const float Tmax = T[nbins], Tlast = T[nbins - 1];
   unsigned int last = 0u;
-  if constexpr (!PERIODIC && SMALL) {
-    // hard walls: the reference arithmetic of rdf_exact_bin without its
-    // early returns, 8 pairs at a time (their LDS reads in flight together)
-    const int jlo = valid ? (diag ? (int)threadIdx.x : -1) : nj;
-    for (int j0b = 0; j0b < nj; j0b += 8) {
-      constexpr int B = 8;
-      float r2[B];
-      int kk[B];
-#pragma unroll
-      for (int b = 0; b < B; ++b) {
-        r2[b] = rdf_wall_r2<RULE>(pi, PJ[min(j0b + b, nj - 1)]);
-        const float e = RULE == LJ_RDF_RBINS ? __builtin_amdgcn_sqrtf(r2[b]) * est_scale
-                                             : r2[b] * est_scale;
-        kk[b] = rdf_bin(r2[b], T, nbins, (int)e);
-      }
-#pragma unroll
-      for (int b = 0; b < B; ++b) {
-        const int jj = j0b + b;
-        // kept: r2 > 1e-6 (GPU rule) or below the last bin's end (the others)
-        const bool keep = RULE == LJ_RDF_REF_GPU ? r2[b] > 1e-6f : r2[b] < Tmax;
-        const bool count = (jj < nj) & (jj > jlo) & keep;
-        const bool inlast = r2[b] >= Tlast;
-        last += (count & inlast) ? 1u : 0u;
-        if (count & !inlast) atomicAdd(&hw[kk[b]], 1u);
-      }
-    }
-  } else {
 #pragma unroll 4
-    for (int jj = 0; jj < nj; ++jj) {
-      if (!valid || (diag && jj <= (int)threadIdx.x)) continue;
-      const int bin = rdf_exact_bin<RULE, PERIODIC>(pi, PJ[jj], L, (float)L, thr, T, nbins, Tmax,
-                                                    Tlast, est_scale);
-      if (bin == nbins - 1) ++last;
-      else if (bin >= 0) atomicAdd(&hw[bin], 1u);
-    }
+  for (int jj = 0; jj < nj; ++jj) {
+    if (!valid || (diag && jj <= (int)threadIdx.x)) continue;
+    const int bin = rdf_exact_bin<RULE, PERIODIC>(pi, PJ[jj], L, (float)L, thr, T, nbins, Tmax, Tlast,
+                                                  est_scale);
+    if (bin == nbins - 1) ++last;
+    else if (bin >= 0) atomicAdd(&hs[bin], 1u);
   }
-  rdf_flush(hs, hw, SMALL ? kWaves : 1, nbins, last, hist);  // !SMALL: the waves share one
+  rdf_flush(hs, hs, 1, nbins, last, hist);
 }
 
 // Periodic boxes, small histograms: every pair is first classified from the
@@ -609,15 +702,15 @@ __global__ __launch_bounds__(kBlock) void k_rdf(const float4* __restrict__ pos, 
 // that may lie in the range by one comparison of r2 with RdfClass's far
 // bound; each lane then walks its marked pairs through the classification.
 template <int RULE, bool FAR>
-__global__ __launch_bounds__(kBlock) void k_rdf_fx(const float4* __restrict__ pos, int N, double L,
+__global__ __launch_bounds__(kBlock)
+    __attribute__((amdgpu_waves_per_eu(FAR || RULE == LJ_RDF_RBINS ? 8 : 4))) void k_rdf_fx(const float4* __restrict__ pos, int N, double L,
                                                    int nbins, const float* __restrict__ tab,
                                                    float est_scale, float t0, float t1, float t2,
                                                    float t3, double qscale,
-                                                   unsigned long long* __restrict__ hist)
+                                                   unsigned long long* __restrict__ hist,
+                                                   unsigned int* __restrict__ rows)
 {
   constexpr bool TAB = RULE != LJ_RDF_RBINS;  // the classification reads (T[k], T[k + 1])
-  const int g = blockIdx.x, hgrp = blockIdx.y;
-  if (hgrp < g) return;  // uniform, before any barrier
   // the j group apart from the histograms, so that the loads of a batch of j
   // may pass the atomics of the previous one
   __shared__ float4 pj_s[kBlock];
@@ -641,127 +734,168 @@ __global__ __launch_bounds__(kBlock) void k_rdf_fx(const float4* __restrict__ po
       if (b > 0) T2[b - 1].y = tq;
     }
   }
-  const int j0 = hgrp * kBlock;
-  const int nj = min(kBlock, N - j0);
-  float cmax = -3.0e38f, cmin = 3.0e38f;
-  if ((int)threadIdx.x < nj) {
-    const float4 p = pos[j0 + threadIdx.x];
-    pj_s[threadIdx.x] = p;
-    qj_s[threadIdx.x] = make_uint4(fixq(p.x, qscale), fixq(p.y, qscale), fixq(p.z, qscale), 0u);
-    cmax = fmaxf(p.x, fmaxf(p.y, p.z));
-    cmin = fminf(p.x, fminf(p.y, p.z));
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    cmax = fmaxf(cmax, __shfl_xor(cmax, o, 64));
-    cmin = fminf(cmin, __shfl_xor(cmin, o, 64));
-  }
-  if ((threadIdx.x & 63) == 0) {
-    bw[0][wv] = cmax;
-    bw[1][wv] = cmin;
-  }
-  __syncthreads();
-
-  const int i = g * kBlock + threadIdx.x;
-  const float4 pi = pos[min(i, N - 1)];
-  const uint4 qi = make_uint4(fixq(pi.x, qscale), fixq(pi.y, qscale), fixq(pi.z, qscale), 0u);
-  // this lane's pairs: j > jlo (the diagonal group counts each pair once)
-  const int jlo = i < N ? (g == hgrp ? (int)threadIdx.x : -1) : kBlock;
   const float thr[4] = {t0, t1, t2, t3};
-  const float Tmax = T[nbins], Tlast = T[nbins - 1];
-  // the bound's span A: the coordinates of this lane's particle and the j group
-  float hmax = fmaxf(pi.x, fmaxf(pi.y, pi.z)), hmin = fminf(pi.x, fminf(pi.y, pi.z));
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    hmax = fmaxf(hmax, bw[0][w]);
-    hmin = fminf(hmin, bw[1][w]);
-  }
-  RdfClass<RULE> cl;
-  cl.init((double)hmax - (double)hmin, L, qscale, est_scale, nbins, Tlast, Tmax);
   unsigned int last = 0u;
-
-  // the reference arithmetic for pair (i, jj), counted
-  auto exact = [&](int jj) {
-    const int bin = rdf_exact_bin<RULE, true>(pi, pj_s[jj], L, (float)L, thr, T, nbins, Tmax, Tlast,
-                                              est_scale);
-    if (bin == nbins - 1) ++last;
-    else if (bin >= 0) atomicAdd(&hw[bin], 1u);
-  };
-  // one pair, decided or walked to the exact path at once (the walks)
-  auto one = [&](int jj) {
-    const float r2 = rdf_r2q(qi, qj_s[jj]);
-    int k;
-    bool dec, gone;
-    if constexpr (TAB) {
-      float lo, hi;
-      cl.measure(r2, k, lo, hi);
-      cl.decide(k, lo, hi, T2[k], dec, gone);
-    } else {
-      cl.rbins(r2, k, dec, gone);
+  // the bound's span A: coordinates in [clo, chi], the box to begin with and
+  // wider from the first unit on that holds one outside
+  float clo = 0.f, chi = (float)L;
+  RdfClass<RULE> cl;
+  bool fresh = true;
+  RdfWalk walk(N);
+  int j0, nj;
+  while (walk.next(N, j0, nj)) {
+    const int i = walk.g * kBlock + threadIdx.x;
+    const float4 pi = pos[min(i, N - 1)];
+    float cmax = fmaxf(pi.x, fmaxf(pi.y, pi.z)), cmin = fminf(pi.x, fminf(pi.y, pi.z));
+    __syncthreads();  // the previous unit is no longer read (first: nothing)
+    if ((int)threadIdx.x < nj) {
+      const float4 p = pos[j0 + threadIdx.x];
+      pj_s[threadIdx.x] = p;
+      qj_s[threadIdx.x] = make_uint4(fixq(p.x, qscale), fixq(p.y, qscale), fixq(p.z, qscale), 0u);
+      cmax = fmaxf(cmax, fmaxf(p.x, fmaxf(p.y, p.z)));
+      cmin = fminf(cmin, fminf(p.x, fminf(p.y, p.z)));
     }
-    if (dec) atomicAdd(&hw[k], 1u);
-    else if (gone) {
-      if constexpr (RULE == LJ_RDF_REF_GPU) ++last;
-    } else {
-      exact(jj);
+    const bool wider = __syncthreads_or(cmax > chi || cmin < clo) != 0;
+    const float Tmax = T[nbins], Tlast = T[nbins - 1];
+    if (wider) {
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        cmax = fmaxf(cmax, __shfl_xor(cmax, o, 64));
+        cmin = fminf(cmin, __shfl_xor(cmin, o, 64));
+      }
+      if ((threadIdx.x & 63) == 0) {
+        bw[0][wv] = cmax;
+        bw[1][wv] = cmin;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        chi = fmaxf(chi, bw[0][w]);
+        clo = fminf(clo, bw[1][w]);
+      }
     }
-  };
+    if (fresh || wider) cl.init((double)chi - (double)clo, L, qscale, est_scale, nbins, Tlast, Tmax);
+    fresh = false;
+    const uint4 qi = make_uint4(fixq(pi.x, qscale), fixq(pi.y, qscale), fixq(pi.z, qscale), 0u);
+    // this lane's pairs: later j only (each pair once)
+    const int jlo = i < N ? i - j0 : kBlock;
+    // every lane counts every j of the unit
+    const bool all = j0 >= (walk.g + 1) * kBlock && (nj & 31) == 0;
 
-  for (int c0 = 0; c0 < nj; c0 += 32) {  // kBlock is a multiple of 32
-    unsigned int mask = 0u;
-    if constexpr (FAR) {
-      const float X = cl.far_bound();
-#pragma unroll 8
-      for (int b = 0; b < 32; ++b) {
-        const int jj = c0 + b;
-        const float r2 = rdf_r2q(qi, qj_s[jj]);
-        const bool ok = (jj > jlo) & (jj < nj);
-        const bool far = r2 >= X;
-        if constexpr (RULE == LJ_RDF_REF_GPU) last += (ok & far) ? 1u : 0u;
-        mask |= (ok & !far) ? (1u << b) : 0u;
+    // the reference arithmetic for pair (i, jj), counted
+    auto exact = [&](int jj) {
+      const int bin = rdf_exact_bin<RULE, true>(pi, pj_s[jj], L, (float)L, thr, T, nbins, Tmax, Tlast,
+                                                est_scale);
+      if (bin == nbins - 1) ++last;
+      else if (bin >= 0) atomicAdd(&hw[bin], 1u);
+    };
+    // one pair, decided or walked to the exact path at once (the walks)
+    auto one = [&](int jj) {
+      const float r2 = rdf_r2q(qi, qj_s[jj]);
+      int k;
+      bool dec, gone;
+      if constexpr (TAB) {
+        float lo, hi;
+        cl.measure(r2, k, lo, hi);
+        cl.decide(k, lo, hi, T2[k], dec, gone);
+      } else {
+        cl.rbins(r2, k, dec, gone);
       }
-      while (mask) {
-        const int b = __builtin_ctz(mask);
-        mask &= mask - 1u;
-        one(c0 + b);
+      if (dec) atomicAdd(&hw[k], 1u);
+      else if (gone) {
+        if constexpr (RULE == LJ_RDF_REF_GPU) ++last;
+      } else {
+        exact(jj);
       }
-    } else {
+    };
+
+    // RBINS over 32 j from c0 on, the undecided pairs left in mask.  ALL: no lane
+    // or j is left out.  A pair clear of the bin edges is counted or beyond the
+    // range; the others, in the range or not, go to the exact path.
+    auto rbins32 = [&](auto whole, int c0, unsigned int& mask) {
+      constexpr bool ALL = decltype(whole)::value;
       constexpr int B = 8;
 #pragma unroll 1
       for (int b0 = 0; b0 < 32; b0 += B) {
         int kk[B];
-        bool dec[B], gone[B];
-        if constexpr (TAB) {
-          float lo[B], hi[B];
-          float2 t[B];
+        bool clear[B];
 #pragma unroll
-          for (int b = 0; b < B; ++b) {
-            cl.measure(rdf_r2q(qi, qj_s[c0 + b0 + b]), kk[b], lo[b], hi[b]);
-            t[b] = T2[kk[b]];
-          }
-#pragma unroll
-          for (int b = 0; b < B; ++b) cl.decide(kk[b], lo[b], hi[b], t[b], dec[b], gone[b]);
-        } else {
-#pragma unroll
-          for (int b = 0; b < B; ++b) cl.rbins(rdf_r2q(qi, qj_s[c0 + b0 + b]), kk[b], dec[b], gone[b]);
-        }
+        for (int b = 0; b < B; ++b) clear[b] = cl.rbins_clear(rdf_r2q(qi, qj_s[c0 + b0 + b]), kk[b]);
 #pragma unroll
         for (int b = 0; b < B; ++b) {
           const int jj = c0 + b0 + b;
-          const bool ok = (jj > jlo) & (jj < nj);
-          if constexpr (RULE == LJ_RDF_REF_GPU) last += (ok & gone[b]) ? 1u : 0u;
-          if (ok & dec[b]) atomicAdd(&hw[kk[b]], 1u);
-          mask |= (ok & !dec[b] & !gone[b]) ? (1u << (b0 + b)) : 0u;
+          const bool ok = ALL || ((jj > jlo) & (jj < nj));
+          if (ok & clear[b] & (kk[b] < nbins)) atomicAdd(&hw[kk[b]], 1u);
+          const bool und = ok & !clear[b];
+          mask |= und ? 1u << (b0 + b) : 0u;
         }
       }
-      while (mask) {
-        const int b = __builtin_ctz(mask);
-        mask &= mask - 1u;
-        exact(c0 + b);
+    };
+
+    for (int c0 = 0; c0 < nj; c0 += 32) {  // a unit is a multiple of 32
+      unsigned int mask = 0u;
+      if constexpr (RULE == LJ_RDF_RBINS && !FAR) {
+        if (all) rbins32(std::true_type{}, c0, mask);
+        else rbins32(std::false_type{}, c0, mask);
+        while (mask) {
+          const int b = __builtin_ctz(mask);
+          mask &= mask - 1u;
+          exact(c0 + b);
+        }
+      } else if constexpr (FAR) {
+        const float X = cl.far_bound();
+#pragma unroll 8
+        for (int b = 0; b < 32; ++b) {
+          const int jj = c0 + b;
+          const float r2 = rdf_r2q(qi, qj_s[jj]);
+          const bool ok = (jj > jlo) & (jj < nj);
+          const bool far = r2 >= X;
+          if constexpr (RULE == LJ_RDF_REF_GPU) last += (ok & far) ? 1u : 0u;
+          mask |= (ok & !far) ? (1u << b) : 0u;
+        }
+        while (mask) {
+          const int b = __builtin_ctz(mask);
+          mask &= mask - 1u;
+          one(c0 + b);
+        }
+      } else {
+        constexpr int B = 8;
+#pragma unroll 1
+        for (int b0 = 0; b0 < 32; b0 += B) {
+          int kk[B];
+          bool dec[B], gone[B];
+          if constexpr (TAB) {
+            float lo[B], hi[B];
+            float2 t[B];
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+              cl.measure(rdf_r2q(qi, qj_s[c0 + b0 + b]), kk[b], lo[b], hi[b]);
+              t[b] = T2[kk[b]];
+            }
+#pragma unroll
+            for (int b = 0; b < B; ++b) cl.decide(kk[b], lo[b], hi[b], t[b], dec[b], gone[b]);
+          } else {
+#pragma unroll
+            for (int b = 0; b < B; ++b) cl.rbins(rdf_r2q(qi, qj_s[c0 + b0 + b]), kk[b], dec[b], gone[b]);
+          }
+#pragma unroll
+          for (int b = 0; b < B; ++b) {
+            const int jj = c0 + b0 + b;
+            const bool ok = (jj > jlo) & (jj < nj);
+            if constexpr (RULE == LJ_RDF_REF_GPU) last += (ok & gone[b]) ? 1u : 0u;
+            if (ok & dec[b]) atomicAdd(&hw[kk[b]], 1u);
+            mask |= (ok & !dec[b] & !gone[b]) ? (1u << (b0 + b)) : 0u;
+          }
+        }
+        while (mask) {
+          const int b = __builtin_ctz(mask);
+          mask &= mask - 1u;
+          exact(c0 + b);
+        }
       }
     }
   }
-  rdf_flush(hs, hw, kWaves, nbins, last, hist);
+  rdf_flush(hs, hw, kWaves, nbins, last, hist, rows);
 }
 
 // speed histogram of MDSystem::initvelo / updatevelo (MDSystem.cpp:651-694):
@@ -1149,49 +1283,87 @@ hipError_t launch_reset_clock(hipStream_t st, lj_obs* obs)
   return hipGetLastError();
 }
 
+namespace {
+// dynamic LDS of the passes with at most kRdfWaveCopy bins
+size_t rdf_lds(const RdfArgs& a)
+{
+  const size_t tab = sizeof(float) * (a.nbins + 1) + sizeof(unsigned) * kWaves * a.nbins;
+  if (!a.periodic) return sizeof(float4) * kBlock + tab;
+  return (a.rule != LJ_RDF_RBINS ? sizeof(float2) * a.nbins : 0) + tab;
+}
+}  // namespace
+
+// Workgroups: runs of four units or more where that leaves three workgroups per
+// CU (each sets up its tables and writes its histogram; one per unit, N = 6000, 500
+// bins: 30 against 24 us), and no more than eight times what the LDS lets 256 CUs
+// hold, six each at most, which bounds the rows.  That many because the runs differ
+// in pairs in range: one run per resident workgroup took 300 us at N = 30000, four
+// 271, eight 272; at N = 70000 1513, 1320 and 1282.
+int rdf_workgroups(const RdfArgs& a)
+{
+  if (a.nbins > kRdfWaveCopy) return 0;
+  const size_t lds = rdf_lds(a) + (a.periodic ? kBlock * 32 + 64 : 0);
+  const long fit = 256 * std::min(6L, 163840 / (long)lds);
+  const long nu = (a.N + kRdfUnit - 1) / kRdfUnit, ng = nblocks(a.N);
+  const long units = ng * nu - kGroupUnits / 2 * ng * (ng - 1);
+  const long n = std::max(std::min(units, 768L), units / 4);
+  return (int)std::max(1L, std::min(n, 8 * fit));
+}
+
 hipError_t launch_rdf(hipStream_t st, const RdfArgs& a)
 {
-  const int ng = nblocks(a.N);
-  const bool small = a.nbins <= kRdfWaveCopy;
-  const dim3 grid(ng, ng), blk(kBlock);
-  const size_t tab = sizeof(float) * (a.nbins + 1);
-  if (small && rdf_uses_cells(a)) return launch_rdf_cells(st, a);
-  if (small && a.periodic) {
-    const size_t lds = (a.rule != LJ_RDF_RBINS ? sizeof(float2) * a.nbins : 0) + tab +
-                       sizeof(unsigned) * kWaves * a.nbins;
+  const dim3 blk(kBlock);
+  if (a.nbins > kRdfWaveCopy) {
+    const int ng = nblocks(a.N);
+    const dim3 grid(ng, ng);
+    const size_t lds = sizeof(unsigned) * a.nbins + sizeof(float) * (a.nbins + 1);
+#define LJ_RDF_ARGS a.pos, a.N, a.L, a.nbins, a.tab, a.est_scale, a.thr[0], a.thr[1], a.thr[2], \
+                    a.thr[3], a.hist
+#define LJ_RDF_LAUNCH(R)                                                                         \
+  do {                                                                                           \
+    if (a.periodic) hipLaunchKernelGGL((k_rdf<R, true>), grid, blk, lds, st, LJ_RDF_ARGS);      \
+    else hipLaunchKernelGGL((k_rdf<R, false>), grid, blk, lds, st, LJ_RDF_ARGS);                \
+  } while (0)
+    if (a.rule == LJ_RDF_REF_CPU) LJ_RDF_LAUNCH(LJ_RDF_REF_CPU);
+    else if (a.rule == LJ_RDF_REF_GPU) LJ_RDF_LAUNCH(LJ_RDF_REF_GPU);
+    else LJ_RDF_LAUNCH(LJ_RDF_RBINS);
+#undef LJ_RDF_LAUNCH
+#undef LJ_RDF_ARGS
+    return hipGetLastError();
+  }
+  if (rdf_uses_cells(a)) return launch_rdf_cells(st, a);
+  const int nwg = rdf_workgroups(a);
+  unsigned* rows = a.rows && (size_t)nwg * a.nbins <= a.rows_cap ? a.rows : nullptr;
+  const size_t lds = rdf_lds(a);
+  if (a.periodic) {
     // the far-pair pass where the counted range holds under 30% of the box
     // (a sphere of radius sqrt(end) against L^3)
     const double re = std::sqrt(std::fmax(a.end, 0.));
     const bool far = re < 0.5 * a.L && 4.18879020478639098 * re * re * re < 0.3 * a.L * a.L * a.L;
 #define LJ_RDF_FX_ARGS a.pos, a.N, a.L, a.nbins, a.tab, a.est_scale, a.thr[0], a.thr[1], a.thr[2], \
-                       a.thr[3], 4294967296. / a.L, a.hist
-#define LJ_RDF_FX(R)                                                                       \
-  do {                                                                                     \
-    if (far) hipLaunchKernelGGL((k_rdf_fx<R, true>), grid, blk, lds, st, LJ_RDF_FX_ARGS); \
-    else hipLaunchKernelGGL((k_rdf_fx<R, false>), grid, blk, lds, st, LJ_RDF_FX_ARGS);    \
+                       a.thr[3], 4294967296. / a.L, a.hist, rows
+#define LJ_RDF_FX(R)                                                                            \
+  do {                                                                                          \
+    if (far) hipLaunchKernelGGL((k_rdf_fx<R, true>), dim3(nwg), blk, lds, st, LJ_RDF_FX_ARGS); \
+    else hipLaunchKernelGGL((k_rdf_fx<R, false>), dim3(nwg), blk, lds, st, LJ_RDF_FX_ARGS);    \
   } while (0)
     if (a.rule == LJ_RDF_REF_CPU) LJ_RDF_FX(LJ_RDF_REF_CPU);
     else if (a.rule == LJ_RDF_REF_GPU) LJ_RDF_FX(LJ_RDF_REF_GPU);
     else LJ_RDF_FX(LJ_RDF_RBINS);
 #undef LJ_RDF_FX
 #undef LJ_RDF_FX_ARGS
-    return hipGetLastError();
+  } else {
+#define LJ_RDF_WALL(R)                                                                            \
+  hipLaunchKernelGGL((k_rdf_wall<R>), dim3(nwg), blk, lds, st, a.pos, a.N, a.nbins, a.tab, a.est_scale, \
+                     a.hist, rows)
+    if (a.rule == LJ_RDF_REF_CPU) LJ_RDF_WALL(LJ_RDF_REF_CPU);
+    else if (a.rule == LJ_RDF_REF_GPU) LJ_RDF_WALL(LJ_RDF_REF_GPU);
+    else LJ_RDF_WALL(LJ_RDF_RBINS);
+#undef LJ_RDF_WALL
   }
-  const size_t lds =
-      (small ? sizeof(float4) * kBlock + sizeof(unsigned) * kWaves * a.nbins : sizeof(unsigned) * a.nbins) + tab;
-#define LJ_RDF_ARGS a.pos, a.N, a.L, a.nbins, a.tab, a.est_scale, a.thr[0], a.thr[1], a.thr[2], \
-                    a.thr[3], a.hist
-#define LJ_RDF_LAUNCH(R)                                                                             \
-  do {                                                                                               \
-    if (small) hipLaunchKernelGGL((k_rdf<R, false, true>), grid, blk, lds, st, LJ_RDF_ARGS);        \
-    else if (a.periodic) hipLaunchKernelGGL((k_rdf<R, true, false>), grid, blk, lds, st, LJ_RDF_ARGS); \
-    else hipLaunchKernelGGL((k_rdf<R, false, false>), grid, blk, lds, st, LJ_RDF_ARGS);             \
-  } while (0)
-  if (a.rule == LJ_RDF_REF_CPU) LJ_RDF_LAUNCH(LJ_RDF_REF_CPU);
-  else if (a.rule == LJ_RDF_REF_GPU) LJ_RDF_LAUNCH(LJ_RDF_REF_GPU);
-  else LJ_RDF_LAUNCH(LJ_RDF_RBINS);
-#undef LJ_RDF_LAUNCH
-#undef LJ_RDF_ARGS
+  if (rows)
+    hipLaunchKernelGGL(k_rdf_rows, dim3((a.nbins + 63) / 64, std::min(kRowParts, (nwg + 15) / 16)),
+                       dim3(1024), 0, st, rows, nwg, a.nbins, a.hist);
   return hipGetLastError();
 }
 

@@ -723,29 +723,46 @@ int rdf_cells_per_axis(double L, double end)
   return nc >= 3 ? nc : 0;
 }
 
+namespace {
+
+// the fewest particles for which the cell lists are taken: below, their four
+// launches cost more than the all-pairs pass (GPU rule, rho* = 0.85: N = 6000 40
+// against 28 us, N = 8000 36 against 38).  The per-step sampling takes them at any
+// N: there a coordinate beyond their span is reported instead of counted.
+constexpr int kCellsFromN = 8192;
+// the average number of particles that a cell holds at least: a workgroup per
+// cell that holds fewer finds little to do (rho* = 0.05, N = 12000: 92 us at the
+// smallest cells, 35 at 8 particles each)
+constexpr int kCellFill = 8;
+
+// LJ_RDF_CELLS: 0 no cell lists, 1 or 2 held at that reach and the smallest cells
+char cells_env()
+{
+  static const char* e = std::getenv("LJ_RDF_CELLS");
+  return e && e[0] >= '0' && e[0] <= '2' ? e[0] : 0;
+}
+
+}  // namespace
+
 // cells per axis and reach (1: side >= sqrt(X), the cell and 13 forward
 // neighbours; 2: side >= sqrt(X) / 2, the cell and 62 forward neighbours) for
 // a periodic range ending at r^2 = end, or 0 where reach 1 gives fewer than 3
 // cells per axis.  The layout with the smaller candidate volume, 27 / nc1^3
 // against 125 / nc2^3 of the box, is taken; reach 2 needs 5 or more cells per
-// axis (distinct neighbours).  LJ_RDF_CELLS=1 / 2 holds the reach at 1 / 2
-// (2 where it applies).
-int rdf_cells_layout(double L, double end, int* reach)
+// axis (distinct neighbours), `most` holds at least that.
+static int rdf_cells_layout(double L, double end, int most, int* reach)
 {
   *reach = 1;
   const int nc1 = rdf_cells_per_axis(L, end);
   if (nc1 <= 0) return 0;
   const double side = rdf_far_side(L, end);
   const int nc2 = (int)std::min((double)kRdfMaxCells, std::floor(2. * 4294967296. / side));
-  static const char* e = std::getenv("LJ_RDF_CELLS");
-  if (nc2 >= 5) {
-    const bool auto2 = 125. / ((double)nc2 * nc2 * nc2) < 27. / ((double)nc1 * nc1 * nc1);
-    if ((e && e[0] == '2') || (!(e && e[0] == '1') && auto2)) {
-      *reach = 2;
-      return nc2;
-    }
-  }
-  return nc1;
+  const char e = cells_env();
+  const bool auto2 = 125. / ((double)nc2 * nc2 * nc2) < 27. / ((double)nc1 * nc1 * nc1);
+  const bool two = nc2 >= 5 && (e == '2' || (e != '1' && auto2));
+  if (two) *reach = 2;
+  const int nc = two ? nc2 : nc1;
+  return e == '1' || e == '2' ? nc : std::min(nc, most);
 }
 
 int rdf_cells_ensure(RdfCellsWs& w, int N, int ncell, int nbins, hipStream_t st, bool* grown)
@@ -802,31 +819,35 @@ void rdf_cells_free(RdfCellsWs& w)
 }
 
 // the cell-list pass serves periodic boxes with at most 1024 bins and 3 or
-// more cells per axis, given a workspace large enough (LJ_RDF_CELLS=0 turns
-// it off)
+// more cells per axis, given a workspace large enough
 // hard walls: reach-2 cells of side at least half the counted range's end
 // (with a relative and an absolute margin over the float rounding of r^2
 // and of the cell coordinates), 6 to 64 per axis, or 0 (fewer than 6: the
 // neighbourhoods would cover most of the box)
-int rdf_wall_cells_per_axis(double L, double end)
+static int rdf_wall_cells_per_axis(double L, double end, int most)
 {
   if (!(L > 0.) || !(end > 0.) || !std::isfinite(end)) return 0;
   const double reach = std::sqrt((double)(float)end) * (1. + 1e-4) + 1e-4;
-  const int nc = (int)std::min((double)kRdfMaxCells, std::floor(2. * L / reach));
+  int nc = (int)std::min((double)kRdfMaxCells, std::floor(2. * L / reach));
+  const char e = cells_env();
+  if (e != '1' && e != '2') nc = std::min(nc, most);
   return nc >= 6 ? nc : 0;
 }
 
 int rdf_cells_grid(const RdfArgs& a, int* reach)
 {
   *reach = 2;
-  return a.periodic ? rdf_cells_layout(a.L, a.end, reach) : rdf_wall_cells_per_axis(a.L, a.end);
+  const char e = cells_env();
+  if (e == '0' || a.nbins > 1024) return 0;
+  if (!e && !a.sampling && a.N < kCellsFromN) return 0;
+  const int most = std::max(6, (int)std::floor(std::cbrt((double)a.N / kCellFill) + 1e-9));
+  return a.periodic ? rdf_cells_layout(a.L, a.end, most, reach)
+                    : rdf_wall_cells_per_axis(a.L, a.end, most);
 }
 
 bool rdf_uses_cells(const RdfArgs& a)
 {
-  static const char* e = std::getenv("LJ_RDF_CELLS");
-  if (e && e[0] == '0') return false;
-  if (!a.cells || a.nbins > 1024) return false;
+  if (!a.cells) return false;
   int reach = 1;
   const int nc = rdf_cells_grid(a, &reach);
   return nc > 0 && a.cells->flag && a.N <= a.cells->cap_n && nc * nc * nc <= a.cells->cap_cells &&

@@ -151,7 +151,7 @@ __device__ __forceinline__ int rdf_exact_bin(const float4& pi, const float4& pj,
 // r2 + delta < T[k + 1] from one read of T2[k] = (T[k], T[k + 1]) S^2.
 template <int RULE>
 struct RdfClass {
-  float Kr, K2, K0, M0, M1, es, kmax, fnb, Tend, Tlow;
+  float Kr, K2, K0, M0, M1, H0, es, kmax, fnb, Tend, Tlow;
   int nbins;
   double Krd, K2d, K0d, Tend_d;
 
@@ -172,6 +172,7 @@ struct RdfClass {
     es = (float)esd;
     M0 = (float)(1.01 * (esd * Krd + esd * esd * K0d));
     M1 = (float)(1.01 * (K2d + 6. * u));
+    H0 = 0.5f - (M0 + 0x1p-22f);
     kmax = (float)(nb - 1);
     fnb = (float)nb;
     // the upper end of the counted range: dropped (REF_CPU, RBINS) or the
@@ -186,6 +187,17 @@ struct RdfClass {
   {
     const double dl2 = Krd * __builtin_sqrt(2. * Tend_d) + K2d * 2. * Tend_d + K0d;
     return (float)((Tend_d + 2. * dl2) * (1. + 0x1p-20));
+  }
+  // RBINS, from r2 alone, for the passes over all pairs: true when r2 lies
+  // clear of the bin edges, k then being its bin (nbins or more: beyond the
+  // range).  The condition of rbins in one comparison: |frac(x) - 1/2| <= 1/2 - m,
+  // with 2^-22 off for the roundings of its two sides, and x < 1 moved onto the
+  // edge at 1.
+  __device__ __forceinline__ bool rbins_clear(float r2, int& k) const
+  {
+    const float x = __builtin_fmaxf(__builtin_amdgcn_sqrtf(r2) * es, 1.f);
+    k = (int)x;
+    return __builtin_fabsf(__builtin_amdgcn_fractf(x) - 0.5f) <= __builtin_fmaf(-M1, x, H0);
   }
   // RBINS, from r2 alone: k (the bin if decided), dec (decided and counted in
   // bin k), gone (decided: beyond the range)

@@ -333,3 +333,53 @@ def test_step_rdf_after_lj_rdf_grows_the_cell_workspace():
     assert runs[0][1] == runs[1][1] == 10
     assert np.array_equal(runs[0][0], runs[1][0])
     assert np.array_equal(runs[0][2], runs[1][2])
+
+
+@pytest.mark.parametrize("rule", [RDF_REF_CPU, RDF_REF_GPU, RDF_RBINS])
+@pytest.mark.parametrize("bc", [ljamd.BC_PERIODIC, ljamd.BC_WALL])
+@pytest.mark.parametrize("N,nbins", [(31, 1), (32, 256), (33, 1024), (255, 64), (256, 1025), (257, 256),
+                                     (289, 1024), (513, 1), (8191, 256), (8192, 1024)])
+def test_rdf_unit_edges(N, nbins, bc, rule):
+    """Around the units of 32 and the groups of 256 particles of the all-pairs
+    pass, at the fewest and the most bins of it, and around N = 8192, from which
+    on lj_rdf takes the cell lists; a few periodic coordinates lie boxes away, so
+    that some units widen the classification's span.  Counts are whole numbers:
+    equal."""
+    rho = 0.3
+    L, pos, _ = perturbed_state(N, rho, 1.0, seed=N)
+    p = pos.reshape(-1, 4).copy()
+    if bc == ljamd.BC_PERIODIC:
+        p[N // 2, 0] += np.float32(L)
+        p[N - 1, 1] -= np.float32(2.0 * L)
+        p[N // 3, 2] += np.float32(4.0 * L)
+    pos = p.reshape(-1)
+    dr2 = ORC.orc_rdf_dr2(N)
+    with ljamd.LJSystem(N, rho, 1.0, boundary=bc) as s:
+        s.set_state(pos)
+        got = s.rdf(RULES[rule], nbins, dr2=dr2, rmax=L / 2)
+    exp = rdf(pos, L, bc == ljamd.BC_PERIODIC, rule, nbins, dr2=dr2, rmax=L / 2)
+    assert np.array_equal(got.astype(np.int64), exp), np.nonzero(got.astype(np.int64) - exp)
+
+
+def test_step_rdf_after_lj_rdf_grows_the_rows():
+    """The same for the all-pairs pass's histogram per workgroup: a call with
+    more bins replaces the rows the sampled steps, captured or launched one by
+    one, write."""
+    N, rho, T0 = 1500, 0.85, 1.0
+    L, pos, vel = perturbed_state(N, rho, T0, seed=14)
+    runs = []
+    for grow in (False, True):
+        with ljamd.LJSystem(N, rho, T0, canonical=ljamd.TVN) as s:
+            s.set_state(pos, vel)
+            s.CalculateForces()
+            s.set_step_sampling(rdf=ljamd.SAMPLE_RDF_SUM, rdf_rule=ljamd.RDF_RBINS, rdf_nbins=100,
+                                rdf_rmax=L / 2)
+            s.Integrate(0.005, 13)
+            if grow:
+                assert s.rdf(ljamd.RDF_RBINS, 1024, rmax=L / 2).sum() > 0
+            s.Integrate(0.005, 13)
+            counts, n = s.step_rdf_counts()
+            runs.append((counts.astype(np.int64), n, s.pos.copy()))
+    assert runs[0][1] == runs[1][1] == 26
+    assert np.array_equal(runs[0][0], runs[1][0])
+    assert np.array_equal(runs[0][2], runs[1][2])
