@@ -274,7 +274,7 @@ int enqueue_step_part(lj_ctx* c, hipStream_t st, double dt, bool first, bool las
   // the drift kernel already wrote the fixed-point copy for periodic boxes
   double* ew = const_cast<double*>(a.ew);
   const ForcePlan& p3 = c->plan3;
-  if (c->emulate_shards > 1 && p3.n3 == 2 && p3.split == 1 && !p3.comp) {
+  if (c->emulate_shards > 1 && p3.n3 == 2 && !p3.comp) {
     // each item writes its own partial entries and totals: the G launches
     // leave the buffers of the single launch
     const int M = p3.nitems_step, G = std::min(c->emulate_shards, M);
@@ -972,7 +972,7 @@ int lj_time_force_items_share(lj_ctx* c, int shard, int nshards, int reps, doubl
   LJ_TRY(ctx_setdev(c));
   const ForcePlan& pl = c->plan3;
   if (reps <= 0 || !us) return fail(LJ_ERR_ARG, "lj_time_force_items_share: bad arguments");
-  if (pl.n3 != 2 || pl.split != 1 || pl.comp)
+  if (pl.n3 != 2 || pl.comp)
     return fail(LJ_ERR_STATE, "lj_time_force_items_share: needs the FP32 pair-once step pass "
                               "with paired diagonal items");
   const int M = pl.nitems_step;

@@ -23,10 +23,10 @@
 //     are idle.  The time step's variant (W = 2) instead takes the diagonal
 //     items two to a workgroup with every pair once (n3_diag_pair), so that
 //     every workgroup carries the same work.
-//   * Split items (groups of 256, sizes whose items fill few of the resident
-//     workgroups, n3_split): two workgroups per item, each taking one of the
-//     two 64-particle j sub-tiles of every wave, with their own slots (S = 2
-//     groups); the diagonal items stay single.
+//   * Small items (groups of 128, W = 1; sizes whose items of 256 fill few of the
+//     resident workgroups, n3_small_groups): the four waves of a workgroup
+//     share one tile pair, each taking one 64-particle j sub-tile and half of its
+//     64 steps, so the same pairs run on four times the waves.
 // Output slots.  Particle p of group a receives exactly one entry per group s:
 // s > a from the i side of item (a, s), s < a from the j side of item (s, a),
 // s == a from the diagonal item.  The partial buffers are therefore the
@@ -102,61 +102,102 @@ __device__ __forceinline__ float rot1(float v)
   return __int_as_float(__builtin_amdgcn_ds_bpermute(((lane + 1) & 63) << 2, __float_as_int(v)));
 }
 
+// STEPS steps from t0 on of one j sub-tile P (64 particles, doubled): i sums in
+// a1/a2, the j sums in j[] travelling with their j particle
+template <bool PERIODIC, bool TIES, bool PARTIAL, bool ENERGY, int STEPS>
+__device__ __forceinline__ void pair_steps(const uint4* P, int t0, int lane,
+                                           const PosT<PERIODIC>& pi1, const PosT<PERIODIC>& pi2,
+                                           bool v1, bool v2, float C1, Acc& a1, Acc& a2,
+                                           float (&j)[4])
+{
+  float jx = 0.f, jy = 0.f, jz = 0.f, jm = 0.f;
+#pragma unroll 8
+  for (int t = 0; t < STEPS; ++t) {
+    const uint4 pj = P[lane + t0 + t];
+    bool ok1 = true, ok2 = true;
+    if constexpr (PARTIAL) {
+      const bool jv = pj.w != 0u;
+      ok1 = v1 && jv;
+      ok2 = v2 && jv;
+    }
+    float dx1, dy1, dz1, s1, e1, w1, dx2, dy2, dz2, s2, e2, w2;
+    terms<PERIODIC, TIES, PARTIAL>(pi1, pj, C1, ok1, dx1, dy1, dz1, s1, e1, w1);
+    terms<PERIODIC, TIES, PARTIAL>(pi2, pj, C1, ok2, dx2, dy2, dz2, s2, e2, w2);
+    a1.fx = __builtin_fmaf(dx1, s1, a1.fx);
+    a1.fy = __builtin_fmaf(dy1, s1, a1.fy);
+    a1.fz = __builtin_fmaf(dz1, s1, a1.fz);
+    a1.a += e1;
+    a1.b += w1;
+    a2.fx = __builtin_fmaf(dx2, s2, a2.fx);
+    a2.fy = __builtin_fmaf(dy2, s2, a2.fy);
+    a2.fz = __builtin_fmaf(dz2, s2, a2.fz);
+    a2.a += e2;
+    a2.b += w2;
+    jx = __builtin_fmaf(-dx2, s2, __builtin_fmaf(-dx1, s1, jx));
+    jy = __builtin_fmaf(-dy2, s2, __builtin_fmaf(-dy1, s1, jy));
+    jz = __builtin_fmaf(-dz2, s2, __builtin_fmaf(-dz1, s1, jz));
+    jx = rot1(jx);
+    jy = rot1(jy);
+    jz = rot1(jz);
+    if constexpr (ENERGY) {
+      jm += (e1 - w1) + (e2 - w2);
+      jm = rot1(jm);
+    }
+  }
+  j[0] = jx;
+  j[1] = jy;
+  j[2] = jz;
+  j[3] = jm;
+}
+
 // one tile pair evaluated once: i sums in a1/a2; j sums in registers that
 // travel with their j particle (lane l holds the sums of j slot (l + t) mod 64
 // at step t and passes them to lane l - 1 afterwards), so after 64 steps lane l
 // holds those of slot l.  J receives (-fx, -fy, -fz, sum (s/r)^6 - w) per
 // sub-tile.
-// nsub: sub-tiles holding a valid j (1 when the second one is past N); st0:
-// the first sub-tile taken (1 for the second half of a split item)
+// nsub: sub-tiles holding a valid j (1 when the second one is past N)
 template <bool PERIODIC, bool TIES, bool PARTIAL, bool ENERGY>
 __device__ __forceinline__ void pair_tile(const uint4* P0, int lane, const PosT<PERIODIC>& pi1,
                                           const PosT<PERIODIC>& pi2, bool v1, bool v2, float C1,
-                                          int nsub, Acc& a1, Acc& a2, float (&J)[2][4], int st0 = 0)
+                                          int nsub, Acc& a1, Acc& a2, float (&J)[2][4])
 {
 #pragma unroll
   for (int st = 0; st < 2; ++st) {
     if (st >= nsub) break;  // wave-uniform
-    if (st < st0) continue;
-    const uint4* P = P0 + st * 128;
-    float jx = 0.f, jy = 0.f, jz = 0.f, jm = 0.f;
+    pair_steps<PERIODIC, TIES, PARTIAL, ENERGY, 64>(P0 + st * 128, 0, lane, pi1, pi2, v1, v2, C1, a1,
+                                                    a2, J[st]);
+  }
+}
+
+// STEPS steps from t0 on of the lane's i particles against one j sub-tile P (j
+// numbers from jbase on), i sums only, self pair excluded
+template <bool PERIODIC, bool TIES, int STEPS>
+__device__ __forceinline__ void self_steps(const uint4* P, int t0, int lane, int i1, int i2,
+                                           int jbase, const PosT<PERIODIC>& pi1,
+                                           const PosT<PERIODIC>& pi2, bool v1, bool v2, float C1,
+                                           Acc& a1, Acc& a2)
+{
 #pragma unroll 8
-    for (int t = 0; t < 64; ++t) {
-      const uint4 pj = P[lane + t];
-      bool ok1 = true, ok2 = true;
-      if constexpr (PARTIAL) {
-        const bool jv = pj.w != 0u;
-        ok1 = v1 && jv;
-        ok2 = v2 && jv;
-      }
-      float dx1, dy1, dz1, s1, e1, w1, dx2, dy2, dz2, s2, e2, w2;
-      terms<PERIODIC, TIES, PARTIAL>(pi1, pj, C1, ok1, dx1, dy1, dz1, s1, e1, w1);
-      terms<PERIODIC, TIES, PARTIAL>(pi2, pj, C1, ok2, dx2, dy2, dz2, s2, e2, w2);
-      a1.fx = __builtin_fmaf(dx1, s1, a1.fx);
-      a1.fy = __builtin_fmaf(dy1, s1, a1.fy);
-      a1.fz = __builtin_fmaf(dz1, s1, a1.fz);
-      a1.a += e1;
-      a1.b += w1;
-      a2.fx = __builtin_fmaf(dx2, s2, a2.fx);
-      a2.fy = __builtin_fmaf(dy2, s2, a2.fy);
-      a2.fz = __builtin_fmaf(dz2, s2, a2.fz);
-      a2.a += e2;
-      a2.b += w2;
-      jx = __builtin_fmaf(-dx2, s2, __builtin_fmaf(-dx1, s1, jx));
-      jy = __builtin_fmaf(-dy2, s2, __builtin_fmaf(-dy1, s1, jy));
-      jz = __builtin_fmaf(-dz2, s2, __builtin_fmaf(-dz1, s1, jz));
-      jx = rot1(jx);
-      jy = rot1(jy);
-      jz = rot1(jz);
-      if constexpr (ENERGY) {
-        jm += (e1 - w1) + (e2 - w2);
-        jm = rot1(jm);
-      }
-    }
-    J[st][0] = jx;
-    J[st][1] = jy;
-    J[st][2] = jz;
-    J[st][3] = jm;
+  for (int t = 0; t < STEPS; ++t) {
+    const int jx = lane + t0 + t;
+    const uint4 pj = P[jx];
+    const int j = jbase + (jx & 63);
+    const bool jv = pj.w != 0u;
+    const bool ok1 = v1 && jv && j != i1;
+    const bool ok2 = v2 && jv && j != i2;
+    float dx, dy, dz, s, e, w;
+    terms<PERIODIC, TIES, true>(pi1, pj, C1, ok1, dx, dy, dz, s, e, w);
+    a1.fx = __builtin_fmaf(dx, s, a1.fx);
+    a1.fy = __builtin_fmaf(dy, s, a1.fy);
+    a1.fz = __builtin_fmaf(dz, s, a1.fz);
+    a1.a += e;
+    a1.b += w;
+    terms<PERIODIC, TIES, true>(pi2, pj, C1, ok2, dx, dy, dz, s, e, w);
+    a2.fx = __builtin_fmaf(dx, s, a2.fx);
+    a2.fy = __builtin_fmaf(dy, s, a2.fy);
+    a2.fz = __builtin_fmaf(dz, s, a2.fz);
+    a2.a += e;
+    a2.b += w;
   }
 }
 
@@ -164,36 +205,13 @@ __device__ __forceinline__ void pair_tile(const uint4* P0, int lane, const PosT<
 template <bool PERIODIC, bool TIES>
 __device__ __forceinline__ void self_tile(const uint4* P0, int lane, int i1, int i2, int jbase,
                                           const PosT<PERIODIC>& pi1, const PosT<PERIODIC>& pi2,
-                                          bool v1, bool v2, float C1, int nsub, Acc& a1, Acc& a2,
-                                          int st0 = 0)
+                                          bool v1, bool v2, float C1, int nsub, Acc& a1, Acc& a2)
 {
 #pragma unroll
   for (int st = 0; st < 2; ++st) {
     if (st >= nsub) break;  // wave-uniform
-    if (st < st0) continue;
-    const uint4* P = P0 + st * 128;
-#pragma unroll 8
-    for (int t = 0; t < 64; ++t) {
-      const int jx = lane + t;
-      const uint4 pj = P[jx];
-      const int j = jbase + st * 64 + (jx & 63);
-      const bool jv = pj.w != 0u;
-      const bool ok1 = v1 && jv && j != i1;
-      const bool ok2 = v2 && jv && j != i2;
-      float dx, dy, dz, s, e, w;
-      terms<PERIODIC, TIES, true>(pi1, pj, C1, ok1, dx, dy, dz, s, e, w);
-      a1.fx = __builtin_fmaf(dx, s, a1.fx);
-      a1.fy = __builtin_fmaf(dy, s, a1.fy);
-      a1.fz = __builtin_fmaf(dz, s, a1.fz);
-      a1.a += e;
-      a1.b += w;
-      terms<PERIODIC, TIES, true>(pi2, pj, C1, ok2, dx, dy, dz, s, e, w);
-      a2.fx = __builtin_fmaf(dx, s, a2.fx);
-      a2.fy = __builtin_fmaf(dy, s, a2.fy);
-      a2.fz = __builtin_fmaf(dz, s, a2.fz);
-      a2.a += e;
-      a2.b += w;
-    }
+    self_steps<PERIODIC, TIES, 64>(P0 + st * 128, 0, lane, i1, i2, jbase + st * 64, pi1, pi2, v1, v2,
+                                   C1, a1, a2);
   }
 }
 
@@ -594,20 +612,13 @@ __device__ __forceinline__ void n3_diag_pair(N3Lds<2>& lds, const uint4* __restr
 // terms.  The j side then carries three sums instead of four.
 // One group pair (g, h) of one box: q/pf/fpart/apart point at the box's
 // arrays, ew (ENERGY = false) at the workgroup's two totals.
-// SPLIT: the item is run by two workgroups, half = 0 / 1 taking the first /
-// second 64-particle sub-tile of every wave's 128 j (half the pairs each), so
-// that sizes whose items leave most SIMDs one to three waves run twice the
-// waves.  Each half writes its own slots, 2 h + half for the i side
-// and 2 g + half for the j side (zeros for the j it did not meet): every
-// particle still receives exactly one entry per slot, S = 2 groups.
-// COMP: the compensated mode's sums (pair_tile_c, self_tile_c; W = 2, no
-// split items).
-template <bool PERIODIC, bool TIES, int W, bool ENERGY, bool SPLIT = false, bool COMP = false>
+// COMP: the compensated mode's sums (pair_tile_c, self_tile_c; W = 2).
+template <bool PERIODIC, bool TIES, int W, bool ENERGY, bool COMP = false>
 __device__ __forceinline__ void n3_item(N3Lds<W>& lds, const uint4* __restrict__ q,
                                         const float4* __restrict__ pf,
                                         float4* __restrict__ fpart, float* __restrict__ apart,
                                         double* __restrict__ ew, int N, int Npad, float C1, int g,
-                                        int h, int half = 0)
+                                        int h)
 {
   constexpr int kG = kTile * W;
   uint4* const s_pos = lds.pos;
@@ -640,8 +651,7 @@ __device__ __forceinline__ void n3_item(N3Lds<W>& lds, const uint4* __restrict__
   // second sub-tile past N is skipped: wave-uniform tests
   const int jt0 = kG * h + kTile * wj, it0 = kG * g + kTile * wi;
   const bool live = jt0 < N && it0 < N;
-  const int nsub = SPLIT ? min(jt0 + 64 < N ? 2 : 1, half + 1) : (jt0 + 64 < N ? 2 : 1);
-  const int st0 = SPLIT ? half : 0;
+  const int nsub = jt0 + 64 < N ? 2 : 1;
   // pair tile / self tile / idle
   const int cls = !live ? 0 : (diag ? (wi < wj ? 1 : (wi == wj ? 2 : 0)) : 1);
   const int i1 = kG * g + kTile * wi + lane, i2 = i1 + 64;
@@ -654,7 +664,7 @@ __device__ __forceinline__ void n3_item(N3Lds<W>& lds, const uint4* __restrict__
   const uint4* P0 = s_pos + wj * 256;
   float J[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
   if constexpr (COMP) {
-    static_assert(W == 2 && !SPLIT, "compensated items: groups of 256, not split");
+    static_assert(W == 2, "compensated items: groups of 256");
     Acc l1, l2;
     acc_zero(l1);
     acc_zero(l2);
@@ -673,13 +683,12 @@ __device__ __forceinline__ void n3_item(N3Lds<W>& lds, const uint4* __restrict__
     a2.fx += l2.fx, a2.fy += l2.fy, a2.fz += l2.fz, a2.a += l2.a, a2.b += l2.b;
   } else if (cls == 1) {
     if (partial)
-      pair_tile<PERIODIC, TIES, true, ENERGY>(P0, lane, pi1, pi2, v1, v2, C1, nsub, a1, a2, J, st0);
+      pair_tile<PERIODIC, TIES, true, ENERGY>(P0, lane, pi1, pi2, v1, v2, C1, nsub, a1, a2, J);
     else
-      pair_tile<PERIODIC, TIES, false, ENERGY>(P0, lane, pi1, pi2, v1, v2, C1, SPLIT ? nsub : 2, a1,
-                                               a2, J, st0);
+      pair_tile<PERIODIC, TIES, false, ENERGY>(P0, lane, pi1, pi2, v1, v2, C1, 2, a1, a2, J);
   } else if (cls == 2) {
     self_tile<PERIODIC, TIES>(P0, lane, i1, i2, kG * h + kTile * wj, pi1, pi2, v1, v2, C1, nsub, a1,
-                              a2, st0);
+                              a2);
   }
   {
     float* A = s_acc + wave * kAccPerWave;
@@ -760,7 +769,7 @@ __device__ __forceinline__ void n3_item(N3Lds<W>& lds, const uint4* __restrict__
       v[4] += jf[3];
     }
     const int i = kG * g + T;
-    const size_t si = SPLIT ? 2 * h + half : h, sj = SPLIT ? 2 * g + half : g;
+    const size_t si = h, sj = g;
     if (i < N) {
       if constexpr (ENERGY) {
         store_part(fpart + si * Npad + i, v[0], v[1], v[2], v[3]);
@@ -783,28 +792,151 @@ __device__ __forceinline__ void n3_item(N3Lds<W>& lds, const uint4* __restrict__
   }
 }
 
-// SPLIT: two workgroups per item (blockIdx.x = 2 item + half), no paired
-// diagonal items; the (E, W) totals of the step variant per workgroup
-template <bool PERIODIC, bool TIES, int W, bool ENERGY, bool SPLIT>
+template <bool PERIODIC, bool TIES, int W, bool ENERGY>
 __global__ __launch_bounds__(64 * W * W) __attribute__((amdgpu_waves_per_eu(8))) void k_force_n3(
     const uint4* __restrict__ q, const float4* __restrict__ pf, const int2* __restrict__ items,
     float4* __restrict__ fpart, float* __restrict__ apart, double* __restrict__ ew, int N, int Npad,
     float C1)
 {
-  static_assert(!SPLIT || W == 2, "split items: groups of 256");
   __shared__ N3Lds<W> lds;
-  const int wg = blockIdx.x;
-  const int k = SPLIT ? wg >> 1 : wg;  // item
+  const int k = blockIdx.x;  // item
   const int2 it = items[k];
-  if constexpr (!ENERGY && W == 2 && !SPLIT) {
+  if constexpr (!ENERGY && W == 2) {
     if (it.y < 0) {  // diagonal pair (it.x, -2 - it.y), the second one absent when -1
       n3_diag_pair<PERIODIC>(lds, q, pf, fpart, ew + 2 * (size_t)k, N, Npad, C1, it.x, -2 - it.y);
       return;
     }
   }
-  n3_item<PERIODIC, TIES, W, ENERGY, SPLIT>(lds, q, pf, fpart, apart,
-                                            ENERGY ? nullptr : ew + 2 * (size_t)wg, N, Npad, C1,
-                                            it.x, it.y, SPLIT ? wg & 1 : 0);
+  n3_item<PERIODIC, TIES, W, ENERGY>(lds, q, pf, fpart, apart, ENERGY ? nullptr : ew + 2 * (size_t)k,
+                                     N, Npad, C1, it.x, it.y);
+}
+
+// Small items: a pair of groups of 128 per workgroup of four waves; wave w takes
+// j sub-tile w / 2 and its steps 32 (w & 1) + [0, 32) for the 128 i (two per
+// lane).  Entries, slots and totals as n3_item's; the last group may lie past N
+// (the group count is even): its items write zeros.
+// Why: a box of N = 5003 has 210 items of 256, 420 workgroups when halved by j
+// sub-tile, one or two waves on a SIMD, which then waits for its own latency
+// (13.6 us against 7.6 us of issue).  As 820 small items the waves are half as
+// long and three or four share a SIMD; the partial slots are those of the
+// halved items.
+template <bool PERIODIC, bool TIES, bool ENERGY>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_force_n3s(
+    const uint4* __restrict__ q, const float4* __restrict__ pf, const int2* __restrict__ items,
+    float4* __restrict__ fpart, float* __restrict__ apart, double* __restrict__ ew, int N, int Npad,
+    float C1)
+{
+  constexpr int NI = ENERGY ? 5 : 3, NJ = ENERGY ? 4 : 3;
+  __shared__ uint4 s_pos[2 * 128];       // [sub-tile][doubled 64]
+  __shared__ float s_j[4][NJ][64];       // j sums [wave][component][slot]
+  __shared__ float s_i[4][NI][kTile];    // i sums [wave][component][i]
+  __shared__ double s_ew[4][2];
+  const int2 it = items[blockIdx.x];
+  const int g = it.x, h = it.y;
+  const int T = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(T >> 6);
+  const int lane = T & 63;
+  const bool diag = g == h;
+  const int i1 = kTile * g + lane, i2 = i1 + 64;
+  const bool v1 = i1 < N, v2 = i2 < N;
+  const PosT<PERIODIC> pi1 = load_pos<PERIODIC>(q, pf, v1 ? i1 : N - 1);
+  const PosT<PERIODIC> pi2 = load_pos<PERIODIC>(q, pf, v2 ? i2 : N - 1);
+  if (T < kTile) {
+    const int j = kTile * h + T;
+    const int jl = j < N ? j : 0;
+    uint4 p;
+    if constexpr (PERIODIC) {
+      p = q[jl];
+    } else {
+      const float4 f = pf[jl];
+      p = make_uint4(__float_as_uint(f.x), __float_as_uint(f.y), __float_as_uint(f.z), 0u);
+    }
+    p.w = j < N ? 1u : 0u;
+    uint4* d = s_pos + (T >> 6) * 128;
+    d[T & 63] = p;
+    d[(T & 63) + 64] = p;
+  }
+  __syncthreads();
+
+  const int st = wave >> 1, t0 = 32 * (wave & 1);
+  const int jb = kTile * h + 64 * st;  // the wave's j sub-tile
+  const bool live = jb < N;            // wave-uniform
+  const int cls = !live ? 0 : (diag ? 2 : 1);
+  Acc a1, a2;
+  acc_zero(a1);
+  acc_zero(a2);
+  float J[4] = {0.f, 0.f, 0.f, 0.f};
+  if (cls == 1) {  // g < h: every i is valid
+    if (jb + 64 > N)
+      pair_steps<PERIODIC, TIES, true, ENERGY, 32>(s_pos + st * 128, t0, lane, pi1, pi2, v1, v2, C1,
+                                                   a1, a2, J);
+    else
+      pair_steps<PERIODIC, TIES, false, ENERGY, 32>(s_pos + st * 128, t0, lane, pi1, pi2, v1, v2, C1,
+                                                    a1, a2, J);
+  } else if (cls == 2) {
+    self_steps<PERIODIC, TIES, 32>(s_pos + st * 128, t0, lane, i1, i2, jb, pi1, pi2, v1, v2, C1, a1,
+                                   a2);
+  }
+  // after the steps lane l holds the sums of j slot (l + t0 + 32) mod 64
+#pragma unroll
+  for (int c = 0; c < NJ; ++c) s_j[wave][c][(lane + t0 + 32) & 63] = J[c];
+  {
+    float e1[5], e2[5];
+    encode(a1, cls, e1);
+    encode(a2, cls, e2);
+#pragma unroll
+    for (int c = 0; c < NI; ++c) {
+      s_i[wave][c][lane] = e1[c];
+      s_i[wave][c][lane + 64] = e2[c];
+    }
+  }
+  if constexpr (!ENERGY) {
+    // ordered-pair convention, as in n3_item
+    const double m = cls == 1 ? 2. : 1.;
+    const double se = (double)a1.a + (double)a2.a, sw = (double)a1.b + (double)a2.b;
+    double te = m * 0.5 * (sw - se), tw = m * sw;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      te += __shfl_xor(te, o, 64);
+      tw += __shfl_xor(tw, o, 64);
+    }
+    if (lane == 0) {
+      s_ew[wave][0] = te;
+      s_ew[wave][1] = tw;
+    }
+  }
+  __syncthreads();
+
+  if constexpr (!ENERGY)
+    if (T < 2)
+      ew[2 * (size_t)blockIdx.x + T] = s_ew[0][T] + s_ew[1][T] + s_ew[2][T] + s_ew[3][T];
+  if (T < kTile) {  // i side: slot h
+    const int i = kTile * g + T;
+    float v[NI];
+#pragma unroll
+    for (int c = 0; c < NI; ++c) v[c] = (s_i[0][c][T] + s_i[1][c][T]) + (s_i[2][c][T] + s_i[3][c][T]);
+    if (i < N) {
+      if constexpr (ENERGY) {
+        store_part(fpart + (size_t)h * Npad + i, v[0], v[1], v[2], v[3]);
+        store_part(apart + (size_t)h * Npad + i, v[4]);
+      } else {
+        store_part3(fpart, (size_t)h * Npad + i, v[0], v[1], v[2]);
+      }
+    }
+  } else if (!diag) {  // j side: slot g
+    const int u = T - kTile, j = kTile * h + u, w = 2 * (u >> 6), x = u & 63;
+    float v[NJ];
+#pragma unroll
+    for (int c = 0; c < NJ; ++c) v[c] = s_j[w][c][x] + s_j[w + 1][c][x];
+    if (j < N) {
+      if constexpr (ENERGY) {
+        store_part(fpart + (size_t)g * Npad + j, v[0], v[1], v[2], 0.f);
+        store_part(apart + (size_t)g * Npad + j, v[3]);
+      } else {
+        store_part3(fpart, (size_t)g * Npad + j, v[0], v[1], v[2]);
+      }
+    }
+  }
 }
 
 // Compensated mode: one workgroup per item of the unpaired list (the diagonal
@@ -823,7 +955,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
 {
   __shared__ N3Lds<2> lds;
   const int2 it = items[blockIdx.x];
-  n3_item<PERIODIC, TIES, 2, ENERGY, false, true>(lds, q, pf, fpart, apart,
+  n3_item<PERIODIC, TIES, 2, ENERGY, true>(lds, q, pf, fpart, apart,
                                                   ENERGY ? nullptr : ew + 2 * (size_t)blockIdx.x, N,
                                                   Npad, C1, it.x, it.y);
 }
@@ -898,43 +1030,44 @@ double n3_pass_time(long n, double work, int cus)
   return w * work / n3_cu_rate(w);
 }
 
-int n3_split(int W, int ng)
+bool n3_small_groups(int W, int ng)
 {
-  // LJ_PAIR_ONCE_SPLIT=0 / 1 turns the split items off / on (groups of 256)
-  if (W != 2) return 1;
+  // LJ_PAIR_ONCE_SPLIT=0 / 1 turns the small items off / on (groups of 256)
+  if (W != 2) return false;
   const char* e = std::getenv("LJ_PAIR_ONCE_SPLIT");
-  if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1' ? 2 : 1;
+  if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
   int cus = 256, dev = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       cus <= 0)
     cus = 256;
-  // split when the model gives the split pass at least 10% less time (its
-  // twice as many partial slots cost the integrator about that much).
-  // Measured step times (TVN, N: split / unsplit us): 4096 21.3 / 32.6, 6144
-  // 26.4 / 33.7, 8192 34.6 / 34.5, 10000 44.6 / 47.2, 11264 48.9 / 48.4.
+  // where halves of the items on two workgroups each would by the model take at
+  // least 10% less time (twice as many partial slots cost the integrator about
+  // that much)
   const long full = (long)ng * (ng + 1) / 2, paired = (long)ng * (ng - 1) / 2 + (ng + 1) / 2;
-  return n3_pass_time(2 * full, 0.5, cus) < 0.9 * n3_pass_time(paired, 1.0, cus) ? 2 : 1;
+  return n3_pass_time(2 * full, 0.5, cus) < 0.9 * n3_pass_time(paired, 1.0, cus);
 }
 
 ForcePlan make_n3_plan(int N, bool comp)
 {
   ForcePlan pl;
-  const int W = comp ? 2 : n3_waves(N);
-  const int G = kTile * W;
+  int W = comp ? 2 : n3_waves(N);
+  int ng = (N + kTile * W - 1) / (kTile * W);
+  if (!comp && n3_small_groups(W, ng)) {
+    W = 1;
+    ng *= 2;
+  }
   pl.N = N;
   pl.n3 = W;
   pl.comp = comp ? 1 : 0;
-  pl.ng = (N + G - 1) / G;
-  pl.split = comp ? 1 : n3_split(W, pl.ng);
-  pl.S = pl.ng * pl.split;
-  pl.jchunk = G;
+  pl.ng = ng;
+  pl.S = ng;
+  pl.jchunk = kTile * W;
   pl.Npad = (N + 63) & ~63;
-  pl.nitems = pl.ng * (pl.ng + 1) / 2;
-  // the time step pairs its diagonal items (n3_step_items), unless split or
-  // compensated
-  pl.nitems_step = W == 2 && pl.split == 1 && !comp ? pl.ng * (pl.ng - 1) / 2 + (pl.ng + 1) / 2
-                                                    : pl.nitems;
+  pl.nitems = ng * (ng + 1) / 2;
+  // the time step of the groups of 256 pairs its diagonal items
+  // (n3_step_items), unless compensated
+  pl.nitems_step = W == 2 && !comp ? ng * (ng - 1) / 2 + (ng + 1) / 2 : pl.nitems;
   return pl;
 }
 
@@ -987,26 +1120,28 @@ void n3_step_items(const ForcePlan& pl, int2* out)
 
 namespace {
 
-template <int W, bool ENERGY, bool SPLIT>
+template <int W, bool ENERGY>
 hipError_t launch_n3_w(hipStream_t st, const ForcePlan& pl, const PairScalars& ps, const uint4* q,
                        const float4* posf, float4* fpart, float* apart, double* ew, bool ties)
 {
   // the time step's variant runs its own item list (diagonal items paired)
   const int nitems = ENERGY ? pl.nitems : pl.nitems_step;
   const int2* items = ENERGY ? pl.items : pl.items_step;
-  dim3 grid(nitems * (SPLIT ? 2 : 1)), block(64 * W * W);
+  dim3 grid(nitems), block(W == 1 ? 256 : 64 * W * W);
   const LaunchStamp ts = tl_force_stamp;
-  if (ps.periodic) {
-    if (ties)
-      hipExtLaunchKernelGGL((k_force_n3<true, true, W, ENERGY, SPLIT>), grid, block, 0, st, ts.start,
-                            ts.stop, 0, q, posf, items, fpart, apart, ew, pl.N, pl.Npad, ps.C1);
-    else
-      hipExtLaunchKernelGGL((k_force_n3<true, false, W, ENERGY, SPLIT>), grid, block, 0, st, ts.start,
-                            ts.stop, 0, q, posf, items, fpart, apart, ew, pl.N, pl.Npad, ps.C1);
-  } else {
-    hipExtLaunchKernelGGL((k_force_n3<false, false, W, ENERGY, SPLIT>), grid, block, 0, st, ts.start,
-                          ts.stop, 0, q, posf, items, fpart, apart, ew, pl.N, pl.Npad, ps.C1);
-  }
+#define LJ_N3(P, T)                                                                              \
+  do {                                                                                           \
+    if constexpr (W == 1)                                                                        \
+      hipExtLaunchKernelGGL((k_force_n3s<P, T, ENERGY>), grid, block, 0, st, ts.start, ts.stop, 0, \
+                            q, posf, items, fpart, apart, ew, pl.N, pl.Npad, ps.C1);             \
+    else                                                                                         \
+      hipExtLaunchKernelGGL((k_force_n3<P, T, W, ENERGY>), grid, block, 0, st, ts.start, ts.stop, 0, \
+                            q, posf, items, fpart, apart, ew, pl.N, pl.Npad, ps.C1);             \
+  } while (0)
+  if (!ps.periodic) LJ_N3(false, false);
+  else if (ties) LJ_N3(true, true);
+  else LJ_N3(true, false);
+#undef LJ_N3
   return hipGetLastError();
 }
 
@@ -1071,19 +1206,19 @@ hipError_t launch_force_n3_step_items(hipStream_t st, const ForcePlan& pl, const
 {
   // the step variant's items [first, first + count), each writing its own
   // partial entries and (E, W) totals: one GPU's share of a pass whose items
-  // are dealt out (W = 2, diagonal items paired, not split)
-  if (pl.n3 != 2 || pl.split != 1 || pl.comp || first < 0 || count < 1 ||
+  // are dealt out (W = 2, diagonal items paired)
+  if (pl.n3 != 2 || pl.comp || first < 0 || count < 1 ||
       first + count > pl.nitems_step)
     return hipErrorInvalidValue;
   const LaunchStamp ts = tl_force_stamp;
   const int2* items = pl.items_step + first;
   double* e = ew + 2 * (size_t)first;
   if (ps.periodic)
-    hipExtLaunchKernelGGL((k_force_n3<true, false, 2, false, false>), dim3(count), dim3(256), 0, st,
+    hipExtLaunchKernelGGL((k_force_n3<true, false, 2, false>), dim3(count), dim3(256), 0, st,
                           ts.start, ts.stop, 0, q, posf, items, fpart, nullptr, e, pl.N, pl.Npad,
                           ps.C1);
   else
-    hipExtLaunchKernelGGL((k_force_n3<false, false, 2, false, false>), dim3(count), dim3(256), 0,
+    hipExtLaunchKernelGGL((k_force_n3<false, false, 2, false>), dim3(count), dim3(256), 0,
                           st, ts.start, ts.stop, 0, q, posf, items, fpart, nullptr, e, pl.N, pl.Npad,
                           ps.C1);
   return hipGetLastError();
@@ -1094,21 +1229,19 @@ hipError_t launch_force_n3(hipStream_t st, const ForcePlan& pl, const PairScalar
                            bool ties, double* ew)
 {
   // ew != null: the time step's variant (force partials + per-workgroup totals)
-  if (pl.split == 2 && pl.n3 != 2) return hipErrorInvalidValue;
   if (pl.comp) {
-    if (pl.n3 != 2 || pl.split != 1 || pl.nitems_step != pl.nitems) return hipErrorInvalidValue;
+    if (pl.n3 != 2 || pl.nitems_step != pl.nitems) return hipErrorInvalidValue;
     return ew ? launch_n3_c<false>(st, pl, ps, q, posf, fpart, apart, ew, false)
               : launch_n3_c<true>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);
   }
   if (ew) {
-    if (pl.split == 2) return launch_n3_w<2, false, true>(st, pl, ps, q, posf, fpart, apart, ew, false);
-    if (pl.n3 == 2) return launch_n3_w<2, false, false>(st, pl, ps, q, posf, fpart, apart, ew, false);
-    return launch_n3_w<4, false, false>(st, pl, ps, q, posf, fpart, apart, ew, false);
+    if (pl.n3 == 1) return launch_n3_w<1, false>(st, pl, ps, q, posf, fpart, apart, ew, false);
+    if (pl.n3 == 2) return launch_n3_w<2, false>(st, pl, ps, q, posf, fpart, apart, ew, false);
+    return launch_n3_w<4, false>(st, pl, ps, q, posf, fpart, apart, ew, false);
   }
-  if (pl.split == 2)
-    return launch_n3_w<2, true, true>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);
-  if (pl.n3 == 2) return launch_n3_w<2, true, false>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);
-  return launch_n3_w<4, true, false>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);
+  if (pl.n3 == 1) return launch_n3_w<1, true>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);
+  if (pl.n3 == 2) return launch_n3_w<2, true>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);
+  return launch_n3_w<4, true>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);
 }
 
 }  // namespace lj

@@ -38,24 +38,25 @@ struct ForcePlan {
   int i0 = 0, i1 = 0;
   int iend() const { return i1 > 0 ? i1 : N; }
   bool sharded() const { return i0 != 0 || iend() != N; }
-  // pair-once kernel (lj_force_n3.hip): S = ng groups, one workgroup per item
+  // pair-once kernel (lj_force_n3.hip): n3 = waves per side of an item's
+  // groups of 128 n3 particles (1: the small items), S = ng groups, one
+  // workgroup per item
   int n3 = 0;
   int ng = 0;
   int nitems = 0;
   const int2* items = nullptr;  // device table of (g, h) group pairs
   // the time step's variant: nitems_step items (the diagonal items in pairs
-  // with W = 2 unless split)
+  // with n3 = 2)
   int nitems_step = 0;
   const int2* items_step = nullptr;
-  // workgroups per item: 2 splits every item's j sub-tiles between two
-  // workgroups (sizes whose items fill under half the resident workgroups);
-  // S = split x ng slots
+  // the FP64 pass: workgroups per item, 2 for sizes whose items fill under half
+  // the resident workgroups; S = split x ng slots
   int split = 1;
-  // 1: the compensated mode's pair-once pass (k_force_n3c: W = 2, not split,
+  // 1: the compensated mode's pair-once pass (k_force_n3c: n3 = 2,
   // diagonal items unpaired)
   int comp = 0;
   // workgroups of the time step's pass, one (E, W) pair of totals each
-  int step_wgs() const { return nitems_step * split; }
+  int step_wgs() const { return nitems_step; }
 };
 ForcePlan make_force_plan(int N, int jslices_override, int ipl);
 // one GPU's share of a force pass sharded by i over nshards <= ceil(N / 64)
@@ -93,7 +94,7 @@ hipError_t launch_prep_q(hipStream_t st, const float4* pos, uint4* q, int N, dou
 // writes force-only partials and per-workgroup (E, W) totals to step_ew
 struct StepArgs;
 // the time step's pair-once pass on its items [first, first + count) (W = 2,
-// paired diagonal items, not split): one GPU's share when items are dealt out
+// paired diagonal items): one GPU's share when items are dealt out
 hipError_t launch_force_n3_step_items(hipStream_t st, const ForcePlan& pl, const PairScalars& ps,
                                       const uint4* q, const float4* posf, float4* fpart, double* ew,
                                       int first, int count);

@@ -219,6 +219,33 @@ def test_pair_once_split_items(N, bc, split_env):
     assert dU <= 1e-5 and dx <= 1e-4, (dU, dx)
 
 
+@pytest.mark.parametrize("bc", [ljamd.BC_PERIODIC, ljamd.BC_WALL])
+@pytest.mark.parametrize("N", [4097, 4161, 4224, 4225, 7808])
+def test_small_items_edges(N, bc):
+    """The pair-once pass over groups of 128 where its last group is past N
+    (4097, 4161, 4224; the group count is even), holds one particle (4225) or
+    nothing is left over (7808), its sub-tile of 64 holds one (4161): forces of a
+    single evaluation against FP64 at the bounds of the pass over groups of 256,
+    and a step's totals against a full evaluation.  (V and W against FP64: the
+    test above; here V is 0.3% of W, and its error that of the fixed-point
+    positions.)"""
+    rho = 0.85
+    L, pos, vel = perturbed_state(N, rho, 1.0, seed=54)
+    with ljamd.LJSystem(N, rho, 1.0, canonical=ljamd.TVN, boundary=bc) as s:
+        assert s.force_plan() == (True, 2 * ((N + 255) // 256))
+        s.set_state(pos, vel)
+        s.CalculateForces()
+        f4 = s.force
+        h = s.Integrate(0.005, 3)
+        o_step = s.observables()
+        o_full = s.CalculateForces()
+    F64, _, _, _ = forces_fp64(pos, L, bc == ljamd.BC_PERIODIC)
+    err = force_errors(xyz(f4), F64)
+    assert err["global_rel"] <= 2e-6 and err["max_rel_floor"] <= 1e-5, err
+    assert abs(h[-1, 3] - o_full["V"]) <= 1e-6 * abs(o_full["V"])
+    assert abs(o_step["W"] - o_full["W"]) <= 1e-6 * abs(o_full["W"])
+
+
 # the kernel choice at the sizes the measurements cover (rho* = 0.85, FP32):
 # (N, pair-once, partial slots per particle); split items give 2 per group
 PLAN_CASES = [(2048, False, 32), (3071, False, 48), (3072, True, 24), (4096, True, 32),
