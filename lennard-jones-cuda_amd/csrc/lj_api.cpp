@@ -1309,10 +1309,13 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
   if (Lperiodic && !(host_L > 0.f)) return fail(LJ_ERR_ARG, "calculateNForces: box side must be positive");
   if (host_RDF && !(host_dr2 > 0.f)) return fail(LJ_ERR_ARG, "calculateNForces: RDF bin width must be positive");
   LJ_TRY(check_device());
-  const ForcePlan pl = make_force_plan(N, 0, 1);
   const PairScalars ps = make_pair_scalars((double)host_L, Lperiodic != 0, 1., 1., true);
   CompatScratch* s = nullptr;
-  LJ_TRY(compat_scratch(N, pl, &s));
+  ForcePlan pl = compat_plan(N, ps);
+  if (compat_scratch(N, pl, &s) != LJ_OK) {  // no room for its partial sums
+    pl = make_force_plan(N, 0, 1);
+    LJ_TRY(compat_scratch(N, pl, &s));
+  }
   hipStream_t st = s->st;
   const float4* p = reinterpret_cast<const float4*>(Pos);
   if (ps.periodic) LJ_HIP(launch_prep_q(st, p, s->q, N, ps.qscale));

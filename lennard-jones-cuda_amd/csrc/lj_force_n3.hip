@@ -66,6 +66,20 @@ struct N3Lds {
   double ew[W * W][2];
 };
 
+// the pair's factors from its separation; returns r2
+template <bool GUARD>
+__device__ __forceinline__ float factors(float dx, float dy, float dz, float C1, bool ok, float& s,
+                                         float& e6, float& w)
+{
+  const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+  float ir2 = __builtin_amdgcn_rcpf(r2) * C1;
+  if constexpr (GUARD) ir2 = ok ? ir2 : 0.f;
+  e6 = ir2 * ir2 * ir2;
+  w = e6 * __builtin_fmaf(e6, 2.f, -1.f);
+  s = w * ir2;
+  return r2;
+}
+
 template <bool PERIODIC, bool TIES, bool GUARD>
 __device__ __forceinline__ void terms(const PosT<PERIODIC>& pi, const uint4& pj, float C1, bool ok,
                                       float& dx, float& dy, float& dz, float& s, float& e6,
@@ -80,13 +94,48 @@ __device__ __forceinline__ void terms(const PosT<PERIODIC>& pi, const uint4& pj,
     dy = pi.y - __uint_as_float(pj.y);
     dz = pi.z - __uint_as_float(pj.z);
   }
-  const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-  float ir2 = __builtin_amdgcn_rcpf(r2) * C1;
-  if constexpr (GUARD) ir2 = ok ? ir2 : 0.f;
-  e6 = ir2 * ir2 * ir2;
-  w = e6 * __builtin_fmaf(e6, 2.f, -1.f);
-  s = w * ir2;
+  factors<GUARD>(dx, dy, dz, C1, ok, s, e6, w);
 }
+
+// The pairs with r2 <= thr, or not comparable, that a pass leaves out (EXCL):
+// kLook notes the least r2 on the way (half an instruction a pair), kTest leaves
+// them out pair by pair.
+enum { kNone = 0, kLook = 1, kTest = 2 };
+struct Excl {
+  float thr, least;
+};
+
+// A lane's particle as the i of a pair.  Periodic boxes with exact ties take the
+// mirrored frame (MirPos): no compare and select per axis, but the j side, whose
+// sums travel through lanes of other frames, needs the frame's sign: g = -s_a,
+// one select an axis (a full evaluation at N = 16384: 131 us with the
+// compares and selects of the unmirrored form, 124 so).
+template <bool PERIODIC, bool TIES>
+struct SideI {
+  LaneI<PERIODIC, TIES> li;
+  __device__ __forceinline__ explicit SideI(const PosT<PERIODIC>& p) { li.set(p); }
+  // separation and factors of the pair with pj, where ok (GUARD); returns r2
+  template <bool GUARD, int EXCL>
+  __device__ __forceinline__ float meet(const uint4& pj, float C1, float thr, bool ok, float& dx,
+                                        float& dy, float& dz, float& s, float& e6, float& w) const
+  {
+    PosT<PERIODIC> p;
+    if constexpr (PERIODIC) p.x = pj.x, p.y = pj.y, p.z = pj.z;
+    else p.x = __uint_as_float(pj.x), p.y = __uint_as_float(pj.y), p.z = __uint_as_float(pj.z);
+    sep(li.p, p, dx, dy, dz);
+    if constexpr (EXCL == kTest)
+      ok = ok && __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)) > thr;
+    return factors<GUARD || EXCL == kTest>(dx, dy, dz, C1, ok, s, e6, w);
+  }
+  // j sums minus this pair's force, from the frame
+  __device__ __forceinline__ void react(float dx, float dy, float dz, float s, float& jx, float& jy,
+                                        float& jz) const
+  {
+    jx = __builtin_fmaf(dx, li.p.mx ? -s : s, jx);
+    jy = __builtin_fmaf(dy, li.p.my ? -s : s, jy);
+    jz = __builtin_fmaf(dz, li.p.mz ? -s : s, jz);
+  }
+};
 
 // rotate a value one lane down the wave: lane l receives lane (l + 1) mod 64.
 // ds_bpermute does the gather in the LDS unit, off the VALU that bounds the
@@ -103,12 +152,12 @@ __device__ __forceinline__ float rot1(float v)
 }
 
 // STEPS steps from t0 on of one j sub-tile P (64 particles, doubled): i sums in
-// a1/a2, the j sums in j[] travelling with their j particle
-template <bool PERIODIC, bool TIES, bool PARTIAL, bool ENERGY, int STEPS>
+// a1/a2 (in the lanes' frames), the j sums in j[] travelling with their j particle
+template <bool PERIODIC, bool TIES, bool PARTIAL, bool ENERGY, int EXCL, int STEPS>
 __device__ __forceinline__ void pair_steps(const uint4* P, int t0, int lane,
-                                           const PosT<PERIODIC>& pi1, const PosT<PERIODIC>& pi2,
-                                           bool v1, bool v2, float C1, Acc& a1, Acc& a2,
-                                           float (&j)[4])
+                                           const SideI<PERIODIC, TIES>& i1,
+                                           const SideI<PERIODIC, TIES>& i2, bool v1, bool v2,
+                                           float C1, Excl& ex, Acc& a1, Acc& a2, float (&j)[4])
 {
   float jx = 0.f, jy = 0.f, jz = 0.f, jm = 0.f;
 #pragma unroll 8
@@ -121,8 +170,9 @@ __device__ __forceinline__ void pair_steps(const uint4* P, int t0, int lane,
       ok2 = v2 && jv;
     }
     float dx1, dy1, dz1, s1, e1, w1, dx2, dy2, dz2, s2, e2, w2;
-    terms<PERIODIC, TIES, PARTIAL>(pi1, pj, C1, ok1, dx1, dy1, dz1, s1, e1, w1);
-    terms<PERIODIC, TIES, PARTIAL>(pi2, pj, C1, ok2, dx2, dy2, dz2, s2, e2, w2);
+    const float r1 = i1.template meet<PARTIAL, EXCL>(pj, C1, ex.thr, ok1, dx1, dy1, dz1, s1, e1, w1);
+    const float r2 = i2.template meet<PARTIAL, EXCL>(pj, C1, ex.thr, ok2, dx2, dy2, dz2, s2, e2, w2);
+    if constexpr (EXCL == kLook) ex.least = __builtin_fminf(ex.least, __builtin_fminf(r1, r2));
     a1.fx = __builtin_fmaf(dx1, s1, a1.fx);
     a1.fy = __builtin_fmaf(dy1, s1, a1.fy);
     a1.fz = __builtin_fmaf(dz1, s1, a1.fz);
@@ -133,9 +183,14 @@ __device__ __forceinline__ void pair_steps(const uint4* P, int t0, int lane,
     a2.fz = __builtin_fmaf(dz2, s2, a2.fz);
     a2.a += e2;
     a2.b += w2;
-    jx = __builtin_fmaf(-dx2, s2, __builtin_fmaf(-dx1, s1, jx));
-    jy = __builtin_fmaf(-dy2, s2, __builtin_fmaf(-dy1, s1, jy));
-    jz = __builtin_fmaf(-dz2, s2, __builtin_fmaf(-dz1, s1, jz));
+    if constexpr (PERIODIC && TIES) {
+      i1.react(dx1, dy1, dz1, s1, jx, jy, jz);
+      i2.react(dx2, dy2, dz2, s2, jx, jy, jz);
+    } else {
+      jx = __builtin_fmaf(-dx2, s2, __builtin_fmaf(-dx1, s1, jx));
+      jy = __builtin_fmaf(-dy2, s2, __builtin_fmaf(-dy1, s1, jy));
+      jz = __builtin_fmaf(-dz2, s2, __builtin_fmaf(-dz1, s1, jz));
+    }
     jx = rot1(jx);
     jy = rot1(jy);
     jz = rot1(jz);
@@ -150,69 +205,85 @@ __device__ __forceinline__ void pair_steps(const uint4* P, int t0, int lane,
   j[3] = jm;
 }
 
-// one tile pair evaluated once: i sums in a1/a2; j sums in registers that
-// travel with their j particle (lane l holds the sums of j slot (l + t) mod 64
-// at step t and passes them to lane l - 1 afterwards), so after 64 steps lane l
-// holds those of slot l.  J receives (-fx, -fy, -fz, sum (s/r)^6 - w) per
+// One tile pair evaluated once, sub-tiles [0, nsub) of 64 j (SUBS = 2) or one
+// (SUBS = 1), STEPS steps from t0 on each; i sums in a1/a2; j sums in registers
+// that travel with their j particle (lane l holds the sums of j slot (l + t) mod
+// 64 at step t and passes them to lane l - 1 afterwards), so after 64 steps lane
+// l holds those of slot l.  J receives (-fx, -fy, -fz, sum (s/r)^6 - w) per
 // sub-tile.
 // nsub: sub-tiles holding a valid j (1 when the second one is past N)
-template <bool PERIODIC, bool TIES, bool PARTIAL, bool ENERGY>
+template <bool PERIODIC, bool TIES, bool PARTIAL, bool ENERGY, int EXCL = kNone, int SUBS = 2,
+          int STEPS = 64>
 __device__ __forceinline__ void pair_tile(const uint4* P0, int lane, const PosT<PERIODIC>& pi1,
                                           const PosT<PERIODIC>& pi2, bool v1, bool v2, float C1,
-                                          int nsub, Acc& a1, Acc& a2, float (&J)[2][4])
+                                          int nsub, Acc& a1, Acc& a2, float (&J)[SUBS][4],
+                                          float thr = 0.f, int t0 = 0)
 {
+  const SideI<PERIODIC, TIES> i1(pi1), i2(pi2);
+  Excl ex{thr, __builtin_inff()};
 #pragma unroll
-  for (int st = 0; st < 2; ++st) {
+  for (int st = 0; st < SUBS; ++st) {
     if (st >= nsub) break;  // wave-uniform
-    pair_steps<PERIODIC, TIES, PARTIAL, ENERGY, 64>(P0 + st * 128, 0, lane, pi1, pi2, v1, v2, C1, a1,
-                                                    a2, J[st]);
+    pair_steps<PERIODIC, TIES, PARTIAL, ENERGY, EXCL, STEPS>(P0 + st * 128, t0, lane, i1, i2, v1, v2,
+                                                             C1, ex, a1, a2, J[st]);
   }
+  if constexpr (EXCL == kLook) {
+    // a pair to leave out shows in the least r2 or, with an r2 that is not a
+    // number, in the sums: the tile is then taken again pair by pair, the same
+    // sums without those pairs
+    const bool bad = !(ex.least > thr) || a1.a != a1.a || a1.b != a1.b || a2.a != a2.a || a2.b != a2.b;
+    if (__any(bad)) {
+      acc_zero(a1);
+      acc_zero(a2);
+      for (int st = 0; st < SUBS; ++st) {
+        if (st >= nsub) break;
+        pair_steps<PERIODIC, TIES, true, ENERGY, kTest, STEPS>(P0 + st * 128, t0, lane, i1, i2, v1,
+                                                               v2, C1, ex, a1, a2, J[st]);
+      }
+    }
+  }
+  i1.li.common_frame(a1);
+  i2.li.common_frame(a2);
 }
 
-// STEPS steps from t0 on of the lane's i particles against one j sub-tile P (j
-// numbers from jbase on), i sums only, self pair excluded
-template <bool PERIODIC, bool TIES, int STEPS>
-__device__ __forceinline__ void self_steps(const uint4* P, int t0, int lane, int i1, int i2,
-                                           int jbase, const PosT<PERIODIC>& pi1,
-                                           const PosT<PERIODIC>& pi2, bool v1, bool v2, float C1,
-                                           Acc& a1, Acc& a2)
-{
-#pragma unroll 8
-  for (int t = 0; t < STEPS; ++t) {
-    const int jx = lane + t0 + t;
-    const uint4 pj = P[jx];
-    const int j = jbase + (jx & 63);
-    const bool jv = pj.w != 0u;
-    const bool ok1 = v1 && jv && j != i1;
-    const bool ok2 = v2 && jv && j != i2;
-    float dx, dy, dz, s, e, w;
-    terms<PERIODIC, TIES, true>(pi1, pj, C1, ok1, dx, dy, dz, s, e, w);
-    a1.fx = __builtin_fmaf(dx, s, a1.fx);
-    a1.fy = __builtin_fmaf(dy, s, a1.fy);
-    a1.fz = __builtin_fmaf(dz, s, a1.fz);
-    a1.a += e;
-    a1.b += w;
-    terms<PERIODIC, TIES, true>(pi2, pj, C1, ok2, dx, dy, dz, s, e, w);
-    a2.fx = __builtin_fmaf(dx, s, a2.fx);
-    a2.fy = __builtin_fmaf(dy, s, a2.fy);
-    a2.fz = __builtin_fmaf(dz, s, a2.fz);
-    a2.a += e;
-    a2.b += w;
-  }
-}
-
-// both orders of the wave's own tile, i sums only, self pair excluded
-template <bool PERIODIC, bool TIES>
+// both orders of the wave's own tile, i sums only, self pair (and with EXCL
+// those to leave out) excluded; sub-tiles and steps as in pair_tile
+template <bool PERIODIC, bool TIES, int EXCL = kNone, int SUBS = 2, int STEPS = 64>
 __device__ __forceinline__ void self_tile(const uint4* P0, int lane, int i1, int i2, int jbase,
                                           const PosT<PERIODIC>& pi1, const PosT<PERIODIC>& pi2,
-                                          bool v1, bool v2, float C1, int nsub, Acc& a1, Acc& a2)
+                                          bool v1, bool v2, float C1, int nsub, Acc& a1, Acc& a2,
+                                          float thr = 0.f, int t0 = 0)
 {
+  const SideI<PERIODIC, TIES> s1(pi1), s2(pi2);
 #pragma unroll
-  for (int st = 0; st < 2; ++st) {
+  for (int st = 0; st < SUBS; ++st) {
     if (st >= nsub) break;  // wave-uniform
-    self_steps<PERIODIC, TIES, 64>(P0 + st * 128, 0, lane, i1, i2, jbase + st * 64, pi1, pi2, v1, v2,
-                                   C1, a1, a2);
+    const uint4* P = P0 + st * 128;
+#pragma unroll 8
+    for (int t = 0; t < STEPS; ++t) {
+      const int jx = lane + t0 + t;
+      const uint4 pj = P[jx];
+      const int j = jbase + st * 64 + (jx & 63);
+      const bool jv = pj.w != 0u;
+      const bool ok1 = v1 && jv && j != i1;
+      const bool ok2 = v2 && jv && j != i2;
+      float dx, dy, dz, s, e, w;
+      s1.template meet<true, EXCL ? kTest : kNone>(pj, C1, thr, ok1, dx, dy, dz, s, e, w);
+      a1.fx = __builtin_fmaf(dx, s, a1.fx);
+      a1.fy = __builtin_fmaf(dy, s, a1.fy);
+      a1.fz = __builtin_fmaf(dz, s, a1.fz);
+      a1.a += e;
+      a1.b += w;
+      s2.template meet<true, EXCL ? kTest : kNone>(pj, C1, thr, ok2, dx, dy, dz, s, e, w);
+      a2.fx = __builtin_fmaf(dx, s, a2.fx);
+      a2.fy = __builtin_fmaf(dy, s, a2.fy);
+      a2.fz = __builtin_fmaf(dz, s, a2.fz);
+      a2.a += e;
+      a2.b += w;
+    }
   }
+  s1.li.common_frame(a1);
+  s2.li.common_frame(a2);
 }
 
 // rotate by k lanes: lane l receives lane (l + k) mod 64 (full execution mask)
@@ -613,12 +684,13 @@ __device__ __forceinline__ void n3_diag_pair(N3Lds<2>& lds, const uint4* __restr
 // One group pair (g, h) of one box: q/pf/fpart/apart point at the box's
 // arrays, ew (ENERGY = false) at the workgroup's two totals.
 // COMP: the compensated mode's sums (pair_tile_c, self_tile_c; W = 2).
-template <bool PERIODIC, bool TIES, int W, bool ENERGY, bool COMP = false>
+// EXCL (kLook): pairs with r2 <= thr are left out.
+template <bool PERIODIC, bool TIES, int W, bool ENERGY, bool COMP = false, int EXCL = kNone>
 __device__ __forceinline__ void n3_item(N3Lds<W>& lds, const uint4* __restrict__ q,
                                         const float4* __restrict__ pf,
                                         float4* __restrict__ fpart, float* __restrict__ apart,
                                         double* __restrict__ ew, int N, int Npad, float C1, int g,
-                                        int h)
+                                        int h, float thr = 0.f)
 {
   constexpr int kG = kTile * W;
   uint4* const s_pos = lds.pos;
@@ -683,12 +755,14 @@ __device__ __forceinline__ void n3_item(N3Lds<W>& lds, const uint4* __restrict__
     a2.fx += l2.fx, a2.fy += l2.fy, a2.fz += l2.fz, a2.a += l2.a, a2.b += l2.b;
   } else if (cls == 1) {
     if (partial)
-      pair_tile<PERIODIC, TIES, true, ENERGY>(P0, lane, pi1, pi2, v1, v2, C1, nsub, a1, a2, J);
+      pair_tile<PERIODIC, TIES, true, ENERGY, EXCL>(P0, lane, pi1, pi2, v1, v2, C1, nsub, a1, a2, J,
+                                                    thr);
     else
-      pair_tile<PERIODIC, TIES, false, ENERGY>(P0, lane, pi1, pi2, v1, v2, C1, 2, a1, a2, J);
+      pair_tile<PERIODIC, TIES, false, ENERGY, EXCL>(P0, lane, pi1, pi2, v1, v2, C1, 2, a1, a2, J,
+                                                     thr);
   } else if (cls == 2) {
-    self_tile<PERIODIC, TIES>(P0, lane, i1, i2, kG * h + kTile * wj, pi1, pi2, v1, v2, C1, nsub, a1,
-                              a2);
+    self_tile<PERIODIC, TIES, EXCL>(P0, lane, i1, i2, kG * h + kTile * wj, pi1, pi2, v1, v2, C1, nsub,
+                                    a1, a2, thr);
   }
   {
     float* A = s_acc + wave * kAccPerWave;
@@ -792,23 +866,38 @@ __device__ __forceinline__ void n3_item(N3Lds<W>& lds, const uint4* __restrict__
   }
 }
 
-template <bool PERIODIC, bool TIES, int W, bool ENERGY>
-__global__ __launch_bounds__(64 * W * W) __attribute__((amdgpu_waves_per_eu(8))) void k_force_n3(
+// item k of ng groups in row order: (g, h) with h >= g; row g starts at
+// g ng - g (g - 1) / 2
+__device__ __forceinline__ int2 row_item(int k, int ng)
+{
+  const float b = ng + 0.5f;
+  int g = max(0, min(ng - 1, (int)(b - sqrtf(fmaxf(b * b - 2.f * k, 0.f)))));
+  while (g > 0 && g * ng - g * (g - 1) / 2 > k) --g;
+  while ((g + 1) * ng - (g + 1) * g / 2 <= k) ++g;
+  return make_int2(g, g + k - (g * ng - g * (g - 1) / 2));
+}
+
+// EXCL (single evaluations that leave out pairs with r2 <= thr): no item table,
+// items in row order
+// The tie rule's frames take about six more registers: seven waves per SIMD then.
+template <bool PERIODIC, bool TIES, int W, bool ENERGY, int EXCL = kNone>
+__global__ __launch_bounds__(64 * W * W) __attribute__((amdgpu_waves_per_eu(TIES && W == 2 ? 7 : 8))) void k_force_n3(
     const uint4* __restrict__ q, const float4* __restrict__ pf, const int2* __restrict__ items,
     float4* __restrict__ fpart, float* __restrict__ apart, double* __restrict__ ew, int N, int Npad,
-    float C1)
+    float C1, int ng, float thr)
 {
   __shared__ N3Lds<W> lds;
   const int k = blockIdx.x;  // item
-  const int2 it = items[k];
+  const int2 it = EXCL ? row_item(k, ng) : items[k];
   if constexpr (!ENERGY && W == 2) {
     if (it.y < 0) {  // diagonal pair (it.x, -2 - it.y), the second one absent when -1
       n3_diag_pair<PERIODIC>(lds, q, pf, fpart, ew + 2 * (size_t)k, N, Npad, C1, it.x, -2 - it.y);
       return;
     }
   }
-  n3_item<PERIODIC, TIES, W, ENERGY>(lds, q, pf, fpart, apart, ENERGY ? nullptr : ew + 2 * (size_t)k,
-                                     N, Npad, C1, it.x, it.y);
+  n3_item<PERIODIC, TIES, W, ENERGY, false, EXCL>(lds, q, pf, fpart, apart,
+                                                  ENERGY ? nullptr : ew + 2 * (size_t)k, N, Npad, C1,
+                                                  it.x, it.y, thr);
 }
 
 // Small items: a pair of groups of 128 per workgroup of four waves; wave w takes
@@ -820,18 +909,18 @@ __global__ __launch_bounds__(64 * W * W) __attribute__((amdgpu_waves_per_eu(8)))
 // (13.6 us against 7.6 us of issue).  As 820 small items the waves are half as
 // long and three or four share a SIMD; the partial slots are those of the
 // halved items.
-template <bool PERIODIC, bool TIES, bool ENERGY>
+template <bool PERIODIC, bool TIES, bool ENERGY, int EXCL = kNone>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_force_n3s(
     const uint4* __restrict__ q, const float4* __restrict__ pf, const int2* __restrict__ items,
     float4* __restrict__ fpart, float* __restrict__ apart, double* __restrict__ ew, int N, int Npad,
-    float C1)
+    float C1, int ng, float thr)
 {
   constexpr int NI = ENERGY ? 5 : 3, NJ = ENERGY ? 4 : 3;
   __shared__ uint4 s_pos[2 * 128];       // [sub-tile][doubled 64]
   __shared__ float s_j[4][NJ][64];       // j sums [wave][component][slot]
   __shared__ float s_i[4][NI][kTile];    // i sums [wave][component][i]
   __shared__ double s_ew[4][2];
-  const int2 it = items[blockIdx.x];
+  const int2 it = EXCL ? row_item(blockIdx.x, ng) : items[blockIdx.x];
   const int g = it.x, h = it.y;
   const int T = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(T >> 6);
@@ -865,21 +954,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
   Acc a1, a2;
   acc_zero(a1);
   acc_zero(a2);
-  float J[4] = {0.f, 0.f, 0.f, 0.f};
+  float J[1][4] = {{0.f, 0.f, 0.f, 0.f}};
   if (cls == 1) {  // g < h: every i is valid
     if (jb + 64 > N)
-      pair_steps<PERIODIC, TIES, true, ENERGY, 32>(s_pos + st * 128, t0, lane, pi1, pi2, v1, v2, C1,
-                                                   a1, a2, J);
+      pair_tile<PERIODIC, TIES, true, ENERGY, EXCL, 1, 32>(s_pos + st * 128, lane, pi1, pi2, v1, v2, C1,
+                                                           1, a1, a2, J, thr, t0);
     else
-      pair_steps<PERIODIC, TIES, false, ENERGY, 32>(s_pos + st * 128, t0, lane, pi1, pi2, v1, v2, C1,
-                                                    a1, a2, J);
+      pair_tile<PERIODIC, TIES, false, ENERGY, EXCL, 1, 32>(s_pos + st * 128, lane, pi1, pi2, v1, v2,
+                                                            C1, 1, a1, a2, J, thr, t0);
   } else if (cls == 2) {
-    self_steps<PERIODIC, TIES, 32>(s_pos + st * 128, t0, lane, i1, i2, jb, pi1, pi2, v1, v2, C1, a1,
-                                   a2);
+    self_tile<PERIODIC, TIES, EXCL, 1, 32>(s_pos + st * 128, lane, i1, i2, jb, pi1, pi2, v1, v2, C1, 1,
+                                           a1, a2, thr, t0);
   }
   // after the steps lane l holds the sums of j slot (l + t0 + 32) mod 64
 #pragma unroll
-  for (int c = 0; c < NJ; ++c) s_j[wave][c][(lane + t0 + 32) & 63] = J[c];
+  for (int c = 0; c < NJ; ++c) s_j[wave][c][(lane + t0 + 32) & 63] = J[0][c];
   {
     float e1[5], e2[5];
     encode(a1, cls, e1);
@@ -1071,6 +1160,15 @@ ForcePlan make_n3_plan(int N, bool comp)
   return pl;
 }
 
+ForcePlan compat_plan(int N, const PairScalars& ps)
+{
+  if (n3_eligible(N) && N <= kCompatOnceMaxN && ps.thr > 0.f) {
+    const ForcePlan pl = make_n3_plan(N);
+    if (pl.n3 != 4) return pl;
+  }
+  return make_force_plan(N, 0, 1);
+}
+
 bool n3_comp_enabled()
 {
   // LJ_PAIR_ONCE_COMP=0 keeps the compensated mode on the sliced kernel
@@ -1120,7 +1218,7 @@ void n3_step_items(const ForcePlan& pl, int2* out)
 
 namespace {
 
-template <int W, bool ENERGY>
+template <int W, bool ENERGY, int EXCL = kNone>
 hipError_t launch_n3_w(hipStream_t st, const ForcePlan& pl, const PairScalars& ps, const uint4* q,
                        const float4* posf, float4* fpart, float* apart, double* ew, bool ties)
 {
@@ -1129,18 +1227,21 @@ hipError_t launch_n3_w(hipStream_t st, const ForcePlan& pl, const PairScalars& p
   const int2* items = ENERGY ? pl.items : pl.items_step;
   dim3 grid(nitems), block(W == 1 ? 256 : 64 * W * W);
   const LaunchStamp ts = tl_force_stamp;
-#define LJ_N3(P, T)                                                                              \
-  do {                                                                                           \
-    if constexpr (W == 1)                                                                        \
-      hipExtLaunchKernelGGL((k_force_n3s<P, T, ENERGY>), grid, block, 0, st, ts.start, ts.stop, 0, \
-                            q, posf, items, fpart, apart, ew, pl.N, pl.Npad, ps.C1);             \
-    else                                                                                         \
-      hipExtLaunchKernelGGL((k_force_n3<P, T, W, ENERGY>), grid, block, 0, st, ts.start, ts.stop, 0, \
-                            q, posf, items, fpart, apart, ew, pl.N, pl.Npad, ps.C1);             \
+#define LJ_N3(P, T)                                                                               \
+  do {                                                                                            \
+    if constexpr (W == 1)                                                                         \
+      hipExtLaunchKernelGGL((k_force_n3s<P, T, ENERGY, EXCL>), grid, block, 0, st, ts.start,      \
+                            ts.stop, 0, q, posf, items, fpart, apart, ew, pl.N, pl.Npad, ps.C1,   \
+                            pl.ng, ps.thr);                                                       \
+    else                                                                                          \
+      hipExtLaunchKernelGGL((k_force_n3<P, T, W, ENERGY, EXCL>), grid, block, 0, st, ts.start,    \
+                            ts.stop, 0, q, posf, items, fpart, apart, ew, pl.N, pl.Npad, ps.C1,   \
+                            pl.ng, ps.thr);                                                       \
   } while (0)
   if (!ps.periodic) LJ_N3(false, false);
-  else if (ties) LJ_N3(true, true);
-  else LJ_N3(true, false);
+  else if (!ties) LJ_N3(true, false);
+  else if constexpr (ENERGY) LJ_N3(true, true);
+  else return hipErrorInvalidValue;  // the time step has no exact-tie rule
 #undef LJ_N3
   return hipGetLastError();
 }
@@ -1216,11 +1317,11 @@ hipError_t launch_force_n3_step_items(hipStream_t st, const ForcePlan& pl, const
   if (ps.periodic)
     hipExtLaunchKernelGGL((k_force_n3<true, false, 2, false>), dim3(count), dim3(256), 0, st,
                           ts.start, ts.stop, 0, q, posf, items, fpart, nullptr, e, pl.N, pl.Npad,
-                          ps.C1);
+                          ps.C1, pl.ng, 0.f);
   else
     hipExtLaunchKernelGGL((k_force_n3<false, false, 2, false>), dim3(count), dim3(256), 0,
                           st, ts.start, ts.stop, 0, q, posf, items, fpart, nullptr, e, pl.N, pl.Npad,
-                          ps.C1);
+                          ps.C1, pl.ng, 0.f);
   return hipGetLastError();
 }
 
@@ -1229,6 +1330,7 @@ hipError_t launch_force_n3(hipStream_t st, const ForcePlan& pl, const PairScalar
                            bool ties, double* ew)
 {
   // ew != null: the time step's variant (force partials + per-workgroup totals)
+  if (ps.thr > 0.f && (pl.comp || ew)) return hipErrorInvalidValue;
   if (pl.comp) {
     if (pl.n3 != 2 || pl.nitems_step != pl.nitems) return hipErrorInvalidValue;
     return ew ? launch_n3_c<false>(st, pl, ps, q, posf, fpart, apart, ew, false)
@@ -1238,6 +1340,13 @@ hipError_t launch_force_n3(hipStream_t st, const ForcePlan& pl, const PairScalar
     if (pl.n3 == 1) return launch_n3_w<1, false>(st, pl, ps, q, posf, fpart, apart, ew, false);
     if (pl.n3 == 2) return launch_n3_w<2, false>(st, pl, ps, q, posf, fpart, apart, ew, false);
     return launch_n3_w<4, false>(st, pl, ps, q, posf, fpart, apart, ew, false);
+  }
+  if (ps.thr > 0.f) {  // pairs with r2 <= thr left out
+    if (pl.n3 == 1)
+      return launch_n3_w<1, true, kLook>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);
+    if (pl.n3 == 2)
+      return launch_n3_w<2, true, kLook>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);
+    return hipErrorInvalidValue;
   }
   if (pl.n3 == 1) return launch_n3_w<1, true>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);
   if (pl.n3 == 2) return launch_n3_w<2, true>(st, pl, ps, q, posf, fpart, apart, nullptr, ties);

@@ -65,6 +65,14 @@ ForcePlan make_force_plan(int N, int jslices_override, int ipl);
 // grid, jslices j slices (0: enough to fill the device at that share)
 ForcePlan make_shard_plan(int N, int shard, int nshards, int jslices);
 ForcePlan make_n3_plan(int N, bool comp = false);
+// The plan of calculateNForces and its no-allocation twin: every pair once from
+// the sizes on at which the time step does so (N = 16384 periodic: 159 against 104
+// us), up to kCompatOnceMaxN particles, since the twin's partial sums, an entry
+// per particle and group, are a file-scope array (81 MiB at that size); else the
+// sliced grid.
+constexpr int kCompatOnceMaxN = 32768;
+struct PairScalars;
+ForcePlan compat_plan(int N, const PairScalars& ps);
 // false when LJ_PAIR_ONCE_COMP=0 keeps the compensated mode on the sliced kernel
 bool n3_comp_enabled();
 // sizes at which the pair-once kernel serves the time step (N >= 3072)

@@ -1132,7 +1132,7 @@ hipError_t launch_force(hipStream_t st, const ForcePlan& pl, const PairScalars& 
 {
   const bool ga = ps.thr > 0.f;
   // the pair-once pass of the matching mode (plans are made per context)
-  if (pl.n3 && compensated == (pl.comp != 0) && !ga)
+  if (pl.n3 && compensated == (pl.comp != 0))
     return launch_force_n3(st, pl, ps, q, posf, fpart, apart, ties, step_ew);
   if (ps.periodic) {
     if (ties)

@@ -23,9 +23,11 @@ using namespace lj;
 
 // largest numBodies served
 constexpr int kNoAllocMaxN = 65536;
-// entries S x Npad of the sliced plan (make_force_plan(N, 0, 1)) at any
-// N <= kNoAllocMaxN: at most 587520 (N = 65280: 9 slices of 65280)
-constexpr size_t kPartCap = 589824;
+// entries S x Npad of compat_plan at any N <= kNoAllocMaxN: the pair-once pass of
+// kCompatOnceMaxN particles in groups of 256; the sliced plan (make_force_plan(N,
+// 0, 1)) has at most 587520 (N = 65280: 9 slices of 65280)
+constexpr size_t kPartCap = (size_t)kCompatOnceMaxN / 256 * kCompatOnceMaxN;
+static_assert(kPartCap >= 589824, "the sliced plan's entries");
 constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 constexpr size_t kBlkRows = (kNoAllocMaxN + kBlock - 1) / kBlock;
 constexpr size_t kOffQ = 0;
@@ -35,7 +37,7 @@ constexpr size_t kOffBlk = align256(kOffApart + sizeof(float) * kPartCap);
 constexpr size_t kOffRdf = align256(kOffBlk + sizeof(double) * kBlkFields * kBlkRows);
 constexpr size_t kOffTab = align256(kOffRdf + sizeof(unsigned long long) * 256);
 constexpr size_t kOffPressure = align256(kOffTab + sizeof(float) * 257);
-constexpr size_t kScratchBytes = align256(kOffPressure + sizeof(float));  // 12.3 MiB
+constexpr size_t kScratchBytes = align256(kOffPressure + sizeof(float));  // 81.5 MiB
 
 }  // namespace
 
@@ -90,11 +92,11 @@ int noalloc_forces(float* Pos, float* Force, float* host_pressure, int N, float 
   if (host_RDF && !(host_dr2 > 0.f))
     return fail(LJ_ERR_ARG, "calculateNForcesNoAlloc: RDF bin width must be positive");
   LJ_TRY(check_device());
-  const ForcePlan pl = make_force_plan(N, 0, 1);
+  const PairScalars ps = make_pair_scalars((double)host_L, Lperiodic != 0, 1., 1., true);
+  const ForcePlan pl = compat_plan(N, ps);
   if ((size_t)pl.S * pl.Npad > kPartCap)
     return fail(LJ_ERR_ARG, "calculateNForcesNoAlloc: %d x %d partial sums exceed the scratch",
                 pl.S, pl.Npad);
-  const PairScalars ps = make_pair_scalars((double)host_L, Lperiodic != 0, 1., 1., true);
   NoAllocDevice* d = nullptr;
   LJ_TRY(noalloc_device(&d));
   unsigned char* base = d->ptr;

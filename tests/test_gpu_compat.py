@@ -84,3 +84,59 @@ def test_excluded_pairs(N, periodic):
         err = force_errors(xyz(f), F64)
         assert err["global_rel"] <= 2e-6 and err["max_rel_floor"] <= 1e-5, err
     assert abs(pr - W / 3.0) <= 1e-5 * max(abs(W / 3.0), 1e-3)
+
+
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("N", [3072, 4097, 8192, 16385])
+def test_excluded_pairs_every_pair_once(N, periodic):
+    """The same where every pair is taken once (groups of 128: 3072 and 4097,
+    whose last group holds one particle; of 256: 8192 and 16385): pairs to leave
+    out inside a group, between two, and with the last particle; the RDF beside
+    it as the oracle's."""
+    rho = 0.3
+    L, pos, _ = perturbed_state(N, rho, 1.0, seed=80)
+    p = pos.reshape(N, 4).copy()
+    for a, b, d in ((0, 1, 0.0), (2, N - 1, 0.0), (70, 200, 5e-4), (300, 900, 0.0), (1000, 3000, 0.0)):
+        p[b] = p[a]
+        p[b, 0] += np.float32(d)
+    dr2 = ORC.orc_rdf_dr2(N)
+    arr = ljamd.CompatArrays(N)
+    f, pr, got = arr.calculate(p.reshape(-1), L, periodic, dr2)
+    arr.close()
+    F64, _, E, W = forces_fp64(p.reshape(-1), float(np.float32(L)), periodic, skip_r2=1e-6)
+    assert np.all(np.isfinite(f))
+    err = force_errors(xyz(f), F64)
+    assert err["global_rel"] <= 2e-6 and err["max_rel_floor"] <= 1e-5, err
+    assert abs(pr - W / 3.0) <= 1e-5 * max(abs(W / 3.0), 1e-3)
+    exp = rdf(p.reshape(-1), float(np.float32(L)), periodic, RDF_REF_GPU, 256, dr2=dr2)
+    assert np.array_equal(got.astype(np.int64), exp)
+
+
+@pytest.mark.parametrize("N", [600, 3500, 8192])
+def test_exact_ties(N):
+    """Particles on the two planes x = 0 and x = L/2: the x separation of a pair
+    is 0 or exactly half the box, so F_x comes from the ties alone, each particle
+    drawn towards the image that rounding half away from zero picks (+L/2 for the
+    lower x, MDSystem.cu:31-33).  All terms of a particle's sum have the same
+    sign, N/2 of them in float sums of at most 128: 1e-5 relative."""
+    L = 16.0
+    rng = np.random.default_rng(5)
+    p = np.zeros((N, 4), np.float32)
+    up = rng.permutation(N) % 2 == 1
+    p[:, 0] = np.where(up, L / 2, 0.0)
+    k = int(np.ceil(np.sqrt(N)))
+    g = rng.permutation(k * k)[:N]
+    p[:, 1] = (g // k + 0.5 + 0.3 * rng.uniform(-1, 1, N)) * (L / k)
+    p[:, 2] = (g % k + 0.5 + 0.3 * rng.uniform(-1, 1, N)) * (L / k)
+    arr = ljamd.CompatArrays(N)
+    f, _, _ = arr.calculate(p.reshape(-1), L, True, 0.1)
+    arr.close()
+    q = p.astype(np.float64)
+    F = np.zeros(N)
+    for i in range(N):
+        o = up != up[i]
+        d = q[i, 1:3] - q[o, 1:3]
+        d -= L * np.round(d / L)
+        r2 = (L / 2) ** 2 + np.sum(d * d, axis=1)
+        F[i] = (1.0 if not up[i] else -1.0) * np.sum(24.0 * (2.0 / r2 ** 7 - 1.0 / r2 ** 4)) * (L / 2)
+    assert np.max(np.abs(f.reshape(N, 4)[:, 0] - F) / np.abs(F)) <= 1e-5
