@@ -2,6 +2,7 @@
 // MDSystem.cu entry points), context API and device-pointer API.
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -443,10 +444,7 @@ int lj_destroy(lj_ctx* c)
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   drop_graph(c);
   adj_free(c);
-  dev_free(c->pos);
-  dev_free(c->vel);
-  dev_free(c->force);
-  dev_free(c->tF);
+  dev_free(c->pos);  // with vel, force and tF
   dev_free(c->q);
   dev_free(c->q2);
   dev_free(c->fpart);
@@ -455,6 +453,7 @@ int lj_destroy(lj_ctx* c)
   dev_free(c->obs);
   dev_free(c->hist);
   dev_free(c->hist_base);
+  if (c->out) (void)hipHostFree(c->out);
   dev_free(c->ev);
   dev_free(c->rdf);
   dev_free(c->edges2);
@@ -531,10 +530,14 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
     c->stream = nullptr;
     A(fail(LJ_ERR_DEVICE, "hipStreamCreate failed"));
   }
-  A(dev_alloc(&c->pos, N));
-  A(dev_alloc(&c->vel, N));
-  A(dev_alloc(&c->force, N));
-  A(dev_alloc(&c->tF, N));
+  // one allocation for the state, each array at a multiple of 256 bytes
+  const size_t pitch = ((size_t)N + 15) & ~(size_t)15;
+  A(dev_alloc(&c->pos, 4 * pitch));
+  if (rc == LJ_OK) {
+    c->vel = c->pos + pitch;
+    c->force = c->vel + pitch;
+    c->tF = c->force + pitch;
+  }
   A(dev_alloc(&c->q, N));
   if (c->small_T) A(dev_alloc(&c->q2, N));
   A(dev_alloc(&c->fpart, npart));
@@ -561,6 +564,9 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
   A(dev_alloc(&c->blk, 2 * blk_rows(c) * kBlkFields));
   A(dev_alloc(&c->obs, 1));
   A(dev_alloc(&c->hist_base, 1));
+  if (rc == LJ_OK && hipHostMalloc(reinterpret_cast<void**>(&c->out), sizeof(*c->out) * kOutWords,
+                                   hipHostMallocDefault) != hipSuccess)
+    A(fail(LJ_ERR_ALLOC, "lj_create: pinned memory"));
   A(dev_alloc(&c->ev, 2));
   if (is_fp64(c)) {
     A(dev_alloc(&c->xd, N));
@@ -578,26 +584,25 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
   if (rc == LJ_OK && hipEventCreate(&c->e1) != hipSuccess) A(fail(LJ_ERR_DEVICE, "hipEventCreate"));
   if (rc == LJ_OK) A(ensure_hist(c, 1024));
   if (rc == LJ_OK) {
-    // zero state: host buffers copied so that no memset node ever enters a
-    // graph, on the context's stream (see the item table above)
-    std::vector<float> z((size_t)4 * N, 0.f);
-    lj_obs o{};
-    const size_t bytes = sizeof(float) * 4 * (size_t)N;
-    hipStream_t st = c->stream;
-    const auto up = [st](void* d, const void* h, size_t n) {
-      return hipMemcpyAsync(d, h, n, hipMemcpyHostToDevice, st) == hipSuccess;
+    // zero state, by a kernel on the context's stream (see the item table above)
+    const auto zero = [&](void* d, size_t bytes) {
+      for (size_t w = 0, n = bytes / 8; w < n && rc == LJ_OK; w += size_t(1) << 28)
+        if (launch_fill_u64(c->stream, static_cast<unsigned long long*>(d) + w,
+                            (int)std::min(n - w, size_t(1) << 28)) != hipSuccess)
+          A(fail(LJ_ERR_DEVICE, "initial state"));
     };
-    if (!up(c->pos, z.data(), bytes) || !up(c->vel, z.data(), bytes) ||
-        !up(c->force, z.data(), bytes) || !up(c->tF, z.data(), bytes) ||
-        !up(c->obs, &o, sizeof(o)) || hipStreamSynchronize(st) != hipSuccess)
-      A(fail(LJ_ERR_DEVICE, "initial upload failed"));
-    if (rc == LJ_OK && is_fp64(c)) {
-      std::vector<double> zd((size_t)4 * N, 0.);
+    static_assert(sizeof(lj_obs) % 8 == 0, "filled by words");
+    zero(c->pos, 4 * pitch * sizeof(float4));
+    zero(c->obs, sizeof(lj_obs));
+    if (is_fp64(c)) {
       const size_t db = sizeof(double) * 4 * (size_t)N;
-      if (!up(c->xd, zd.data(), db) || !up(c->vd, zd.data(), db) || !up(c->fd, zd.data(), db) ||
-          !up(c->tfd, zd.data(), db) || hipStreamSynchronize(st) != hipSuccess)
-        A(fail(LJ_ERR_DEVICE, "initial upload failed"));
+      zero(c->xd, db);
+      zero(c->vd, db);
+      zero(c->fd, db);
+      zero(c->tfd, db);
     }
+    if (rc == LJ_OK && hipStreamSynchronize(c->stream) != hipSuccess)
+      A(fail(LJ_ERR_DEVICE, "initial state"));
   }
   if (rc != LJ_OK) {
     std::string msg = g_err;
@@ -728,6 +733,7 @@ int lj_sample_initial_state_ex(lj_ctx* c, uint64_t seed, int velocities)
   LJ_TRY(lj_set_array(c, LJ_ARRAY_POS, p.data()));
   LJ_TRY(lj_set_array(c, LJ_ARRAY_VEL, v.data()));
   LJ_HIP(launch_reset_clock(c->stream, c->obs));
+  c->base_set = false;
   // MDSystem::Reinitialize: CalculateForces, CalculateParameters, reset averages (:101-113)
   LJ_TRY(lj_compute_forces(c, nullptr));
   LJ_TRY(lj_compute_parameters(c, nullptr));
@@ -743,12 +749,19 @@ int lj_integrate(lj_ctx* c, double dt, int nsteps, double* hist)
   LJ_TRY(ensure_hist(c, nsteps));
   LJ_TRY(ensure_graph(c, dt));
   hipStream_t st = c->stream;
-  LJ_HIP(launch_set_hist_base(st, c->obs, c->hist_base));
+  if (!c->base_set) LJ_HIP(launch_set_hist_base(st, c->obs, c->hist_base));
+  c->base_set = false;
   LJ_TRY(launch_steps(c, nsteps));
   c->rdf_step_n = c->smp_rdf == LJ_SAMPLE_RDF_LAST ? 1 : c->rdf_step_n + nsteps;
-  if (hist)
+  // short histories by the kernel that also sets the next call's base
+  const bool brief = hist && nsteps <= kOutWords / 5;
+  if (brief)
+    LJ_HIP(launch_results_out(st, c->hist, c->out, 5 * nsteps, nullptr, nullptr, c->obs, c->hist_base));
+  else if (hist)
     LJ_HIP(hipMemcpyAsync(hist, c->hist, sizeof(double) * 5 * nsteps, hipMemcpyDeviceToHost, st));
   LJ_HIP(hipStreamSynchronize(st));
+  if (brief) std::memcpy(hist, c->out, sizeof(double) * 5 * nsteps);
+  c->base_set = brief;
   return LJ_OK;
 }
 
@@ -760,6 +773,7 @@ int lj_integrate_async(lj_ctx* c, double dt, int nsteps)
   if (nsteps == 0) return LJ_OK;
   LJ_TRY(ensure_graph(c, dt));
   LJ_HIP(launch_set_hist_base(c->stream, c->obs, c->hist_base));
+  c->base_set = false;
   LJ_TRY(launch_steps(c, nsteps));
   c->rdf_step_n = c->smp_rdf == LJ_SAMPLE_RDF_LAST ? 1 : c->rdf_step_n + nsteps;
   return LJ_OK;
@@ -804,21 +818,27 @@ int prepare_rdf(lj_ctx* c, int rule, int nbins, float dr2, double rmax, int accu
   if (rule == LJ_RDF_REF_GPU) gpu_minimage_thresholds(c->L, a.thr);
   else cpu_minimage_thresholds(c->L, a.thr);
   a.est_scale = rule == LJ_RDF_RBINS ? (float)(nbins / rmax) : (float)(1.0 / dr2);
-  std::vector<float> e(nbins + 1);
-  rdf_bin_thresholds(rule, nbins, dr2, rmax, e.data());
-  a.end = rule == LJ_RDF_REF_GPU ? e[nbins - 1] : e[nbins];
-  LJ_TRY(attach_rdf_workspace(c, a));
-  if (nbins + 1 > c->edges_cap) {
+  // the binning's table stays on the device while calls ask for the same binning
+  if (!same || !c->edges_set) {
+    c->edges_set = false;
+    std::vector<float> e(nbins + 1);
+    rdf_bin_thresholds(rule, nbins, dr2, rmax, e.data());
+    if (nbins + 1 > c->edges_cap) {
+      LJ_HIP(hipStreamSynchronize(st));
+      dev_free(c->edges2);
+      c->edges_cap = 0;
+      LJ_TRY(dev_alloc(&c->edges2, nbins + 1));
+      c->edges_cap = nbins + 1;
+    }
+    // synchronous: the host table goes out of scope on return
+    LJ_HIP(hipMemcpyAsync(c->edges2, e.data(), sizeof(float) * (nbins + 1), hipMemcpyHostToDevice, st));
     LJ_HIP(hipStreamSynchronize(st));
-    dev_free(c->edges2);
-    c->edges_cap = 0;
-    LJ_TRY(dev_alloc(&c->edges2, nbins + 1));
-    c->edges_cap = nbins + 1;
+    c->edges_end = rule == LJ_RDF_REF_GPU ? e[nbins - 1] : e[nbins];
+    c->edges_set = true;
   }
-  // synchronous: the host table goes out of scope on return
-  LJ_HIP(hipMemcpyAsync(c->edges2, e.data(), sizeof(float) * (nbins + 1), hipMemcpyHostToDevice, st));
-  LJ_HIP(hipStreamSynchronize(st));
+  a.end = c->edges_end;
   a.tab = c->edges2;
+  LJ_TRY(attach_rdf_workspace(c, a));
   *out = a;
   return LJ_OK;
 }
@@ -835,21 +855,20 @@ int lj_rdf(lj_ctx* c, int rule, int nbins, float dr2, double rmax, uint64_t* cou
   LJ_TRY(prepare_rdf(c, rule, nbins, dr2, rmax, accumulate, "lj_rdf", &a));
   hipStream_t st = c->stream;
   LJ_HIP(launch_rdf(st, a));
-  if (rdf_uses_cells(a)) {
+  const unsigned* flagged = rdf_uses_cells(a) ? a.cells->result : nullptr;
+  LJ_HIP(launch_results_out(st, c->rdf, c->out, a.nbins, flagged));
+  LJ_HIP(hipStreamSynchronize(st));
+  if (flagged && c->out[a.nbins]) {
     // coordinates beyond [-L, 2 L): the cell-list pass counted nothing; the
     // all-pairs pass counts instead
-    unsigned bad = 0u;
-    LJ_HIP(hipMemcpyAsync(&bad, a.cells->result, sizeof(unsigned), hipMemcpyDeviceToHost, st));
+    LJ_HIP(hipMemsetAsync(a.cells->result, 0, sizeof(unsigned), st));
+    RdfArgs b = a;
+    b.cells = nullptr;
+    LJ_HIP(launch_rdf(st, b));
+    LJ_HIP(launch_results_out(st, c->rdf, c->out, a.nbins));
     LJ_HIP(hipStreamSynchronize(st));
-    if (bad) {
-      LJ_HIP(hipMemsetAsync(a.cells->result, 0, sizeof(unsigned), st));
-      RdfArgs b = a;
-      b.cells = nullptr;
-      LJ_HIP(launch_rdf(st, b));
-    }
   }
-  LJ_HIP(hipMemcpyAsync(counts, c->rdf, sizeof(uint64_t) * a.nbins, hipMemcpyDeviceToHost, st));
-  LJ_HIP(hipStreamSynchronize(st));
+  std::memcpy(counts, c->out, sizeof(uint64_t) * a.nbins);
   return LJ_OK;
 }
 
@@ -1062,6 +1081,7 @@ int lj_renormalize_to_energy(lj_ctx* c, double ust)
   o.K = Kdes;
   o.U = o.K + o.V;
   LJ_HIP(hipMemcpyAsync(c->obs, &o, sizeof(o), hipMemcpyHostToDevice, c->stream));
+  c->base_set = false;
   LJ_HIP(hipStreamSynchronize(c->stream));
   return LJ_OK;
 }
@@ -1216,6 +1236,8 @@ struct CompatResult {
   float pressure;
   unsigned flagged;  // the cell-list RDF pass counted nothing
 };
+static_assert(offsetof(CompatResult, pressure) == 2048 && offsetof(CompatResult, flagged) == 2052,
+              "the words of launch_results_out");
 
 struct CompatScratch {
   int device = -1;
@@ -1323,7 +1345,6 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
   LJ_HIP(launch_reduce_forces(st, pl, ps, s->fpart, s->apart, reinterpret_cast<float4*>(Force), s->blk));
   LJ_HIP(launch_finalize_forces(st, s->blk, (N + kBlock - 1) / kBlock, 1., nullptr, s->pressure));
   CompatResult& r = *s->host;
-  r.flagged = 0;
   RdfArgs a{};
   if (host_RDF) {
     LJ_HIP(launch_fill_u64(st, s->rdf, 256));
@@ -1367,11 +1388,9 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
       a.rows_cap = s->rows_cap;
     }
     LJ_HIP(launch_rdf(st, a));
-    if (rdf_uses_cells(a))
-      LJ_HIP(hipMemcpyAsync(&r.flagged, a.cells->result, sizeof(unsigned), hipMemcpyDeviceToHost, st));
-    LJ_HIP(hipMemcpyAsync(r.rdf, s->rdf, sizeof(r.rdf), hipMemcpyDeviceToHost, st));
   }
-  LJ_HIP(hipMemcpyAsync(&r.pressure, s->pressure, sizeof(float), hipMemcpyDeviceToHost, st));
+  LJ_HIP(launch_results_out(st, s->rdf, &r, 256, reinterpret_cast<const unsigned*>(s->pressure),
+                            host_RDF && rdf_uses_cells(a) ? a.cells->result : nullptr));
   LJ_HIP(hipStreamSynchronize(st));
   if (host_RDF && r.flagged) {
     // a coordinate beyond [-L, 2 L): the all-pairs pass counts instead

@@ -33,6 +33,9 @@ struct lj_ctx {
   double* hist = nullptr;
   int hist_cap = 0;
   int64_t* hist_base = nullptr;
+  bool base_set = false;  // *hist_base is the current step count
+  // pinned, kOutWords: a call's history rows or RDF counts on their way out
+  unsigned long long* out = nullptr;
   double* ev = nullptr;
   unsigned long long* rdf = nullptr;
   int rdf_cap = 0;
@@ -89,6 +92,8 @@ struct lj_ctx {
   int64_t rdf_step_n = 0;              // steps the step histogram holds
   lj::RdfCellsWs rdf_cells;            // workspace of the cell-list RDF pass
   unsigned* rdf_rows = nullptr;        // and of the all-pairs pass
+  bool edges_set = false;              // edges2 holds the table of rdf_rule .. rdf_rmax
+  double edges_end = 0.;               // the counted range's end in it
   size_t rdf_rows_cap = 0;
   bool sampling() const { return smp_rdf != LJ_SAMPLE_RDF_OFF || smp_fl != 0; }
 };
@@ -109,6 +114,7 @@ void adj_free(lj_ctx* c);
 inline bool is_fp64(const lj_ctx* c) { return c->cfg.precision == LJ_PREC_FP64; }
 // the double state array of LJ_ARRAY_POS / VEL / FORCE (LJ_PREC_FP64 contexts)
 double4* state64(lj_ctx* c, int type);
+constexpr int kOutWords = 8192;
 // plan of the force pass that fills fpart/apart
 inline const ForcePlan& fplan(const lj_ctx* c) { return c->plan3.n3 ? c->plan3 : c->plan; }
 // gives an RDF pass of the context the workspace of the cell-list pass where

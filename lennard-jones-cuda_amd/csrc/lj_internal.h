@@ -184,6 +184,11 @@ hipError_t launch_small_tvn(hipStream_t st, int T, const StepArgs& a, float C1, 
 // observables of the current state (no time advance): K from vel, V/W from blk
 hipError_t launch_params(hipStream_t st, const StepArgs& a, int include_force_terms);
 hipError_t launch_set_hist_base(hipStream_t st, lj_obs* obs, int64_t* base);
+// n 8-byte words of src to out (pinned host memory), word n = *lo | *hi << 32
+// where either is given, *base = obs->step where base is
+hipError_t launch_results_out(hipStream_t st, const void* src, void* out, int n,
+                              const unsigned* lo = nullptr, const unsigned* hi = nullptr,
+                              const lj_obs* obs = nullptr, int64_t* base = nullptr);
 // velocity rescale by sqrt(T0/Tkin) or by a host factor (factor > 0)
 hipError_t launch_kinetic_partials(hipStream_t st, const float4* vel, int N, double* blk);
 hipError_t launch_scale_velocities(hipStream_t st, float4* vel, int N, const double* blk,

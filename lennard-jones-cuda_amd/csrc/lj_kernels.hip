@@ -405,6 +405,24 @@ __global__ __launch_bounds__(kBlock) void k_params(StepArgs a, int nblk, int for
 
 __global__ void k_set_hist_base(lj_obs* obs, int64_t* base) { *base = obs->step; }
 
+// a call's results on their way out, written to pinned host memory: n words of
+// src, then one of *lo and *hi (0 where null); the base of the next call's
+// history rows with it.  (A copy to pageable memory behind the call's last kernel
+// took 8 us longer, one to pinned memory 4.)
+__global__ __launch_bounds__(kBlock) void k_results_out(const unsigned long long* __restrict__ src,
+                                                        unsigned long long* __restrict__ out, int n,
+                                                        const unsigned* __restrict__ lo,
+                                                        const unsigned* __restrict__ hi,
+                                                        const lj_obs* __restrict__ obs,
+                                                        int64_t* __restrict__ base)
+{
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) out[i] = src[i];
+  if (i != 0) return;
+  if (lo || hi) out[n] = (unsigned long long)(hi ? *hi : 0u) << 32 | (lo ? *lo : 0u);
+  if (base) *base = obs->step;
+}
+
 __global__ __launch_bounds__(kBlock) void k_kinetic_partials(const float4* __restrict__ vel, int N,
                                                              double* __restrict__ blk)
 {
@@ -1236,6 +1254,15 @@ hipError_t launch_params(hipStream_t st, const StepArgs& a, int include_force_te
 {
   hipLaunchKernelGGL(k_params, dim3(1), dim3(kBlock), 0, st, a, nblocks(a.N),
                      include_force_terms);
+  return hipGetLastError();
+}
+
+hipError_t launch_results_out(hipStream_t st, const void* src, void* out, int n, const unsigned* lo,
+                              const unsigned* hi, const lj_obs* obs, int64_t* base)
+{
+  hipLaunchKernelGGL(k_results_out, dim3(std::max(1, nblocks(n))), dim3(kBlock), 0, st,
+                     static_cast<const unsigned long long*>(src),
+                     static_cast<unsigned long long*>(out), n, lo, hi, obs, base);
   return hipGetLastError();
 }
 

@@ -203,3 +203,36 @@ def test_compensated_trajectory_vs_reference(N, canon, bc, nsteps, tolU):
     finally:
         g.close()
 
+
+
+def test_history_rows_over_mixed_calls():
+    """The history rows of a call start at its own first step whatever came
+    before it: a call with few rows (they leave with the kernel that notes the
+    step count for the next call), one without a history, one with more rows than
+    that kernel takes, a restart.  Bit-identical to one run's rows."""
+    N, rho, T0 = 128, 0.5, 1.0
+    dt = 0.002
+    calls = (3, 1, 2, 1700, 5)
+    with ljamd.LJSystem(N, rho, T0, seed=9) as s:
+        whole = s.Integrate(dt, sum(calls))
+    with ljamd.LJSystem(N, rho, T0, seed=9) as s:
+        at = 0
+        for k, n in enumerate(calls):
+            if k == 1:
+                s.integrate_async(dt, n)
+            else:
+                assert np.array_equal(s.Integrate(dt, n), whole[at:at + n]), k
+            at += n
+        s.sample_initial_state(9)
+        assert np.array_equal(s.Integrate(dt, 4), whole[:4])
+
+
+def test_rdf_table_follows_the_binning():
+    """Calls that alternate between binnings each count with their own table."""
+    N, rho = 500, 0.4
+    with ljamd.LJSystem(N, rho, 1.0, seed=3) as s:
+        s.Integrate(0.004, 20)
+        first = [s.rdf(ljamd.RDF_RBINS, 100, rmax=r) for r in (2.0, 3.0)]
+        for r, e in zip((2.0, 3.0, 3.0, 2.0), (first[0], first[1], first[1], first[0])):
+            assert np.array_equal(s.rdf(ljamd.RDF_RBINS, 100, rmax=r), e)
+    assert not np.array_equal(*first)
