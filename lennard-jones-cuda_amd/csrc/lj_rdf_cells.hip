@@ -727,7 +727,7 @@ namespace {
 
 // the fewest particles for which the cell lists are taken: below, their four
 // launches cost more than the all-pairs pass (GPU rule, rho* = 0.85: N = 6000 40
-// against 28 us, N = 8000 36 against 38).  The per-step sampling takes them at any
+// against 29 us, N = 8000 36 against 37).  The per-step sampling takes them at any
 // N: there a coordinate beyond their span is reported instead of counted.
 constexpr int kCellsFromN = 8192;
 // the average number of particles that a cell holds at least: a workgroup per
