@@ -1335,6 +1335,7 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
   CompatScratch* s = nullptr;
   ForcePlan pl = compat_plan(N, ps);
   if (compat_scratch(N, pl, &s) != LJ_OK) {  // no room for its partial sums
+    (void)hipGetLastError();                 // else the next launch reports it
     pl = make_force_plan(N, 0, 1);
     LJ_TRY(compat_scratch(N, pl, &s));
   }
@@ -1373,16 +1374,18 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
     const int nc = rdf_cells_grid(a, &reach);
     if (nc > 0) {
       bool grown = false;
-      LJ_TRY(rdf_cells_ensure(s->cells, N, nc * nc * nc, a.nbins, st, &grown));
-      a.cells = &s->cells;
+      if (rdf_cells_ensure(s->cells, N, nc * nc * nc, a.nbins, st, &grown) == LJ_OK)
+        a.cells = &s->cells;
+      else
+        (void)hipGetLastError();  // without the lists: all pairs
     } else {
       const size_t need = (size_t)rdf_workgroups(a) * a.nbins;
       if (need > s->rows_cap) {
         LJ_HIP(hipStreamSynchronize(st));
         dev_free(s->rows);
         s->rows_cap = 0;
-        LJ_TRY(dev_alloc(&s->rows, need));
-        s->rows_cap = need;
+        if (dev_alloc(&s->rows, need) == LJ_OK) s->rows_cap = need;
+        else (void)hipGetLastError();  // without rows: atomics
       }
       a.rows = s->rows;
       a.rows_cap = s->rows_cap;

@@ -130,14 +130,14 @@ inline int attach_rdf_workspace(lj_ctx* c, RdfArgs& a)
     if (need > c->rdf_rows_cap) {
       LJ_HIP(hipStreamSynchronize(c->stream));
       // the steps that sample the RDF, captured or not, hold the old rows
-      drop_graph(c);
       const bool sampled = c->smp_args.rows != nullptr;
+      if (sampled) drop_graph(c);
       dev_free(c->rdf_rows);
       c->rdf_rows_cap = c->smp_args.rows_cap = 0;
-      c->smp_args.rows = nullptr;  // (atomics instead, should the growth fail)
-      LJ_TRY(dev_alloc(&c->rdf_rows, need));
-      c->rdf_rows_cap = need;
-      if (sampled) {
+      c->smp_args.rows = nullptr;
+      if (dev_alloc(&c->rdf_rows, need) == LJ_OK) c->rdf_rows_cap = need;
+      else (void)hipGetLastError();  // without rows: atomics
+      if (sampled && c->rdf_rows) {
         c->smp_args.rows = c->rdf_rows;
         c->smp_args.rows_cap = need;
       }
