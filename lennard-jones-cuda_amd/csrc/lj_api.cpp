@@ -1379,7 +1379,8 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
       else
         (void)hipGetLastError();  // without the lists: all pairs
     } else {
-      const size_t need = (size_t)rdf_workgroups(a) * a.nbins;
+      size_t need = 0;
+      (void)rdf_workgroups(a, &need);
       if (need > s->rows_cap) {
         LJ_HIP(hipStreamSynchronize(st));
         dev_free(s->rows);

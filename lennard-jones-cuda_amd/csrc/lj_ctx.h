@@ -126,7 +126,8 @@ inline int attach_rdf_workspace(lj_ctx* c, RdfArgs& a)
   int reach = 1;
   const int nc = rdf_cells_grid(a, &reach);
   if (nc <= 0) {
-    const size_t need = (size_t)rdf_workgroups(a) * a.nbins;
+    size_t need = 0;
+    (void)rdf_workgroups(a, &need);
     if (need > c->rdf_rows_cap) {
       LJ_HIP(hipStreamSynchronize(c->stream));
       // the steps that sample the RDF, captured or not, hold the old rows

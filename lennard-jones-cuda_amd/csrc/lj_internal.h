@@ -256,8 +256,10 @@ struct RdfArgs {
   int sampling;             // the per-step sampling's pass (its own result word)
 };
 hipError_t launch_rdf(hipStream_t st, const RdfArgs& a);
-// workgroups of the all-pairs pass with at most 1024 bins (0: more bins)
-int rdf_workgroups(const RdfArgs& a);
+// workgroups of the all-pairs pass with at most 1024 bins (0: more bins); rows: the
+// words its histogram rows take, 0 where it runs without (more bins, or so many
+// workgroups that their atomics do not matter)
+int rdf_workgroups(const RdfArgs& a, size_t* rows);
 hipError_t launch_rdf_cells(hipStream_t st, const RdfArgs& a);
 // cells per axis (0: none) and reach of the cell-list pass for these
 // arguments, periodic or hard-wall

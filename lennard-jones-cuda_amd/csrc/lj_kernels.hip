@@ -1325,16 +1325,24 @@ size_t rdf_lds(const RdfArgs& a)
 // workgroups 21 us, 2048 33), and no more than eight times what the LDS lets 256 CUs
 // hold, six each at most, which bounds the rows.  That many because the runs differ
 // in pairs in range: one run per resident workgroup took 300 us at N = 30000, four
-// 271, eight 272; at N = 70000 1513, 1320 and 1282.
-int rdf_workgroups(const RdfArgs& a)
+// 271, eight 272; at N = 70000 1513, 1320 and 1282.  More than that only where a run
+// would exceed kRdfRunUnits (N above about 7e6): a workgroup counts its pairs in
+// 32-bit words.
+constexpr long kRdfRunUnits = 1L << 18;
+static_assert(kRdfRunUnits * kRdfUnit * kBlock < 1L << 32, "a workgroup's counts");
+
+int rdf_workgroups(const RdfArgs& a, size_t* rows)
 {
+  if (rows) *rows = 0;
   if (a.nbins > kRdfWaveCopy) return 0;
   const size_t lds = rdf_lds(a) + (a.periodic ? kBlock * 32 + 64 : 0);
-  const long fit = 256 * std::min(6L, 163840 / (long)lds);
+  const long fit = 8 * 256 * std::min(6L, 163840 / (long)lds);
   const long nu = (a.N + kRdfUnit - 1) / kRdfUnit, ng = nblocks(a.N);
   const long units = ng * nu - kGroupUnits / 2 * ng * (ng - 1);
-  const long n = std::max(std::min(units, 768L), units / 4);
-  return (int)std::max(1L, std::min(n, 8 * fit));
+  const long n = std::max(1L, std::min(std::max(std::min(units, 768L), units / 4), fit));
+  const long nwg = std::max(n, (units + kRdfRunUnits - 1) / kRdfRunUnits);
+  if (rows && nwg <= fit) *rows = (size_t)nwg * a.nbins;
+  return (int)nwg;
 }
 
 hipError_t launch_rdf(hipStream_t st, const RdfArgs& a)
@@ -1359,8 +1367,9 @@ hipError_t launch_rdf(hipStream_t st, const RdfArgs& a)
     return hipGetLastError();
   }
   if (rdf_uses_cells(a)) return launch_rdf_cells(st, a);
-  const int nwg = rdf_workgroups(a);
-  unsigned* rows = a.rows && (size_t)nwg * a.nbins <= a.rows_cap ? a.rows : nullptr;
+  size_t need = 0;
+  const int nwg = rdf_workgroups(a, &need);
+  unsigned* rows = a.rows && need > 0 && need <= a.rows_cap ? a.rows : nullptr;
   const size_t lds = rdf_lds(a);
   if (a.periodic) {
     // the far-pair pass where the counted range holds under 30% of the box
