@@ -118,43 +118,45 @@ constexpr int kOutWords = 8192;
 // plan of the force pass that fills fpart/apart
 inline const ForcePlan& fplan(const lj_ctx* c) { return c->plan3.n3 ? c->plan3 : c->plan; }
 // gives an RDF pass of the context the workspace of the cell-list pass where
-// that pass applies, else of the all-pairs pass, grown first
+// that pass applies and finds room, else of the all-pairs pass, grown first
 inline int attach_rdf_workspace(lj_ctx* c, RdfArgs& a)
 {
   a.cells = nullptr;
   a.rows = nullptr;
   int reach = 1;
   const int nc = rdf_cells_grid(a, &reach);
-  if (nc <= 0) {
-    size_t need = 0;
-    (void)rdf_workgroups(a, &need);
-    if (need > c->rdf_rows_cap) {
-      LJ_HIP(hipStreamSynchronize(c->stream));
-      // the steps that sample the RDF, captured or not, hold the old rows
-      const bool sampled = c->smp_args.rows != nullptr;
-      if (sampled) drop_graph(c);
-      dev_free(c->rdf_rows);
-      c->rdf_rows_cap = c->smp_args.rows_cap = 0;
-      c->smp_args.rows = nullptr;
-      if (dev_alloc(&c->rdf_rows, need) == LJ_OK) c->rdf_rows_cap = need;
-      else (void)hipGetLastError();  // without rows: atomics
-      if (sampled && c->rdf_rows) {
-        c->smp_args.rows = c->rdf_rows;
-        c->smp_args.rows_cap = need;
-      }
+  if (nc > 0) {
+    bool grown = false;
+    const int rc = rdf_cells_ensure(c->rdf_cells, a.N, nc * nc * nc, a.nbins, c->stream, &grown);
+    // captured steps that sample the RDF hold the old arrays' addresses (lj_rdf and
+    // the per-step sampling share the workspace); they are captured again on the
+    // next run, without the lists where those found no room
+    if (grown) drop_graph(c);
+    if (rc == LJ_OK) {
+      a.cells = &c->rdf_cells;
+      return LJ_OK;
     }
-    a.rows = c->rdf_rows;
-    a.rows_cap = c->rdf_rows_cap;
-    return LJ_OK;
+    (void)hipGetLastError();  // else the next launch reports it
   }
-  bool grown = false;
-  const int rc = rdf_cells_ensure(c->rdf_cells, a.N, nc * nc * nc, a.nbins, c->stream, &grown);
-  if (rc != LJ_OK) return rc;
-  // reallocated: captured steps that sample the RDF hold the old arrays'
-  // addresses (lj_rdf and the per-step sampling share the workspace); they
-  // are captured again on the next run
-  if (grown) drop_graph(c);
-  a.cells = &c->rdf_cells;
+  size_t need = 0;
+  (void)rdf_workgroups(a, &need);
+  if (need > c->rdf_rows_cap) {
+    LJ_HIP(hipStreamSynchronize(c->stream));
+    // the steps that sample the RDF, captured or not, hold the old rows
+    const bool sampled = c->smp_args.rows != nullptr;
+    if (sampled) drop_graph(c);
+    dev_free(c->rdf_rows);
+    c->rdf_rows_cap = c->smp_args.rows_cap = 0;
+    c->smp_args.rows = nullptr;
+    if (dev_alloc(&c->rdf_rows, need) == LJ_OK) c->rdf_rows_cap = need;
+    else (void)hipGetLastError();  // without rows: atomics
+    if (sampled && c->rdf_rows) {
+      c->smp_args.rows = c->rdf_rows;
+      c->smp_args.rows_cap = need;
+    }
+  }
+  a.rows = c->rdf_rows;
+  a.rows_cap = c->rdf_rows_cap;
   return LJ_OK;
 }
 }  // namespace lj

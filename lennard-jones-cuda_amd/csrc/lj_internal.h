@@ -232,7 +232,8 @@ struct RdfCellsWs {
 // cells per axis for a periodic range ending at r^2 = end, or 0 (fewer than 3)
 int rdf_cells_per_axis(double L, double end);
 // LJ_OK or a status; st: the owner's stream (its work is waited for, and the
-// new arrays are cleared on it); *grown: whether the arrays were reallocated
+// new arrays are cleared on it); *grown: whether the old arrays were freed, also
+// where the new ones found no room (the workspace is then empty)
 int rdf_cells_ensure(RdfCellsWs& w, int N, int ncell, int nbins, hipStream_t st, bool* grown);
 void rdf_cells_free(RdfCellsWs& w);
 

@@ -777,25 +777,33 @@ int rdf_cells_ensure(RdfCellsWs& w, int N, int ncell, int nbins, hipStream_t st,
   // grown to at least the old capacities, so that alternating layouts settle
   const int cn = std::max(N, w.cap_n), cc = std::max(ncell, w.cap_cells), cb = std::max(nbins, w.cap_bins);
   rdf_cells_free(w);
-  LJ_TRY(dev_alloc(&w.count, cc));
-  LJ_TRY(dev_alloc(&w.start, (size_t)cc + 1));
-  LJ_TRY(dev_alloc(&w.cellof, cn));
-  LJ_TRY(dev_alloc(&w.rank, cn));
-  LJ_TRY(dev_alloc(&w.sorted, cn));
-  LJ_TRY(dev_alloc(&w.reps, (size_t)kRdfReps * cb));
-  LJ_TRY(dev_alloc(&w.other, kRdfReps));
-  LJ_TRY(dev_alloc(&w.flag, 3));
-  w.result = w.flag + 1;
-  w.result_step = w.flag + 2;
-  LJ_TRY(dev_alloc(&w.bcnt, kCellScanMax));
+  const auto fill = [&]() -> int {
+    LJ_TRY(dev_alloc(&w.count, cc));
+    LJ_TRY(dev_alloc(&w.start, (size_t)cc + 1));
+    LJ_TRY(dev_alloc(&w.cellof, cn));
+    LJ_TRY(dev_alloc(&w.rank, cn));
+    LJ_TRY(dev_alloc(&w.sorted, cn));
+    LJ_TRY(dev_alloc(&w.reps, (size_t)kRdfReps * cb));
+    LJ_TRY(dev_alloc(&w.other, kRdfReps));
+    LJ_TRY(dev_alloc(&w.flag, 3));
+    w.result = w.flag + 1;
+    w.result_step = w.flag + 2;
+    LJ_TRY(dev_alloc(&w.bcnt, kCellScanMax));
+    // the counts, replicas and flags start at zero; the passes clear them after use
+    if (hipMemsetAsync(w.count, 0, sizeof(int) * cc, st) != hipSuccess ||
+        hipMemsetAsync(w.reps, 0, sizeof(unsigned) * kRdfReps * cb, st) != hipSuccess ||
+        hipMemsetAsync(w.other, 0, sizeof(unsigned long long) * kRdfReps, st) != hipSuccess ||
+        hipMemsetAsync(w.flag, 0, sizeof(unsigned) * 3, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess)
+      return fail(LJ_ERR_DEVICE, "rdf_cells_ensure: clearing the workspace failed");
+    return LJ_OK;
+  };
+  const int rc = fill();
+  if (rc != LJ_OK) {  // nothing is held: rdf_uses_cells says no
+    rdf_cells_free(w);
+    return rc;
+  }
   w.cap_m = kCellScanMax;
-  // the counts, replicas and flags start at zero; the passes clear them after use
-  if (hipMemsetAsync(w.count, 0, sizeof(int) * cc, st) != hipSuccess ||
-      hipMemsetAsync(w.reps, 0, sizeof(unsigned) * kRdfReps * cb, st) != hipSuccess ||
-      hipMemsetAsync(w.other, 0, sizeof(unsigned long long) * kRdfReps, st) != hipSuccess ||
-      hipMemsetAsync(w.flag, 0, sizeof(unsigned) * 3, st) != hipSuccess ||
-      hipStreamSynchronize(st) != hipSuccess)
-    return fail(LJ_ERR_DEVICE, "rdf_cells_ensure: clearing the workspace failed");
   w.cap_n = cn;
   w.cap_cells = cc;
   w.cap_bins = cb;

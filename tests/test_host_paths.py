@@ -33,3 +33,41 @@ for N in [1, 255, 257, 400, 16384, 70000, 131072, 1000003, 10400000, 15000001, (
         assert grid[0] <= 8 * 256 * 6, (N, grid)
     s.close()
 """, env={"LJ_RDF_CELLS": "0"})
+
+
+@pytest.mark.parametrize("refused", range(9))
+def test_rdf_cell_lists_without_room(so, refused):
+    """Steps that sample the RDF through the cell lists are captured with the lists'
+    addresses.  A later lj_rdf that grows the lists frees them first: the captured
+    steps are dropped also where one of the new arrays finds no room, nothing
+    half-allocated stays, and both passes go on over all pairs."""
+    hip_stub.run(so, f"""
+s = ljamd.LJSystem(16384, 0.85, 1.0)
+s.set_step_sampling(ljamd.SAMPLE_RDF_SUM, rdf_rule=ljamd.RDF_REF_GPU, rdf_nbins=256)
+s.rdf(ljamd.RDF_RBINS, 1000)  # all pairs: the histogram and table of 1000 bins
+s.Integrate(0.005, 3)
+dr2 = L.lib().lj_rdf_dr2_default(16384) * 256 / 1000
+assert any("k_rdf_cells" in n for n, _ in kernels())
+held, captured = stub.stub_live(), stub.stub_instantiated()
+stub.stub_fail_in({refused})
+try:
+    s.rdf(ljamd.RDF_REF_GPU, 1000, dr2)
+finally:
+    stub.stub_fail_in(-1)
+    # the captured steps are gone before anything else can run them
+    assert stub.stub_graphs() == 0, "captured steps hold freed lists"
+assert stub.stub_refused() > 0
+names = [n for n, _ in kernels()]
+assert any("k_rdf_fx" in n for n in names) and not any("k_rdf_cells" in n for n in names)
+assert stub.stub_live() < held
+s.Integrate(0.005, 3)
+assert stub.stub_instantiated() > captured
+names = [n for n, _ in kernels()]
+assert any("k_rdf_fx" in n for n in names) and not any("k_rdf_cells" in n for n in names)
+s.step_rdf_counts()
+# room again: the next pass takes the lists
+s.rdf(ljamd.RDF_REF_GPU, 1000, dr2)
+assert any("k_rdf_cells" in n for n, _ in kernels())
+s.close()
+assert stub.stub_live() == 0
+""")
