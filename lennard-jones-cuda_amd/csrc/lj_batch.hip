@@ -374,13 +374,13 @@ __global__ __launch_bounds__(kBlock) void k_batch_finalize(BatchArgs a, int adva
 
 // ---- one-launch steps (lj_small.h): the workgroup that computes the whole
 // force on kBatchTile particles of a box also runs their integrator.  FIN: the
-// first nboxes workgroups finalise the run's previous step.  They serve every
-// batch whose tuning was not set: an ensemble of a few small boxes had one wave
-// per 64 particles and slice, each meeting up to 512 j one after another (16
-// boxes of 400: 131 us per EVN step, 9.4 us here; 64 of 1000: 173 / 53; 100 of
-// 3000: 534 / 462; the 512-box ensemble 1542 / 1530), which is why the launch is
-// bound by the pairs' issue slots only from about 1e8 pairs on.  Tiles of 16:
-// 8 and 4 re-read the box for fewer pairs each (16 of 400: 11.8 and 16.3). ----
+// first nboxes workgroups finalise the run's previous step.  They serve the batches
+// whose tuning was not set (small_steps says up to which size): an ensemble of a few
+// small boxes had one wave per 64 particles and slice, each meeting up to 512 j one
+// after another (EVN steps, us, before / here: 16 boxes of 400 131 / 9.0, 64 of 1000
+// 173 / 55, 64 of 3000 397 / 293, 8 of 10,000 490 / 362).  From about 1e8 pairs on the
+// launch is bound by the pairs' issue slots.  Tiles of 16: 8 and 4 re-read the box
+// for fewer pairs each (16 of 400: 11.8 and 16.3). ----
 
 template <bool PERIODIC, bool DRIFT, bool FIN>
 __global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(8))) void

@@ -37,10 +37,11 @@ struct lj_batch {
   float* apart = nullptr;
   size_t part_cap = 0;
   double* blk = nullptr;
-  // one-launch steps (until a tuning is set): the other coordinate buffer, the
-  // tiles, the boxes with the tiles' rows, and two buffers of block rows that
+  // one-launch steps (small; until a tuning is set): the other coordinate buffer,
+  // the tiles, the boxes with the tiles' rows, and two buffers of block rows that
   // the steps alternate between
   bool tuned = false;
+  bool small = false;
   uint4* q2 = nullptr;
   BoxParam* box_s = nullptr;
   int2* tiles = nullptr;
@@ -145,10 +146,27 @@ BatchArgs small_args(lj_batch* b, double dt, int par)
   return a;
 }
 
+// Whether an untuned batch takes the one-launch step.  A tile costs it a workgroup
+// of 1024 threads, 8.7e-3 us however few particles its box has; the four launches
+// of the default tiling cost 105 to 145 us a step and then less per tile: 4.4e-3 us
+// up to 512 particles a box, 7.5e-3 (one launch: 11.8e-3) at 1000, 14.2e-3 (16.3e-3) at
+// 2000.  EVN steps, us, one launch / tiling: 327 boxes of 200 41 / 130, 1310 154 / 186,
+// 2621 300 / 261, 5242 594 / 407; 655 of 400 157 / 193, 1310 308 / 268; 262 of 1000
+// 202 / 262, 524 393 / 390, 1048 778 / 640; 262 of 2000 539 / 617, 524 1068 / 1071; 131 of
+// 4000 1005 / 1057; one of 100,000 4388 / 4397.  So the line lies at 24,576 tiles of
+// boxes up to 512 particles, 32,768 up to 1200 and 49,152 above.
+bool small_steps(const std::vector<int>& N)
+{
+  long units = 0;
+  for (int n : N) units += (long)((n + kBatchTile - 1) / kBatchTile) * (n <= 512 ? 4 : n <= 1200 ? 3 : 2);
+  return units <= 4 * 24576;
+}
+
 // tables of the one-launch steps, from the boxes' parameters
 int build_small(lj_batch* b, const std::vector<BoxParam>& bp)
 {
-  if (b->tuned) return LJ_OK;
+  b->small = !b->tuned && small_steps(b->N);
+  if (!b->small) return LJ_OK;
   const int T = kBatchTile;
   std::vector<BoxParam> bs = bp;
   std::vector<int2> tiles;
@@ -287,7 +305,7 @@ int build_tables(lj_batch* b)
 int enqueue_batch_step(lj_batch* b, hipStream_t st, double dt, bool first = true, bool last = true,
                        int par = 0)
 {
-  if (!b->tuned) {
+  if (b->small) {
     const BatchArgs a = small_args(b, dt, par), prev = small_args(b, dt, par ^ 1);
     if (first) LJ_HIP(launch_batch_drift(st, a));
     if (b->canonical == LJ_EVN) {

@@ -71,3 +71,25 @@ assert any("k_rdf_cells" in n for n, _ in kernels())
 s.close()
 assert stub.stub_live() == 0
 """)
+
+
+@pytest.mark.parametrize("boxes,N,small", [(16, 400, 1), (1310, 200, 1), (2621, 200, 0), (5242, 200, 0),
+                                           (768, 512, 1), (769, 512, 0), (262, 1000, 1),
+                                           (524, 1000, 0), (262, 2000, 1), (131, 4000, 1),
+                                           (8, 10000, 1), (1, 100000, 1)])
+def test_untuned_batch_route(so, boxes, N, small):
+    """Untuned batches of many small boxes keep the default tiling's launches, which
+    the one-launch step is slower than there; a tuning always selects its own."""
+    hip_stub.run(so, f"""
+b = ljamd.LJBatch(np.full({boxes}, {N}, np.int32), np.full({boxes}, .5), np.full({boxes}, 1.))
+def step_kernels():
+    kernels()
+    b.integrate(0.005, 1)
+    return [n for n, _ in kernels()]
+one, tiled = "k_batch_small", "k_batch_force"
+assert any((one if {small} else tiled) in n for n in step_kernels())
+assert not any((tiled if {small} else one) in n for n in step_kernels())
+b.set_tuning(2, 256, 0)
+names = step_kernels()
+assert any(tiled in n for n in names) and not any(one in n for n in names)
+""")
