@@ -449,7 +449,11 @@ typedef struct lj_batch lj_batch;
  *                  groups of a box, run by 4-wave workgroups: one per item
  *                  (blocks_per_cu 0) or a persistent grid of blocks_per_cu
  *                  workgroups per CU draining the item queue (ipl and jchunk
- *                  are then unused); 0: the tiling above */
+ *                  are then unused); 0: the tiling above
+ * A new batch has {1, 512, 8, 0}.  That tuning also leaves the form of the time
+ * step open: batches of few or large boxes run it as one launch (two with the
+ * thermostat), without a force pass of its own; the others, and single evaluations,
+ * use the tiling.  Setting it again returns to that. */
 typedef struct lj_batch_tuning {
   int ipl;
   int jchunk;
@@ -484,13 +488,16 @@ int lj_batch_get_stats(lj_batch* b, double* out /* nboxes * LJ_BATCH_NSTAT */);
 int lj_batch_reset_stats(lj_batch* b);
 int lj_batch_set_tuning(lj_batch* b, const lj_batch_tuning* t);
 int lj_batch_get_tuning(lj_batch* b, lj_batch_tuning* t);
-/* average time of one batched force pass (HIP events), microseconds: the
- * time step's pass (with pair_once: force-only partials and per-box energy and
+/* average time of one batched force pass of the tuning's tiling (HIP events),
+ * microseconds: the time step's pass, except where the step is one launch (with pair_once: force-only partials and per-box energy and
  * virial totals; after lj_batch_integrate with pair_once the force array's w
  * is 0 until the next lj_batch_compute_forces) */
 int lj_batch_time_force(lj_batch* b, int reps, double* us);
-/* Times every candidate tiling on this batch (reps force passes each), keeps
- * the fastest; cached in the file named by LJ_AUTOTUNE_CACHE when set. */
+/* Times every candidate tiling on this batch (reps force passes each), then whole
+ * steps of the fastest against the one-launch step where a new batch takes that
+ * (on copies of the state), and keeps the faster; *best_us is the time of the
+ * tiling's force pass, or of the one-launch step.  Cached in the file named by
+ * LJ_AUTOTUNE_CACHE when set. */
 int lj_batch_autotune(lj_batch* b, int reps, lj_batch_tuning* best, double* best_us);
 
 /* Fluctuation counters of every box (the single-box lj_fl_* for each box with

@@ -16,6 +16,12 @@
 
 using namespace lj;
 
+namespace {
+// the tuning of a new batch: its steps are one launch where that is faster
+// (small_steps), else this tiling's; single evaluations use the tiling
+constexpr lj_batch_tuning kDefaultTuning{1, 512, 8, 0};
+}  // namespace
+
 struct lj_batch {
   int device = 0;
   int nboxes = 0;
@@ -28,7 +34,7 @@ struct lj_batch {
   std::vector<int> off;
   int Ntot = 0;
   double sub_fraction = 0.5;
-  lj_batch_tuning tune{1, 512, 8, 0};
+  lj_batch_tuning tune = kDefaultTuning;
   hipStream_t stream = nullptr;
   // device
   float4 *pos = nullptr, *vel = nullptr, *force = nullptr, *tF = nullptr;
@@ -37,10 +43,9 @@ struct lj_batch {
   float* apart = nullptr;
   size_t part_cap = 0;
   double* blk = nullptr;
-  // one-launch steps (small; until a tuning is set): the other coordinate buffer,
+  // one-launch steps (small; with the default tuning): the other coordinate buffer,
   // the tiles, the boxes with the tiles' rows, and two buffers of block rows that
   // the steps alternate between
-  bool tuned = false;
   bool small = false;
   uint4* q2 = nullptr;
   BoxParam* box_s = nullptr;
@@ -146,7 +151,14 @@ BatchArgs small_args(lj_batch* b, double dt, int par)
   return a;
 }
 
-// Whether an untuned batch takes the one-launch step.  A tile costs it a workgroup
+bool default_tuning(const lj_batch_tuning& t)
+{
+  const lj_batch_tuning& d = kDefaultTuning;
+  return t.ipl == d.ipl && t.jchunk == d.jchunk && t.blocks_per_cu == d.blocks_per_cu &&
+         t.pair_once == d.pair_once;
+}
+
+// Whether a batch with the default tuning takes the one-launch step.  A tile costs it a workgroup
 // of 1024 threads, 8.7e-3 us however few particles its box has; the four launches
 // of the default tiling cost 105 to 145 us a step and then less per tile: 4.4e-3 us
 // up to 512 particles a box, 7.5e-3 (one launch: 11.8e-3) at 1000, 14.2e-3 (16.3e-3) at
@@ -165,7 +177,7 @@ bool small_steps(const std::vector<int>& N)
 // tables of the one-launch steps, from the boxes' parameters
 int build_small(lj_batch* b, const std::vector<BoxParam>& bp)
 {
-  b->small = !b->tuned && small_steps(b->N);
+  b->small = default_tuning(b->tune) && small_steps(b->N);
   if (!b->small) return LJ_OK;
   const int T = kBatchTile;
   std::vector<BoxParam> bs = bp;
@@ -366,6 +378,62 @@ int enqueue_batch_forces(lj_batch* b, hipStream_t st, bool ties, bool lean = fal
   return LJ_OK;
 }
 
+// us of one of the batch's steps as it is tuned now: replays of a captured run, on
+// copies of the state
+int time_steps(lj_batch* b, int reps, double* us)
+{
+  struct Copies {
+    lj_batch* b;
+    float4 *pos = b->pos, *vel = b->vel, *force = b->force, *tF = b->tF;  // the batch's own
+    lj_obs* own_obs = b->obs;
+    double *own_stats = b->stats, *hist = b->hist;
+    int smp_fl = b->smp_fl;
+    float4* state = nullptr;
+    lj_obs* obs = nullptr;
+    double* stats = nullptr;
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    ~Copies()
+    {
+      (void)hipStreamSynchronize(b->stream);
+      b->pos = pos, b->vel = vel, b->force = force, b->tF = tF;
+      b->obs = own_obs, b->stats = own_stats, b->hist = hist, b->smp_fl = smp_fl;
+      if (exec) (void)hipGraphExecDestroy(exec);
+      if (graph) (void)hipGraphDestroy(graph);
+      dev_free(state);
+      dev_free(obs);
+      dev_free(stats);
+    }
+  } c{b};
+  const size_t n = b->Ntot;
+  hipStream_t st = b->stream;
+  LJ_TRY(dev_alloc(&c.state, 4 * n));
+  LJ_TRY(dev_alloc(&c.obs, b->nboxes));
+  LJ_TRY(dev_alloc(&c.stats, (size_t)b->nboxes * kNStat));
+  const auto copy = [st](void* d, const void* s, size_t bytes) {
+    return hipMemcpyAsync(d, s, bytes, hipMemcpyDeviceToDevice, st);
+  };
+  LJ_HIP(copy(c.state, b->pos, sizeof(float4) * n));
+  LJ_HIP(copy(c.state + n, b->vel, sizeof(float4) * n));
+  LJ_HIP(copy(c.state + 2 * n, b->force, sizeof(float4) * n));
+  LJ_HIP(copy(c.state + 3 * n, b->tF, sizeof(float4) * n));
+  LJ_HIP(copy(c.obs, b->obs, sizeof(lj_obs) * b->nboxes));
+  LJ_HIP(copy(c.stats, b->stats, sizeof(double) * b->nboxes * kNStat));
+  b->pos = c.state, b->vel = c.state + n, b->force = c.state + 2 * n, b->tF = c.state + 3 * n;
+  b->obs = c.obs, b->stats = c.stats, b->hist = nullptr, b->smp_fl = 0;
+  LJ_HIP(hipStreamSynchronize(st));
+  LJ_TRY(capture_batch_steps(b, 0., kGraphSteps, &c.graph, &c.exec));
+  LJ_HIP(hipGraphLaunch(c.exec, st));  // warm
+  LJ_HIP(hipEventRecord(b->e0, st));
+  for (int k = 0; k < reps; ++k) LJ_HIP(hipGraphLaunch(c.exec, st));
+  LJ_HIP(hipEventRecord(b->e1, st));
+  LJ_HIP(hipEventSynchronize(b->e1));
+  float ms = 0.f;
+  LJ_HIP(hipEventElapsedTime(&ms, b->e0, b->e1));
+  *us = 1000.0 * ms / reps / kGraphSteps;
+  return LJ_OK;
+}
+
 std::string tune_key(lj_batch* b)
 {
   hipDeviceProp_t prop;
@@ -377,7 +445,7 @@ std::string tune_key(lj_batch* b)
     h *= 1099511628211ull;
   }
   std::ostringstream os;
-  os << "v4:" << dev << ":" << b->ncu << ":" << b->nboxes << ":" << b->boundary << ":" << std::hex << h;
+  os << "v5:" << dev << ":" << b->ncu << ":" << b->nboxes << ":" << b->boundary << ":" << std::hex << h;
   return os.str();
 }
 
@@ -595,7 +663,6 @@ int lj_batch_set_tuning(lj_batch* b, const lj_batch_tuning* t)
       t->blocks_per_cu < 0 || t->blocks_per_cu > 64 || (t->pair_once != 0 && t->pair_once != 1))
     return fail(LJ_ERR_ARG, "lj_batch_set_tuning: ipl in {1,2}, jchunk in [8, 2^20], blocks_per_cu in [0, 64], pair_once in {0,1}");
   b->tune = *t;
-  b->tuned = true;
   return build_tables(b);
 }
 
@@ -676,6 +743,19 @@ int lj_batch_autotune(lj_batch* b, int reps, lj_batch_tuning* best_out, double* 
     best_t = best_p;
   }
   LJ_TRY(lj_batch_set_tuning(b, &best));
+  // the one-launch step has no force pass of its own: whole steps decide (16 boxes
+  // of 400, EVN: 9 us against 28 with the best tiling)
+  double tiled = 0., one = 0.;
+  if (small_steps(b->N) && time_steps(b, reps, &tiled) == LJ_OK) {
+    LJ_TRY(lj_batch_set_tuning(b, &kDefaultTuning));
+    if (time_steps(b, reps, &one) == LJ_OK && one <= tiled) {
+      best = kDefaultTuning;
+      best_t = one;
+    } else {
+      LJ_TRY(lj_batch_set_tuning(b, &best));
+    }
+  }
+  (void)hipGetLastError();  // copies without room: the best tiling stays
   if (cache) {
     std::ofstream o(cache, std::ios::app);
     o << key << " " << best.ipl << " " << best.jchunk << " " << best.blocks_per_cu << " "

@@ -1,7 +1,8 @@
 // A HIP runtime on the host for tests of the library's host code without a GPU:
 // device memory is host memory, copies are copies, kernels are recorded and do
 // nothing, and allocations can be refused.  Loaded with RTLD_GLOBAL ahead of
-// libljhip.so, whose HIP calls then arrive here (tests/hip_stub.py).
+// libljhip.so, whose HIP calls then arrive here (tests/hip_stub.py).  Time is
+// counted in launches, a microsecond each, for the events.
 //
 // Single-threaded.  stub_* functions read and set its state.
 #include <hip/hip_runtime_api.h>
@@ -32,6 +33,9 @@ struct State {
   dim3 grid, block;
   size_t shared = 0;
   hipStream_t stream = nullptr;
+  bool capturing = false;
+  long clock = 0, captured = 0;       // launches run, and in the present capture
+  std::map<const void*, long> times;  // of events; launches of graphs
   hipError_t last = hipSuccess;
 };
 
@@ -116,6 +120,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* sh, hipStream_t* 
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t, hipStream_t)
 {
   S().launches.push_back({S().kernels[f], g, b});
+  ++(S().capturing ? S().captured : S().clock);
   return hipSuccess;
 }
 hipError_t hipExtLaunchKernel(const void* f, dim3 g, dim3 b, void** a, size_t sh, hipStream_t st,
@@ -221,20 +226,32 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned)
 }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode)
+{
+  S().capturing = true;
+  S().captured = 0;
+  return hipSuccess;
+}
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g)
 {
   *g = handle<hipGraph_t>();
+  S().times[*g] = S().captured;
+  S().capturing = false;
   return hipSuccess;
 }
-hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t)
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t*, char*, size_t)
 {
   *e = handle<hipGraphExec_t>();
+  S().times[*e] = S().times[g];
   ++S().instantiated;
   ++S().graphs;
   return hipSuccess;
 }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t)
+{
+  S().clock += S().times[e];
+  return hipSuccess;
+}
 hipError_t hipGraphExecDestroy(hipGraphExec_t)
 {
   --S().graphs;
@@ -252,11 +269,15 @@ hipError_t hipEventDestroy(hipEvent_t)
   --S().events;
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t)
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t)
 {
-  *ms = 1.f;
+  S().times[e] = S().clock;
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b)
+{
+  *ms = 1e-3f * (float)(S().times[b] - S().times[a]);
   return hipSuccess;
 }
 

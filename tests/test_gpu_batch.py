@@ -146,7 +146,7 @@ def test_batch_pair_once_step_totals(canon, bc):
 
 @pytest.mark.parametrize("canon,tuning", [(ljamd.EVN, (1, 512, 8, 0)), (ljamd.EVN, (1, 512, 0, 1)),
                                           (ljamd.TVN, (1, 512, 0, 1)), (ljamd.TVN, (2, 1024, 4, 0)),
-                                          (ljamd.TVN, (1, 512, 8, 1))])
+                                          (ljamd.TVN, (1, 512, 8, 1)), (ljamd.EVN, (1, 512, 4, 0))])
 def test_batch_graph_replay_deterministic(canon, tuning):
     """20 steps as 8 + 8 + 4 x 1 (8-step graphs whose kick kernels do the next
     drift and reset the work queue) and as 7 x 1 + (8 + 5 x 1): the same bits

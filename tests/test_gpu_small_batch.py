@@ -1,7 +1,7 @@
 """The one-launch time steps of a batch whose tuning was not set, at the edges
 of their tiles (16 particles) and LDS chunks (2048): box sizes 1 to 4097 in one
-batch, against the same boxes run one by one through the separate kernels of
-the sliced tuning, and in any split of the run."""
+batch, against the separate kernels of a sliced tuning (the default tuning, set
+again, gives the one-launch step's bits), and in any split of the run."""
 import numpy as np
 import pytest
 
@@ -22,7 +22,8 @@ def test_small_batch_edges(canon, bc):
     steps = 20
     print(f"\n[case] small batch canon={canon} bc={bc}", flush=True)
     out = []
-    for chunks, tuning in (([steps], None), ([7, 13], None), ([steps], (1, 512, 8, 0))):
+    for chunks, tuning in (([steps], None), ([7, 13], None), ([steps], (1, 512, 8, 0)),
+                           ([steps], (1, 512, 4, 0))):
         with ljamd.LJBatch(N, RHO, T0, canonical=canon, boundary=bc, seed=31) as b:
             if tuning:
                 b.set_tuning(*tuning)
@@ -35,9 +36,11 @@ def test_small_batch_edges(canon, bc):
             b.compute_forces()
             full = b.observables()
         out.append((h, obs, p, v, f, st, full))
-    a, split, sliced = out
-    for x, y in zip((a[0], a[5], *a[2], *a[3], *a[4]), (split[0], split[5], *split[2], *split[3], *split[4])):
-        assert np.array_equal(x, y)
+    a, split, again, sliced = out
+    for o in (split, again):
+        for x, y in zip((a[0], a[5], *a[2], *a[3], *a[4]), (o[0], o[5], *o[2], *o[3], *o[4])):
+            assert np.array_equal(x, y)
+    assert any(not np.array_equal(x, y) for x, y in zip(a[3], sliced[3]))  # another route
     assert np.all(a[5][:, 0] == steps) and np.array_equal(a[5][:, 9], sliced[5][:, 9])
     for k in range(N.size):
         assert np.max(np.abs(a[0][:, k, 0] - sliced[0][:, k, 0])) / N[k] <= 2e-5, k
@@ -47,3 +50,24 @@ def test_small_batch_edges(canon, bc):
         assert abs(a[1][k]["W"] - a[6][k]["W"]) <= 1e-5 * max(abs(a[6][k]["W"]), N[k]), k
         e = np.sum(a[4][k].reshape(-1, 4)[:, 3].astype(np.float64)) * 2.0
         assert rel(e, a[1][k]["V"]) <= 1e-5 or abs(e) < 1e-5, k
+
+
+def test_autotune_keeps_the_one_launch_step():
+    """16 boxes of 400, where the one-launch step takes a third of the best tiling's
+    time: the autotuner leaves it on, and the batch's state alone."""
+    n, r, t = np.full(16, 400, np.int32), np.linspace(0.05, 0.8, 16), np.full(16, 1.4)
+    print("\n[case] autotune 16 of 400", flush=True)
+    out = []
+    for tune in (False, True):
+        with ljamd.LJBatch(n, r, t, seed=5) as b:
+            b.integrate(0.004, 5)
+            fresh = b.tuning()
+            if tune:
+                best, us = b.autotune(reps=3)
+                print(f"  {best} {us:.1f} us", flush=True)
+                assert best == b.tuning() == fresh
+            a = [b.get_array(k) for k in (ljamd.ARRAY_POS, ljamd.ARRAY_VEL, ljamd.ARRAY_FORCE)]
+            h = b.integrate_hist(0.004, 20)
+            out.append((*a, h, b.stats(), b.get_array(ljamd.ARRAY_POS), b.get_array(ljamd.ARRAY_VEL)))
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)

@@ -93,3 +93,35 @@ b.set_tuning(2, 256, 0)
 names = step_kernels()
 assert any(tiled in n for n in names) and not any(one in n for n in names)
 """)
+
+
+def test_batch_returns_to_its_default_step(so):
+    """What lj_batch_get_tuning gives for a new batch sets the new batch's step again,
+    and the autotuner keeps the one-launch step where that is faster (here, where
+    time is launches, always within its sizes), leaving the batch's arrays alone."""
+    hip_stub.run(so, """
+b = ljamd.LJBatch(np.full(16, 400, np.int32), np.full(16, .5), np.full(16, 1.))
+def one_launch():
+    kernels()
+    b.integrate(0.005, 1)
+    return any("k_batch_small" in n for n, _ in kernels())
+fresh = b.tuning()
+assert one_launch()
+b.set_tuning(*fresh)
+assert one_launch() and b.tuning() == fresh
+b.set_tuning(1, 512, 0, 1)
+assert not one_launch()
+b.set_tuning(*fresh)
+assert one_launch()
+live = stub.stub_live()
+best, us = b.autotune(reps=2)
+assert best == b.tuning() == fresh and us < 1.5 and one_launch()
+# no room for the copies it times steps on: the best tiling
+stub.stub_fail_in(0)
+best, _ = b.autotune(reps=2)
+stub.stub_fail_in(-1)
+assert best == b.tuning() != fresh and not one_launch()
+big = ljamd.LJBatch(np.full(2000, 400, np.int32), np.full(2000, .5), np.full(2000, 1.))
+best, _ = big.autotune(reps=2)
+assert best == big.tuning() != fresh
+""")
