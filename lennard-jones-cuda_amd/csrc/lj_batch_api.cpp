@@ -35,6 +35,7 @@ struct lj_batch {
   int Ntot = 0;
   double sub_fraction = 0.5;
   lj_batch_tuning tune = kDefaultTuning;
+  bool ready = false;  // the tuning's tables stand
   hipStream_t stream = nullptr;
   // device
   float4 *pos = nullptr, *vel = nullptr, *force = nullptr, *tF = nullptr;
@@ -97,6 +98,13 @@ int bsetdev(lj_batch* b)
 {
   if (!b) return fail(LJ_ERR_ARG, "null batch");
   LJ_HIP(hipSetDevice(b->device));
+  return LJ_OK;
+}
+
+int bready(lj_batch* b)
+{
+  LJ_TRY(bsetdev(b));
+  if (!b->ready) return fail(LJ_ERR_STATE, "the batch has no tables (no room at lj_batch_set_tuning)");
   return LJ_OK;
 }
 
@@ -272,6 +280,9 @@ int build_tables(lj_batch* b)
     return bp[x.box].N > bp[y.box].N;
   });
   LJ_HIP(hipStreamSynchronize(b->stream));
+  // the captured steps hold the tables' addresses; a failure below leaves none
+  bdrop_graph(b);
+  b->ready = false;
   if (pbase > b->part_cap) {
     dev_free(b->fpart);
     dev_free(b->apart);
@@ -307,7 +318,7 @@ int build_tables(lj_batch* b)
   b->hbox = bp;
   b->nblocks = (int)pblock.size();
   b->nitems = (int)items.size();
-  bdrop_graph(b);
+  b->ready = true;
   return LJ_OK;
 }
 
@@ -596,7 +607,7 @@ int lj_batch_get_array(lj_batch* b, int box, int type, float* host4N)
 
 int lj_batch_compute_forces(lj_batch* b)
 {
-  LJ_TRY(bsetdev(b));
+  LJ_TRY(bready(b));
   hipStream_t st = b->stream;
   LJ_TRY(enqueue_batch_forces(b, st, true));
   const BatchArgs a = bargs(b, 0.);
@@ -662,8 +673,16 @@ int lj_batch_set_tuning(lj_batch* b, const lj_batch_tuning* t)
   if (!t || (t->ipl != 1 && t->ipl != 2) || t->jchunk < 8 || t->jchunk > (1 << 20) ||
       t->blocks_per_cu < 0 || t->blocks_per_cu > 64 || (t->pair_once != 0 && t->pair_once != 1))
     return fail(LJ_ERR_ARG, "lj_batch_set_tuning: ipl in {1,2}, jchunk in [8, 2^20], blocks_per_cu in [0, 64], pair_once in {0,1}");
+  const lj_batch_tuning old = b->tune;
   b->tune = *t;
-  return build_tables(b);
+  const int rc = build_tables(b);
+  if (rc == LJ_OK) return LJ_OK;
+  // no room for the new tables: the old ones again, if they find it
+  const std::string msg = last_error();
+  (void)hipGetLastError();
+  b->tune = old;
+  if (build_tables(b) != LJ_OK) (void)hipGetLastError();
+  return fail(rc, "%s", msg.c_str());
 }
 
 int lj_batch_get_tuning(lj_batch* b, lj_batch_tuning* t)
@@ -675,7 +694,7 @@ int lj_batch_get_tuning(lj_batch* b, lj_batch_tuning* t)
 
 int lj_batch_time_force(lj_batch* b, int reps, double* us)
 {
-  LJ_TRY(bsetdev(b));
+  LJ_TRY(bready(b));
   if (reps <= 0 || !us) return fail(LJ_ERR_ARG, "lj_batch_time_force: bad arguments");
   hipStream_t st = b->stream;
   LJ_TRY(enqueue_batch_forces(b, st, false, true));  // warm
@@ -773,7 +792,7 @@ int lj_batch_integrate(lj_batch* b, double dt, int nsteps)
 
 int lj_batch_integrate_hist(lj_batch* b, double dt, int nsteps, double* hist)
 {
-  LJ_TRY(bsetdev(b));
+  LJ_TRY(bready(b));
   if (nsteps < 0 || !std::isfinite(dt)) return fail(LJ_ERR_ARG, "lj_batch_integrate: bad arguments");
   if (nsteps == 0) return LJ_OK;
   hipStream_t st = b->stream;

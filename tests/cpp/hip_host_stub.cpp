@@ -28,7 +28,8 @@ struct State {
   std::map<std::string, void*> symbols;
   std::map<const void*, std::pair<std::string, size_t>> vars;
   size_t refuse_above = ~size_t(0);  // hipMalloc of more bytes fails
-  long fail_in = -1;                 // the hipMalloc after that many fails, and all later
+  long fail_in = -1;                 // the hipMalloc after that many fails,
+  bool fail_once = false;            // or all from there on
   long mallocs = 0, refused = 0, instantiated = 0, graphs = 0, events = 0;
   dim3 grid, block;
   size_t shared = 0;
@@ -71,7 +72,11 @@ extern "C" {
 
 // ---- the stub's own interface ----
 void stub_refuse_above(size_t bytes) { S().refuse_above = bytes; }
-void stub_fail_in(long n) { S().fail_in = n; }
+void stub_fail_in(long n, int once)
+{
+  S().fail_in = n;
+  S().fail_once = once != 0;
+}
 long stub_mallocs() { return S().mallocs; }
 long stub_refused() { return S().refused; }
 long stub_instantiated() { return S().instantiated; }
@@ -143,7 +148,7 @@ hipError_t hipMalloc(void** p, size_t n)
   State& s = S();
   ++s.mallocs;
   const bool no = n > s.refuse_above || s.fail_in == 0;
-  if (s.fail_in > 0) --s.fail_in;
+  if (s.fail_in > 0 || s.fail_once) --s.fail_in;
   *p = no ? nullptr : pages(n);
   if (!*p) {
     ++s.refused;

@@ -21,7 +21,7 @@ sys.path.insert(0, {python!r})
 import ljamd
 from ljamd import _lib as L
 stub.stub_refuse_above.argtypes = [C.c_size_t]
-stub.stub_fail_in.argtypes = [C.c_long]
+stub.stub_fail_in.argtypes = [C.c_long, C.c_int]
 stub.stub_launch_name.argtypes = stub.stub_launch_grid.argtypes = [C.c_long]
 stub.stub_launch_name.restype = C.c_char_p
 stub.stub_launch_grid.restype = C.c_uint

@@ -49,11 +49,11 @@ s.Integrate(0.005, 3)
 dr2 = L.lib().lj_rdf_dr2_default(16384) * 256 / 1000
 assert any("k_rdf_cells" in n for n, _ in kernels())
 held, captured = stub.stub_live(), stub.stub_instantiated()
-stub.stub_fail_in({refused})
+stub.stub_fail_in({refused}, 0)
 try:
     s.rdf(ljamd.RDF_REF_GPU, 1000, dr2)
 finally:
-    stub.stub_fail_in(-1)
+    stub.stub_fail_in(-1, 0)
     # the captured steps are gone before anything else can run them
     assert stub.stub_graphs() == 0, "captured steps hold freed lists"
 assert stub.stub_refused() > 0
@@ -117,11 +117,50 @@ live = stub.stub_live()
 best, us = b.autotune(reps=2)
 assert best == b.tuning() == fresh and us < 1.5 and one_launch()
 # no room for the copies it times steps on: the best tiling
-stub.stub_fail_in(0)
+stub.stub_fail_in(0, 0)
 best, _ = b.autotune(reps=2)
-stub.stub_fail_in(-1)
+stub.stub_fail_in(-1, 0)
 assert best == b.tuning() != fresh and not one_launch()
 big = ljamd.LJBatch(np.full(2000, 400, np.int32), np.full(2000, .5), np.full(2000, 1.))
 best, _ = big.autotune(reps=2)
 assert best == big.tuning() != fresh
+""")
+
+
+@pytest.mark.parametrize("once", [1, 0])
+@pytest.mark.parametrize("refused", range(3))  # two arrays of slots, one of totals
+def test_batch_tuning_without_room(so, refused, once):
+    """A tuning whose tables find no room leaves the batch as it was tuned before, or,
+    where the old tables find none either, with calls that refuse to run; never
+    with captured steps, or a tuning, that do not fit the tables."""
+    hip_stub.run(so, f"""
+b = ljamd.LJBatch(np.full(32, 1000, np.int32), np.full(32, .5), np.full(32, 1.))
+b.set_tuning(2, 2048, 0)
+b.integrate(0.005, 1)
+captured = stub.stub_instantiated()
+stub.stub_fail_in({refused}, {once})
+try:
+    b.set_tuning(1, 256, 0, 1)
+    assert False
+except ljamd.LJError:
+    pass
+assert stub.stub_graphs() == 0, "captured steps hold freed tables"
+assert b.tuning() == (2, 2048, 0, 0)
+kernels()
+if {once} or {refused} == 2:  # the old tables need no totals
+    b.integrate(0.005, 1)
+    assert stub.stub_instantiated() > captured
+    assert any("k_batch_force" in n for n, _ in kernels())
+else:
+    for call in (lambda: b.integrate(0.005, 1), b.compute_forces, b.time_force):
+        try:
+            call()
+            assert False
+        except ljamd.LJError as e:
+            assert "no tables" in str(e)
+    assert not kernels()
+    stub.stub_fail_in(-1, 0)
+    b.set_tuning(1, 256, 0, 1)
+    b.integrate(0.005, 1)
+    assert any("k_batch_force_n3" in n for n, _ in kernels())
 """)
