@@ -1335,7 +1335,6 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
   CompatScratch* s = nullptr;
   ForcePlan pl = compat_plan(N, ps);
   if (compat_scratch(N, pl, &s) != LJ_OK) {  // no room for its partial sums
-    (void)hipGetLastError();                 // else the next launch reports it
     pl = make_force_plan(N, 0, 1);
     LJ_TRY(compat_scratch(N, pl, &s));
   }
@@ -1375,9 +1374,7 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
     if (nc > 0) {
       bool grown = false;
       if (rdf_cells_ensure(s->cells, N, nc * nc * nc, a.nbins, st, &grown) == LJ_OK)
-        a.cells = &s->cells;
-      else
-        (void)hipGetLastError();  // without the lists: all pairs
+        a.cells = &s->cells;  // else all pairs
     } else {
       size_t need = 0;
       (void)rdf_workgroups(a, &need);
@@ -1385,8 +1382,7 @@ int compat_forces(float* Pos, float* Force, float* host_pressure, int N, float h
         LJ_HIP(hipStreamSynchronize(st));
         dev_free(s->rows);
         s->rows_cap = 0;
-        if (dev_alloc(&s->rows, need) == LJ_OK) s->rows_cap = need;
-        else (void)hipGetLastError();  // without rows: atomics
+        if (dev_alloc(&s->rows, need) == LJ_OK) s->rows_cap = need;  // else atomics
       }
       a.rows = s->rows;
       a.rows_cap = s->rows_cap;

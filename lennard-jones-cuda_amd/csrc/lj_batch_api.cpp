@@ -679,9 +679,8 @@ int lj_batch_set_tuning(lj_batch* b, const lj_batch_tuning* t)
   if (rc == LJ_OK) return LJ_OK;
   // no room for the new tables: the old ones again, if they find it
   const std::string msg = last_error();
-  (void)hipGetLastError();
   b->tune = old;
-  if (build_tables(b) != LJ_OK) (void)hipGetLastError();
+  (void)build_tables(b);
   return fail(rc, "%s", msg.c_str());
 }
 
@@ -764,7 +763,7 @@ int lj_batch_autotune(lj_batch* b, int reps, lj_batch_tuning* best_out, double* 
   LJ_TRY(lj_batch_set_tuning(b, &best));
   // the one-launch step has no force pass of its own: whole steps decide (16 boxes
   // of 400, EVN: 9 us against 28 with the best tiling)
-  double tiled = 0., one = 0.;
+  double tiled = 0., one = 0.;  // no room for the copies: the best tiling stays
   if (small_steps(b->N) && time_steps(b, reps, &tiled) == LJ_OK) {
     LJ_TRY(lj_batch_set_tuning(b, &kDefaultTuning));
     if (time_steps(b, reps, &one) == LJ_OK && one <= tiled) {
@@ -774,7 +773,6 @@ int lj_batch_autotune(lj_batch* b, int reps, lj_batch_tuning* best_out, double* 
       LJ_TRY(lj_batch_set_tuning(b, &best));
     }
   }
-  (void)hipGetLastError();  // copies without room: the best tiling stays
   if (cache) {
     std::ofstream o(cache, std::ios::app);
     o << key << " " << best.ipl << " " << best.jchunk << " " << best.blocks_per_cu << " "

@@ -136,7 +136,6 @@ inline int attach_rdf_workspace(lj_ctx* c, RdfArgs& a)
       a.cells = &c->rdf_cells;
       return LJ_OK;
     }
-    (void)hipGetLastError();  // else the next launch reports it
   }
   size_t need = 0;
   (void)rdf_workgroups(a, &need);
@@ -148,8 +147,7 @@ inline int attach_rdf_workspace(lj_ctx* c, RdfArgs& a)
     dev_free(c->rdf_rows);
     c->rdf_rows_cap = c->smp_args.rows_cap = 0;
     c->smp_args.rows = nullptr;
-    if (dev_alloc(&c->rdf_rows, need) == LJ_OK) c->rdf_rows_cap = need;
-    else (void)hipGetLastError();  // without rows: atomics
+    if (dev_alloc(&c->rdf_rows, need) == LJ_OK) c->rdf_rows_cap = need;  // else atomics
     if (sampled && c->rdf_rows) {
       c->smp_args.rows = c->rdf_rows;
       c->smp_args.rows_cap = need;

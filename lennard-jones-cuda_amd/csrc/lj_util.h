@@ -35,6 +35,7 @@ int dev_alloc(T** p, size_t count)
   hipError_t e = hipMalloc((void**)p, count * sizeof(T));
   if (e != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();  // told here: the next launch is not to report it
     return fail(LJ_ERR_ALLOC, "hipMalloc(%zu bytes): %s", count * sizeof(T), hipGetErrorString(e));
   }
   return LJ_OK;

@@ -164,3 +164,19 @@ else:
     b.integrate(0.005, 1)
     assert any("k_batch_force_n3" in n for n, _ in kernels())
 """)
+
+
+def test_refused_allocation_is_told_once(so):
+    """A call that found no room says so; the next call, which needs none, runs."""
+    hip_stub.run(so, """
+s = ljamd.LJSystem(400, 0.5, 1.0)
+s.Integrate(0.005, 1)
+stub.stub_fail_in(0, 1)
+try:
+    s.trajectory_loss(0.005, 2)
+    assert False
+except ljamd.LJError as e:
+    assert "hipMalloc" in str(e)
+s.CalculateForces()
+s.Integrate(0.005, 1)
+""")
