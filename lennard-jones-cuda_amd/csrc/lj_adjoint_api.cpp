@@ -94,37 +94,48 @@ bool adj_pass_chosen()
   return false;
 }
 
+// the arrays whose sizes only N decides
+int adj_alloc(lj_ctx* c)
+{
+  AdjState* a = c->adj = new AdjState();
+  a->N = c->cfg.N;
+  a->nblk = adj_rows(c->cfg.N);  // rows of k_adj_reduce / k_dkick
+  const int N = a->N;
+  a->plan = adj_force_plan(N);
+  LJ_TRY(dev_alloc(&a->part, (size_t)3 * a->plan.S * a->plan.Npad));
+  if (c->small_T && !adj_pass_chosen()) a->T = c->small_T;
+  a->rows = a->T ? std::max(a->nblk, (N + a->T - 1) / a->T) : a->nblk;
+  LJ_TRY(dev_alloc(&a->z, N));
+  if (a->T) LJ_TRY(dev_alloc(&a->z2, N));
+  LJ_TRY(dev_alloc(&a->hz, N));
+  LJ_TRY(dev_alloc(&a->f, N));
+  LJ_TRY(dev_alloc(&a->gw, N));
+  LJ_TRY(dev_alloc(&a->u, N));
+  LJ_TRY(dev_alloc(&a->lv, N));
+  LJ_TRY(dev_alloc(&a->dx0, N));
+  LJ_TRY(dev_alloc(&a->blk, (size_t)2 * a->rows * 8));  // two buffers
+  LJ_TRY(dev_alloc(&a->rowacc, (size_t)a->rows * 8));
+  LJ_TRY(dev_alloc(&a->scal, kAdjScalars));
+  LJ_TRY(dev_alloc(&a->theta, 2));
+  LJ_TRY(dev_alloc(&a->acc, 4));
+  LJ_TRY(dev_alloc(&a->xd, (size_t)3 * N));
+  a->vd = a->xd + N;
+  a->fd = a->xd + 2 * N;
+  LJ_TRY(dev_alloc(&a->dxf, N));
+  LJ_TRY(dev_alloc(&a->xf, N));
+  return LJ_OK;
+}
+
 int adj_ensure(lj_ctx* c, int ncheck, int seg)
 {
-  AdjState*& a = c->adj;
-  if (!a) {
-    a = new AdjState();
-    a->N = c->cfg.N;
-    a->nblk = adj_rows(c->cfg.N);  // rows of k_adj_reduce / k_dkick
-    const int N = a->N;
-    a->plan = adj_force_plan(N);
-    LJ_TRY(dev_alloc(&a->part, (size_t)3 * a->plan.S * a->plan.Npad));
-    if (c->small_T && !adj_pass_chosen()) a->T = c->small_T;
-    a->rows = a->T ? std::max(a->nblk, (N + a->T - 1) / a->T) : a->nblk;
-    LJ_TRY(dev_alloc(&a->z, N));
-    if (a->T) LJ_TRY(dev_alloc(&a->z2, N));
-    LJ_TRY(dev_alloc(&a->hz, N));
-    LJ_TRY(dev_alloc(&a->f, N));
-    LJ_TRY(dev_alloc(&a->gw, N));
-    LJ_TRY(dev_alloc(&a->u, N));
-    LJ_TRY(dev_alloc(&a->lv, N));
-    LJ_TRY(dev_alloc(&a->dx0, N));
-    LJ_TRY(dev_alloc(&a->blk, (size_t)2 * a->rows * 8));  // two buffers
-    LJ_TRY(dev_alloc(&a->rowacc, (size_t)a->rows * 8));
-    LJ_TRY(dev_alloc(&a->scal, kAdjScalars));
-    LJ_TRY(dev_alloc(&a->theta, 2));
-    LJ_TRY(dev_alloc(&a->acc, 4));
-    LJ_TRY(dev_alloc(&a->xd, (size_t)3 * N));
-    a->vd = a->xd + N;
-    a->fd = a->xd + 2 * N;
-    LJ_TRY(dev_alloc(&a->dxf, N));
-    LJ_TRY(dev_alloc(&a->xf, N));
+  if (!c->adj) {
+    const int rc = adj_alloc(c);
+    if (rc != LJ_OK) {  // all of them or none: the next call starts again
+      adj_free(c);
+      return rc;
+    }
   }
+  AdjState* a = c->adj;
   if (ncheck > a->ck_cap) {
     LJ_HIP(hipStreamSynchronize(c->stream));
     dev_free(a->ck);

@@ -180,3 +180,33 @@ except ljamd.LJError as e:
 s.CalculateForces()
 s.Integrate(0.005, 1)
 """)
+
+
+@pytest.mark.parametrize("N", [400, 5000])
+def test_adjoint_arrays_without_room(so, N):
+    """The differentiable path's arrays are allocated all or not at all: a call after
+    one that found no room starts again instead of using what is missing."""
+    hip_stub.run(so, f"""
+def first(s):
+    n = stub.stub_mallocs()
+    s.trajectory_grad(0.005, 6, 3)
+    return stub.stub_mallocs() - n
+with ljamd.LJSystem({N}, 0.5, 1.0) as s:
+    whole = first(s)
+assert whole > 15
+for refused in range(whole):
+    with ljamd.LJSystem({N}, 0.5, 1.0) as s:
+        live = stub.stub_live()
+        stub.stub_fail_in(refused, 1)
+        try:
+            first(s)
+            assert False
+        except ljamd.LJError:
+            pass
+        if refused < whole - 2:  # before the checkpoints and the segment's states
+            assert stub.stub_live() == live
+            assert first(s) == whole
+        else:
+            assert first(s) == whole - refused
+    assert stub.stub_live() == 0
+""")
