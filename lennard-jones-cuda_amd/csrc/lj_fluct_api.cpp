@@ -105,6 +105,11 @@ int lj_set_step_sampling(lj_ctx* c, const lj_step_sampling* s)
       return fail(LJ_ERR_ARG, "lj_set_step_sampling: unknown rule %d", rule);
     if (nbins <= 0 || nbins > 8000)
       return fail(LJ_ERR_ARG, "lj_set_step_sampling: nbins must be in [1, 8000]");
+    // the captured steps hold the old sampling's arrays: from here on nothing is
+    // sampled until the new arrays stand
+    drop_graph(c);
+    c->smp_rdf = LJ_SAMPLE_RDF_OFF;
+    c->smp_args = RdfArgs{};
     const float dr2 = s->rdf_dr2 > 0.f ? s->rdf_dr2 : rdf_dr2_rule(c->cfg.N);
     const double rmax = s->rdf_rmax > 0. ? s->rdf_rmax : c->L / 2.;
     if (nbins > c->rdf_step_cap) {

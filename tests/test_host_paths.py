@@ -210,3 +210,27 @@ for refused in range(whole):
             assert first(s) == whole - refused
     assert stub.stub_live() == 0
 """)
+
+
+@pytest.mark.parametrize("refused", range(2))
+def test_step_sampling_without_room(so, refused):
+    """Sampling more bins than before where the histogram or its table finds no room:
+    the captured steps, which hold the old ones, are dropped and nothing is sampled."""
+    hip_stub.run(so, f"""
+s = ljamd.LJSystem(400, 0.5, 1.0)
+s.set_step_sampling(ljamd.SAMPLE_RDF_SUM, rdf_rule=ljamd.RDF_REF_CPU, rdf_nbins=100)
+s.Integrate(0.005, 2)
+stub.stub_fail_in({refused}, 1)
+try:
+    s.set_step_sampling(ljamd.SAMPLE_RDF_SUM, rdf_rule=ljamd.RDF_REF_CPU, rdf_nbins=500)
+    assert False
+except ljamd.LJError:
+    pass
+assert stub.stub_graphs() == 0, "captured steps hold a freed histogram"
+kernels()
+s.Integrate(0.005, 2)
+assert not any("rdf" in n for n, _ in kernels())
+s.set_step_sampling(ljamd.SAMPLE_RDF_SUM, rdf_rule=ljamd.RDF_REF_CPU, rdf_nbins=500)
+s.Integrate(0.005, 2)
+assert any("rdf" in n for n, _ in kernels())
+""")
