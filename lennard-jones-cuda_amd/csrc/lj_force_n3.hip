@@ -1164,7 +1164,7 @@ ForcePlan compat_plan(int N, const PairScalars& ps)
 {
   if (n3_eligible(N) && N <= kCompatOnceMaxN && ps.thr > 0.f) {
     const ForcePlan pl = make_n3_plan(N);
-    if (pl.n3 != 4) return pl;
+    if (pl.n3 != 4 && (size_t)pl.S * pl.Npad <= kCompatSlots) return pl;
   }
   return make_force_plan(N, 0, 1);
 }

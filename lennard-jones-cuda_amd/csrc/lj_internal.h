@@ -67,10 +67,12 @@ ForcePlan make_shard_plan(int N, int shard, int nshards, int jslices);
 ForcePlan make_n3_plan(int N, bool comp = false);
 // The plan of calculateNForces and its no-allocation twin: every pair once from
 // the sizes on at which the time step does so (N = 16384 periodic: 159 against 104
-// us), up to kCompatOnceMaxN particles, since the twin's partial sums, an entry
-// per particle and group, are a file-scope array (81 MiB at that size); else the
-// sliced grid.
+// us), up to kCompatOnceMaxN particles and kCompatSlots entries, since the twin's
+// partial sums, an entry per particle and group, are a file-scope array (80 MiB);
+// else the sliced grid.  The entries hold the groups of 256 at that size; groups of
+// 128, which LJ_PAIR_ONCE_SPLIT=1 takes at any size, to N of about 23,000.
 constexpr int kCompatOnceMaxN = 32768;
+constexpr size_t kCompatSlots = (size_t)kCompatOnceMaxN / 256 * kCompatOnceMaxN;
 struct PairScalars;
 ForcePlan compat_plan(int N, const PairScalars& ps);
 // false when LJ_PAIR_ONCE_COMP=0 keeps the compensated mode on the sliced kernel

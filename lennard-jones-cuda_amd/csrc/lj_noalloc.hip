@@ -23,10 +23,10 @@ using namespace lj;
 
 // largest numBodies served
 constexpr int kNoAllocMaxN = 65536;
-// entries S x Npad of compat_plan at any N <= kNoAllocMaxN: the pair-once pass of
-// kCompatOnceMaxN particles in groups of 256; the sliced plan (make_force_plan(N,
-// 0, 1)) has at most 587520 (N = 65280: 9 slices of 65280)
-constexpr size_t kPartCap = (size_t)kCompatOnceMaxN / 256 * kCompatOnceMaxN;
+// entries S x Npad of compat_plan at any N <= kNoAllocMaxN: its pair-once passes keep
+// to this; the sliced plan (make_force_plan(N, 0, 1)) has at most 587520 (N = 65280:
+// 9 slices of 65280)
+constexpr size_t kPartCap = kCompatSlots;
 static_assert(kPartCap >= 589824, "the sliced plan's entries");
 constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 constexpr size_t kBlkRows = (kNoAllocMaxN + kBlock - 1) / kBlock;

@@ -234,3 +234,23 @@ s.set_step_sampling(ljamd.SAMPLE_RDF_SUM, rdf_rule=ljamd.RDF_REF_CPU, rdf_nbins=
 s.Integrate(0.005, 2)
 assert any("rdf" in n for n, _ in kernels())
 """)
+
+
+@pytest.mark.parametrize("split", ["", "0", "1"])
+def test_noalloc_forces_at_every_size(so, split):
+    """calculateNForcesNoAlloc serves every N up to 65536 whatever groups
+    LJ_PAIR_ONCE_SPLIT asks for, with the launches of calculateNForces."""
+    hip_stub.run(so, """
+p, f = C.c_void_p(), C.c_void_p()
+L.lib().allocateArray(C.byref(p), 65536)
+L.lib().allocateArray(C.byref(f), 65536)
+def force_pass(call, N):
+    kernels()
+    rc = call(p, f, None, N, 30., 1, None, 0.1, 256, 1)
+    got = [k for k in kernels() if "force" in k[0]]
+    assert got, N
+    return rc, got
+for N in [1, 400, 3071, 3072, 5003, 16384, 23039, 23040, 24001, 32767, 32768, 32769, 65536]:
+    rc, got = force_pass(L.lib().calculateNForcesNoAlloc, N)
+    assert rc == 0 and got == force_pass(L.lib().calculateNForces, N)[1], (N, rc, got)
+""", env={"LJ_PAIR_ONCE_SPLIT": split} if split else {})
