@@ -1296,18 +1296,24 @@ int compat_scratch(int N, const ForcePlan& pl, CompatScratch** out)
   s.device = dev;
   if (!s.st) LJ_HIP(hipStreamCreateWithFlags(&s.st, hipStreamNonBlocking));
   const size_t part = (size_t)pl.S * pl.Npad;
-  if (N > s.capN || part > s.capPart) {
+  // grown apart from each other, so that alternating sizes settle: the entries are
+  // not monotonic in N (4.2e6 at 32,768, every pair once; below 0.6e6 above)
+  if (N > s.capN) {
     LJ_HIP(hipStreamSynchronize(s.st));
     dev_free(s.q);
-    dev_free(s.fpart);
-    dev_free(s.apart);
     dev_free(s.blk);
     s.capN = 0;
     LJ_TRY(dev_alloc(&s.q, N));
-    LJ_TRY(dev_alloc(&s.fpart, (size_t)pl.S * pl.Npad));
-    LJ_TRY(dev_alloc(&s.apart, (size_t)pl.S * pl.Npad));
     LJ_TRY(dev_alloc(&s.blk, (size_t)((N + kBlock - 1) / kBlock) * kBlkFields));
     s.capN = N;
+  }
+  if (part > s.capPart) {
+    LJ_HIP(hipStreamSynchronize(s.st));
+    dev_free(s.fpart);
+    dev_free(s.apart);
+    s.capPart = 0;
+    LJ_TRY(dev_alloc(&s.fpart, part));
+    LJ_TRY(dev_alloc(&s.apart, part));
     s.capPart = part;
   }
   if (!s.rdf) LJ_TRY(dev_alloc(&s.rdf, 256));

@@ -254,3 +254,30 @@ for N in [1, 400, 3071, 3072, 5003, 16384, 23039, 23040, 24001, 32767, 32768, 32
     rc, got = force_pass(L.lib().calculateNForcesNoAlloc, N)
     assert rc == 0 and got == force_pass(L.lib().calculateNForces, N)[1], (N, rc, got)
 """, env={"LJ_PAIR_ONCE_SPLIT": split} if split else {})
+
+
+def test_force_call_scratch_settles(so):
+    """calculateNForces on boxes of two sizes in turn allocates for each once; where the
+    pair-once sums find no room it takes the sliced pass, and later them again."""
+    hip_stub.run(so, """
+p, f = C.c_void_p(), C.c_void_p()
+L.lib().allocateArray(C.byref(p), 65536)
+L.lib().allocateArray(C.byref(f), 65536)
+rdf = np.zeros(256, np.int32)
+def call(N):
+    kernels()
+    n, r = stub.stub_mallocs(), stub.stub_refused()
+    L.lib().calculateNForces(p, f, None, N, 40., 1, rdf.ctypes.data, 0.02, 256, 1)
+    names = [k for k, _ in kernels()]
+    assert any("force" in k for k in names) and any("rdf" in k for k in names), N
+    return stub.stub_mallocs() - n, stub.stub_refused() - r, any("k_force_n3" in k for k in names)
+first = [call(N) for N in (30000, 40000, 400)]
+assert first[0][2] and not first[1][2]
+for N in (30000, 40000, 400) * 2:
+    assert call(N)[0] == 0, N
+L.lib().threadExit()
+stub.stub_refuse_above(50 << 20)  # 30000: 57 MB of entries
+assert call(30000)[1:] == (1, False)
+stub.stub_refuse_above(1 << 40)
+assert call(30000)[1:] == (0, True)
+""")
