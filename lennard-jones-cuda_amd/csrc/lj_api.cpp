@@ -577,7 +577,13 @@ int lj_create(const lj_config* cfg, lj_ctx** out)
       A(dev_alloc(&c->xs, N));
       A(dev_alloc(&c->xs2, N));
     }
-    A(dev_alloc(&c->part64, (size_t)c->plan64.S * c->plan64.Npad));
+    if (rc == LJ_OK && c->plan64.n3 &&
+        dev_alloc(&c->part64, (size_t)c->plan64.S * c->plan64.Npad) != LJ_OK) {
+      // no room for the slots of every group (2 GiB at N = 131072): the sliced pass
+      c->plan64 = make_force_plan(N, 0, 1);
+      dev_free(c->n3items);
+    }
+    if (!c->part64) A(dev_alloc(&c->part64, (size_t)c->plan64.S * c->plan64.Npad));
     A(dev_alloc(&c->wt64, force64_totals(c->plan64)));
   }
   if (rc == LJ_OK && hipEventCreate(&c->e0) != hipSuccess) A(fail(LJ_ERR_DEVICE, "hipEventCreate"));

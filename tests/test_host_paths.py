@@ -281,3 +281,31 @@ assert call(30000)[1:] == (1, False)
 stub.stub_refuse_above(1 << 40)
 assert call(30000)[1:] == (0, True)
 """)
+
+
+def test_fp64_context_without_room_for_pair_once(so):
+    """The FP64 mode's slots of every pair once take 2 GiB at N = 131072; a device with
+    less room serves the size with the sliced pass."""
+    hip_stub.run(so, """
+def passes(**kw):
+    with ljamd.LJSystem(131072, 0.3, 1.0, precision=ljamd.PREC_FP64, **kw) as s:
+        kernels()
+        s.Integrate(0.002, 2)
+        s.CalculateForces()
+        return [k for k in kernels() if "k_force64" in k[0]]
+once = passes()
+assert once and all("k_force64_n3" in n for n, _ in once)
+assert stub.stub_live() == 0
+stub.stub_refuse_above(1 << 30)
+sliced = passes()
+assert stub.stub_refused() == 1
+stub.stub_refuse_above(1 << 40)
+assert sliced and not any("n3" in n for n, _ in sliced) and len(sliced) == len(once)
+stub.stub_refuse_above(1 << 20)
+try:
+    passes()
+    assert False
+except ljamd.LJError:
+    pass
+assert stub.stub_live() == 0
+""")
