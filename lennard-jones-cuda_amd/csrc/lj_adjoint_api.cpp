@@ -61,7 +61,7 @@ struct AdjState {
   hipGraph_t graph_k = nullptr, graph_seg = nullptr;
   hipGraphExec_t gexec_k = nullptr, gexec_seg = nullptr;
   int g_k = 0;
-  std::vector<hipEvent_t> ev;  // of a gradient's timing: four, then two per segment
+  std::vector<hipEvent_t> ev;  // of a gradient's timing: three, then two per segment
 };
 
 namespace {
@@ -499,7 +499,10 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
   AdjState* a = c->adj;
   const int N = c->cfg.N;
   hipStream_t st = c->stream;
-  while (a->ev.size() < (size_t)4 + 2 * ncheck) {
+  // timed only where the caller asks; the segments take turns with kSegEvents pairs
+  constexpr int kSegEvents = 32;
+  const bool timed = times_ms3 != nullptr;
+  while (timed && a->ev.size() < (size_t)3 + 2 * std::min(ncheck, kSegEvents)) {
     hipEvent_t e = nullptr;
     LJ_HIP(hipEventCreate(&e));
     a->ev.push_back(e);
@@ -511,8 +514,14 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
       rc = fail(LJ_ERR_DEVICE, "lj_trajectory_grad: %s", hipGetErrorString(e));
     return rc == LJ_OK;
   };
-  if (check(hipEventRecord(ev[0], st)) && (rc = forward(c, dt, M, k, p_target, w_p, out3)) == LJ_OK &&
-      check(hipEventRecord(ev[1], st))) {
+  const auto mark = [&](int e) { return !timed || check(hipEventRecord(ev[e], st)); };
+  float recompute_ms = 0.f;
+  const auto add_segment = [&](int e) {  // the pair at e, recorded
+    float ms = 0.f;
+    if (check(hipEventSynchronize(ev[e + 1])) && check(hipEventElapsedTime(&ms, ev[e], ev[e + 1])))
+      recompute_ms += ms;
+  };
+  if (mark(0) && (rc = forward(c, dt, M, k, p_target, w_p, out3)) == LJ_OK && mark(1)) {
     const double vol = std::pow(c->L, 3.);
     const double cP = 2. * w_p * (out3[2] - p_target);
     const double invM = 1. / M;
@@ -531,7 +540,9 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
       const int s0 = cseg * k, s1 = std::min(M, s0 + k);
       // recompute the segment's states s0+1..s1 from its checkpoint (the
       // one-launch forward run left those of the last segment)
-      if (!check(hipEventRecord(ev[4 + 2 * cseg], st))) break;
+      const int e = 3 + 2 * (cseg % kSegEvents);
+      if (timed && cseg + kSegEvents < ncheck) add_segment(e);  // of segment cseg + kSegEvents
+      if (!mark(e)) break;
       const double4* ckp = a->ck + (size_t)3 * cseg * N;
       if (!(a->T && cseg == ncheck - 1)) {
         if ((rc = dcopy(c, a->xd, ckp, 3))) break;
@@ -546,7 +557,7 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
           }
         }
       }
-      if (rc || !check(hipEventRecord(ev[5 + 2 * cseg], st))) break;
+      if (rc || !mark(e + 1)) break;
       // state m of the segment: positions, then velocities
       const auto state = [&](int m) { return m == s0 ? ckp : a->seg + (size_t)2 * (m - s0) * N; };
       // reverse over m = s1 .. s0+1 (and m = 0 in the first segment)
@@ -610,7 +621,7 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
       check(launch_adj_finalize(st, a->rowacc, nrow, make_adj_scales(c->ps), a->scal, fin));
     }
   }
-  if (rc == LJ_OK && check(hipEventRecord(ev[3], st)) &&
+  if (rc == LJ_OK && mark(2) &&
       check(hipMemcpyAsync(grad_eps_sigma, a->theta, 2 * sizeof(double), hipMemcpyDeviceToHost, st))) {
     if (dx0_host4 || d_dx0_4) {
       check(launch_adj_narrow(st, a->dx0, N, a->dxf));
@@ -619,15 +630,11 @@ int lj_trajectory_grad(lj_ctx* c, double dt, int nsteps, int checkpoint_every, d
       if (d_dx0_4)
         check(hipMemcpyAsync(d_dx0_4, a->dxf, sizeof(float4) * N, hipMemcpyDeviceToDevice, st));
     }
-    if (check(hipStreamSynchronize(st)) && times_ms3) {
-      float f_ms = 0.f, all_ms = 0.f, recompute_ms = 0.f;
-      for (int g = 0; g < ncheck; ++g) {
-        float ms = 0.f;
-        check(hipEventElapsedTime(&ms, ev[4 + 2 * g], ev[5 + 2 * g]));
-        recompute_ms += ms;
-      }
+    if (check(hipStreamSynchronize(st)) && timed) {
+      float f_ms = 0.f, all_ms = 0.f;
+      for (int g = 0; g < std::min(ncheck, kSegEvents); ++g) add_segment(3 + 2 * g);
       check(hipEventElapsedTime(&f_ms, ev[0], ev[1]));
-      check(hipEventElapsedTime(&all_ms, ev[1], ev[3]));
+      check(hipEventElapsedTime(&all_ms, ev[1], ev[2]));
       times_ms3[0] = f_ms;
       times_ms3[1] = recompute_ms;
       times_ms3[2] = all_ms - recompute_ms;

@@ -309,3 +309,25 @@ except ljamd.LJError:
     pass
 assert stub.stub_live() == 0
 """)
+
+
+def test_gradient_timing_events(so):
+    """The gradient's timing takes a bounded number of events however many segments the
+    sweep has, none where no times are asked for, and still covers every segment (one
+    launch of the stub is a microsecond: a one-step segment's recomputation takes two,
+    the last segment's none)."""
+    hip_stub.run(so, """
+s = ljamd.LJSystem(400, 0.5, 1.0)
+out, g = np.zeros(3), np.zeros(2)
+before = stub.stub_events()
+assert L.lib().lj_trajectory_grad(s.h, 0.005, 600, 1, 1.0, 1.0, out.ctypes.data, g.ctypes.data,
+                                  None, None, None) == 0
+assert stub.stub_events() == before
+for M in (1, 31, 32, 33, 600):
+    times = s.trajectory_grad(0.005, M, 1)[3]
+    assert stub.stub_events() - before <= 67
+    assert abs(times[1] - 2e-3 * (M - 1)) < 1e-6 * M, (M, times)
+    assert times[0] >= 1e-3 * M and times[2] >= 1e-3 * M, (M, times)
+s.close()
+assert stub.stub_events() == 0
+""")
