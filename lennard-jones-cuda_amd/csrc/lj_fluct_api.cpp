@@ -144,6 +144,7 @@ int lj_set_step_sampling(lj_ctx* c, const lj_step_sampling* s)
     a.end = rule == LJ_RDF_REF_GPU ? e[nbins - 1] : e[nbins];
     a.sampling = 1;
     LJ_TRY(attach_rdf_workspace(c, a));
+    c->rdf_cells.step_void = false;  // of the old sampling
     a.hist = c->rdf_step;
     LJ_HIP(launch_fill_u64(st, c->rdf_step, nbins));
     LJ_HIP(hipStreamSynchronize(st));
@@ -170,9 +171,10 @@ int lj_step_rdf_counts(lj_ctx* c, uint64_t* counts, int64_t* nsamples, int clear
     LJ_HIP(hipMemcpyAsync(&bad, c->smp_args.cells->result_step, sizeof(unsigned),
                           hipMemcpyDeviceToHost, st));
   LJ_HIP(hipStreamSynchronize(st));
-  if (bad) {
-    LJ_HIP(hipMemsetAsync(c->smp_args.cells->result_step, 0, sizeof(unsigned), st));
+  if (bad || c->rdf_cells.step_void) {
+    if (bad) LJ_HIP(hipMemsetAsync(c->smp_args.cells->result_step, 0, sizeof(unsigned), st));
     LJ_HIP(hipStreamSynchronize(st));
+    c->rdf_cells.step_void = false;
     return fail(LJ_ERR_STATE, "lj_step_rdf_counts: particle coordinates left [-L, 2L) during the "
                               "sampled steps; the step RDF is incomplete");
   }

@@ -228,6 +228,7 @@ struct RdfCellsWs {
   unsigned* flag = nullptr;        // coordinates beyond [-L, 2 L) in the current pass
   unsigned* result = nullptr;      // a flagged lj_rdf pass, for the host
   unsigned* result_step = nullptr; // a flagged pass of the per-step sampling, for the host
+  bool step_void = false;          // the same in arrays that have been replaced since
   int* bcnt = nullptr;             // [cap_m]: each block's offset within each cell, block-major
   int cap_n = 0, cap_cells = 0, cap_bins = 0, cap_m = 0;
 };

@@ -774,6 +774,13 @@ int rdf_cells_ensure(RdfCellsWs& w, int N, int ncell, int nbins, hipStream_t st,
   // that stream: a device-wide wait can break another thread's capture)
   if (hipStreamSynchronize(st) != hipSuccess)
     return fail(LJ_ERR_DEVICE, "rdf_cells_ensure: synchronizing the stream failed");
+  if (w.flag) {  // a flagged pass of the sampling is still to be told
+    unsigned v = 0u;
+    if (hipMemcpyAsync(&v, w.result_step, sizeof(v), hipMemcpyDeviceToHost, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess)
+      return fail(LJ_ERR_DEVICE, "rdf_cells_ensure: reading the flag failed");
+    w.step_void |= v != 0u;
+  }
   // grown to at least the old capacities, so that alternating layouts settle
   const int cn = std::max(N, w.cap_n), cc = std::max(ncell, w.cap_cells), cb = std::max(nbins, w.cap_bins);
   rdf_cells_free(w);

@@ -241,6 +241,30 @@ def test_step_rdf_out_of_span_reported_after_lj_rdf():
         assert n == 2 and counts.sum() == 2 * N * (N - 1)
 
 
+def test_step_rdf_out_of_span_reported_after_growth():
+    """The same when the lj_rdf call in between replaces the cell lists, with which the
+    sampled step's flag lay."""
+    N, rho = 9000, 0.85
+    L, pos, vel = perturbed_state(N, rho, 1.0, seed=8)
+    p = pos.reshape(-1, 4).copy()
+    p[17, 0] += np.float32(3.0 * L)
+    dr2 = ORC.orc_rdf_dr2(N)
+    with ljamd.LJSystem(N, rho, 1.0, canonical=ljamd.TVN) as s:
+        s.set_state(p.reshape(-1), vel)
+        s.CalculateForces()
+        s.set_step_sampling(rdf=ljamd.SAMPLE_RDF_SUM, rdf_rule=ljamd.RDF_REF_GPU, rdf_nbins=256)
+        s.Integrate(0.005, 1)
+        s.set_state(pos, vel)
+        got = s.rdf(ljamd.RDF_REF_GPU, 1000, dr2=dr2 * 256 / 1000)  # more bins: larger lists
+        assert got.sum() == N * (N - 1)
+        with pytest.raises(ljamd.LJError):
+            s.step_rdf_counts()
+        s.step_rdf_counts(clear=True)  # the flag was reported once
+        s.Integrate(0.005, 2)
+        counts, n = s.step_rdf_counts()
+        assert n == 2 and counts.sum() == 2 * N * (N - 1)
+
+
 def test_rdf_cells_crowded_cells_equal_all_pairs_pass(tmp_path):
     """Cells holding more particles than a workgroup has lanes: N = 70000,
     1024 bins of dr2 = 0.18 (range r^2 < 184), 3 cells per axis at reach 1
