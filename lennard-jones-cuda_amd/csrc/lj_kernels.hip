@@ -882,20 +882,15 @@ __global__ __launch_bounds__(kBlock)
         for (int b0 = 0; b0 < 32; b0 += B) {
           int kk[B];
           bool dec[B], gone[B];
-          if constexpr (TAB) {
-            float lo[B], hi[B];
-            float2 t[B];
+          float lo[B], hi[B];
+          float2 t[B];
 #pragma unroll
-            for (int b = 0; b < B; ++b) {
-              cl.measure(rdf_r2q(qi, qj_s[c0 + b0 + b]), kk[b], lo[b], hi[b]);
-              t[b] = T2[kk[b]];
-            }
-#pragma unroll
-            for (int b = 0; b < B; ++b) cl.decide(kk[b], lo[b], hi[b], t[b], dec[b], gone[b]);
-          } else {
-#pragma unroll
-            for (int b = 0; b < B; ++b) cl.rbins(rdf_r2q(qi, qj_s[c0 + b0 + b]), kk[b], dec[b], gone[b]);
+          for (int b = 0; b < B; ++b) {
+            cl.measure(rdf_r2q(qi, qj_s[c0 + b0 + b]), kk[b], lo[b], hi[b]);
+            t[b] = T2[kk[b]];
           }
+#pragma unroll
+          for (int b = 0; b < B; ++b) cl.decide(kk[b], lo[b], hi[b], t[b], dec[b], gone[b]);
 #pragma unroll
           for (int b = 0; b < B; ++b) {
             const int jj = c0 + b0 + b;
