@@ -112,22 +112,24 @@ def test_excluded_pairs_every_pair_once(N, periodic):
     assert np.array_equal(got.astype(np.int64), exp)
 
 
+@pytest.mark.parametrize("axis", [0, 1, 2])
 @pytest.mark.parametrize("N", [600, 3500, 8192])
-def test_exact_ties(N):
-    """Particles on the two planes x = 0 and x = L/2: the x separation of a pair
-    is 0 or exactly half the box, so F_x comes from the ties alone, each particle
-    drawn towards the image that rounding half away from zero picks (+L/2 for the
-    lower x, MDSystem.cu:31-33).  All terms of a particle's sum have the same
+def test_exact_ties(N, axis):
+    """Particles on the two planes x = 0 and x = L/2 (or of y, of z): the x
+    separation of a pair is 0 or exactly half the box, so F_x comes from the ties
+    alone, each particle drawn towards the image that rounding half away from zero
+    picks (+L/2 for the lower x, MDSystem.cu:31-33).  All terms of a particle's sum have the same
     sign, N/2 of them in float sums of at most 128: 1e-5 relative."""
     L = 16.0
     rng = np.random.default_rng(5)
     p = np.zeros((N, 4), np.float32)
     up = rng.permutation(N) % 2 == 1
-    p[:, 0] = np.where(up, L / 2, 0.0)
+    others = [a for a in range(3) if a != axis]
+    p[:, axis] = np.where(up, L / 2, 0.0)
     k = int(np.ceil(np.sqrt(N)))
     g = rng.permutation(k * k)[:N]
-    p[:, 1] = (g // k + 0.5 + 0.3 * rng.uniform(-1, 1, N)) * (L / k)
-    p[:, 2] = (g % k + 0.5 + 0.3 * rng.uniform(-1, 1, N)) * (L / k)
+    p[:, others[0]] = (g // k + 0.5 + 0.3 * rng.uniform(-1, 1, N)) * (L / k)
+    p[:, others[1]] = (g % k + 0.5 + 0.3 * rng.uniform(-1, 1, N)) * (L / k)
     arr = ljamd.CompatArrays(N)
     f, _, _ = arr.calculate(p.reshape(-1), L, True, 0.1)
     arr.close()
@@ -135,8 +137,35 @@ def test_exact_ties(N):
     F = np.zeros(N)
     for i in range(N):
         o = up != up[i]
-        d = q[i, 1:3] - q[o, 1:3]
+        d = q[i, others] - q[o][:, others]
         d -= L * np.round(d / L)
         r2 = (L / 2) ** 2 + np.sum(d * d, axis=1)
         F[i] = (1.0 if not up[i] else -1.0) * np.sum(24.0 * (2.0 / r2 ** 7 - 1.0 / r2 ** 4)) * (L / 2)
-    assert np.max(np.abs(f.reshape(N, 4)[:, 0] - F) / np.abs(F)) <= 1e-5
+    assert np.max(np.abs(f.reshape(N, 4)[:, axis] - F) / np.abs(F)) <= 1e-5
+
+
+@pytest.mark.parametrize("N", [1000, 3072, 5003])
+def test_coordinate_that_is_no_number(N):
+    """A hard-wall box with one NaN coordinate: r^2 of its particle's pairs is not
+    comparable, so they are left out like those at r^2 <= 1e-6, whichever pass finds
+    them (its least r^2 does not show them, its sums do).  Only the axis of the NaN
+    has no force, since NaN times a factor of 0 is NaN; the others, the energies and
+    the pressure are those of the box without the particle (the bounds are the
+    other tests')."""
+    L, pos, _ = perturbed_state(N, 0.3, 1.0, seed=81)
+    k = N - 70
+    p = pos.reshape(N, 4).copy()
+    p[k, 0] = np.nan
+    arr = ljamd.CompatArrays(N)
+    f, pr, _ = arr.calculate(p.reshape(-1), L, False, 0.1)
+    arr.close()
+    rest = np.arange(N) != k
+    F64, ew, E, W = forces_fp64(p[rest].reshape(-1), float(np.float32(L)), False, skip_r2=1e-6)
+    f = f.reshape(N, 4)
+    assert np.all(np.isnan(f[:, 0])) and not np.any(f[k, 1:])
+    got, exp = xyz(f[rest]), np.asarray(F64)[:, :3].copy()
+    got[:, 0] = exp[:, 0] = 0.0
+    err = force_errors(got, exp)
+    assert err["global_rel"] <= 2e-6 and err["max_rel_floor"] <= 1e-5, err
+    assert np.max(np.abs(f[rest, 3] - ew[:, 0]) / np.maximum(np.abs(ew[:, 0]), 1.0)) <= 1e-5
+    assert abs(pr - W / 3.0) <= 1e-5 * max(abs(W / 3.0), 1e-3)

@@ -71,3 +71,48 @@ def test_autotune_keeps_the_one_launch_step():
             out.append((*a, h, b.stats(), b.get_array(ljamd.ARRAY_POS), b.get_array(ljamd.ARRAY_VEL)))
     for x, y in zip(*out):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("n,steps", [([10007, 300, 5003, 1], 8), ([40001], 2)])
+@pytest.mark.parametrize("canon", [ljamd.EVN, ljamd.TVN])
+def test_large_boxes_untuned(canon, n, steps):
+    """Boxes well above the sizes a single box takes in one launch, against the
+    sliced tuning, with the bounds of the small boxes.  (A single particle's seeded
+    velocity, without its mean and scaled to T, is no number: alike on both sides.)"""
+    def gap(x, y):
+        no = np.isnan(x)
+        assert np.array_equal(no, np.isnan(y))
+        return np.max(np.abs(np.where(no, 0.0, x - y)))
+
+    n = np.array(n, np.int32)
+    print(f"\n[case] large untuned batch {n} canon={canon}", flush=True)
+    out = []
+    for tuning in (None, (1, 512, 4, 0)):
+        with ljamd.LJBatch(n, np.full(n.size, 0.6), np.full(n.size, 1.2), canonical=canon, seed=33) as b:
+            if tuning:
+                b.set_tuning(*tuning)
+            h = b.integrate_hist(0.004, steps)
+            out.append((h, *[[b.get_array(a, box=k) for k in range(n.size)]
+                             for a in (ljamd.ARRAY_POS, ljamd.ARRAY_VEL)]))
+    (h, p, v), (hs, ps, vs) = out
+    for k in range(n.size):
+        assert np.any(np.isnan(h[:, k])) == (n[k] == 1)
+        assert gap(h[:, k, 0], hs[:, k, 0]) / n[k] <= 2e-5, k
+        assert gap(xyz(p[k]), xyz(ps[k])) <= 4e-5, k
+        assert gap(xyz(v[k]), xyz(vs[k])) <= 1e-3, k
+
+
+def test_many_small_boxes_untuned():
+    """2000 boxes of 200, beyond the one-launch step's sizes: the default tiling's
+    step, whose bits do not depend on how its items are handed out."""
+    n = np.full(2000, 200, np.int32)
+    out = []
+    for tuning in (None, (1, 512, 4, 0)):
+        with ljamd.LJBatch(n, np.full(2000, 0.5), np.full(2000, 1.0), seed=34) as b:
+            if tuning:
+                b.set_tuning(*tuning)
+            h = b.integrate_hist(0.004, 9)
+            out.append((h, b.get_array(ljamd.ARRAY_POS), b.get_array(ljamd.ARRAY_VEL),
+                        b.get_array(ljamd.ARRAY_FORCE)))
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
