@@ -102,8 +102,8 @@ void calculateNForces(float* Pos, float* Force, float* host_pressure, int numBod
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments, results and synchronous behaviour as calculateNForces, with
  * the same kernels (bit-identical results), but every device scratch buffer
- * lives in a file-scope device array of 12.3 MiB that each GPU the library
- * runs on holds until the process ends; no hipMalloc, hipFree or stream
+ * lives in a file-scope device array of 81.5 MiB, which a GPU holds from the
+ * process's first such call on it until the process ends; no hipMalloc, hipFree or stream
  * creation.  Runs on the null stream.  numBodies <= 65536.  Returns LJ_OK or
  * a negative status (message in lj_last_error()).  The array is shared by
  * every call on a GPU and keeps the last call's contents: calls overlapping

@@ -1181,12 +1181,11 @@ bool n3_eligible(int N)
   // LJ_PAIR_ONCE=0 / 1 turns the kernel off / on at any size (tuning)
   const char* e = std::getenv("LJ_PAIR_ONCE");
   if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1' && N >= 256;
-  // measured against the sliced kernel (TVN step at rho* = 0.85, us per step,
-  // with split items): N = 2560 19.2 vs 21.4, 3072 19.3 vs 22.6, 4096 21.2 vs
-  // 25.1, 6144 26.4 vs 36.8.  Below N = 3584 the pass itself is slower (one
-  // wave per SIMD: 10.9 against 9.4 us at 3072), the step faster for its
-  // fused observables; the threshold keeps single evaluations of small boxes
-  // on the sliced kernel
+  // Up to N = 4096 this decides single evaluations (steps are one launch there).
+  // Measured at rho* = 0.85, us, pair-once / sliced: lj_compute_forces N = 2048
+  // 38.8 / 38.4, 2560 41.0 / 42.1, 3072 42.6 / 44.4, 3584 43.2 / 48.1, 5003 50.0 /
+  // 57.8, most of it launches and the wait; the step's force pass 6.8 / 6.0 at 2560,
+  // 8.0 / 7.1 at 3072, 8.1 / 8.9 at 3584, 12.3 / 17.4 at 5003.
   return N >= 3072;
 }
 

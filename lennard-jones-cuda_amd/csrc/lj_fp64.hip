@@ -140,8 +140,9 @@ __global__ __launch_bounds__(kBlock) void k_force64(const double4* __restrict__ 
 // receives its i sums, slot g of one of group h its j sums.
 //   35 FP64 instructions and one v_rcp_f64 (four issue slots) per unordered pair of
 // a periodic box against 2 x 33 of the sliced pass; bound by their issue (N = 40000:
-// 912 us, 88% of the slots; 16384: 258 -> 175 us, where the last, partly filled
-// round of workgroups shows).  SPLIT: two workgroups per item, one j
+// 1671 -> 1046 us on one card, 912 on a faster one, 77 to 88% of the slots; 16384:
+// 301 -> 197 us, where the last, partly filled round of workgroups shows; 8000:
+// 75 -> 55).  SPLIT: two workgroups per item, one j
 // sub-tile of every wave each (2 ng slots), for sizes whose items leave most
 // SIMDs a wave or less.
 constexpr int kG64 = 256;
@@ -807,7 +808,8 @@ inline int nb(int n) { return (n + kBlock - 1) / kBlock; }
 }  // namespace
 
 // Pair-once from N = 4097 on, as long as its slots stay within 4 GiB (N about
-// 180,000); measured steps (EVN, periodic, us; sliced / pair-once): N = 3000 26.5 /
+// 180,000; a context that finds no room for them takes the sliced pass); measured
+// steps (EVN, periodic, us; sliced / pair-once): N = 3000 26.5 /
 // 24.1, 4000 31.0 / 32.5, 5000 42.0 / 35.9, 8000 77.9 / 62.2, 16384 273 / 190,
 // 131072 16900 / 10700.  Split while the items fit two rounds of the 1024 workgroups
 // that the kernel's registers let the device hold: their length is the granularity of the

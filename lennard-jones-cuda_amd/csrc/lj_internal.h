@@ -144,7 +144,7 @@ struct StepArgs {
   const double* ew;
   int nitems;
   // block rows of the step's sums (K2, TV2, E, B): one per kRowParticles
-  // particles in the FP32 step kernels, one per kBlock in the FP64 ones
+  // particles, in the one-launch steps one per tile
   int nrow;
   // one-launch steps of small boxes (lj_small.hip): the coordinates of the
   // next step's force pass, and whether Force.w receives e_i (else 0)
@@ -157,7 +157,7 @@ struct StepArgs {
 // of kLongGraphSteps first (N = 16384, TVN: 80.8 against 82.1 us per step).
 constexpr int kGraphSteps = 8;
 constexpr int kLongGraphSteps = 32;
-// particles per block row of the FP32 time-step kernels
+// particles per block row of the time-step kernels with a force pass of their own
 constexpr int kRowParticles = 64;
 inline int step_rows(int N) { return (N + kRowParticles - 1) / kRowParticles; }
 hipError_t launch_drift(hipStream_t st, const StepArgs& a);

@@ -512,7 +512,7 @@ __global__ void k_reset_averaging(lj_obs* obs)
 // (to a row of its own where the caller has rows, k_rdf_rows adds them up; else
 // by atomics).
 // One workgroup per pair of groups left a box of N = 400 to three workgroups
-// that walked 256 j each (36 us against 10), and at N = 16384 its 2080 histograms
+// that walked 256 j each (35 to 38 us by rule, here 10), and at N = 16384 its 2080 histograms
 // of 500 bins cost 1e6 atomics on 500 addresses.  Periodic boxes take k_rdf_fx,
 // which decides almost every pair from the fixed-point image with a proven error
 // bound and runs the reference arithmetic only near bin edges; the others

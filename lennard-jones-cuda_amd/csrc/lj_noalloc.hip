@@ -3,8 +3,9 @@
 //
 // All of its device scratch (fixed-point positions, the force pass's slice
 // partials, block rows, the RDF histogram and bin table, the pressure word)
-// sits in one file-scope device array, `scratch`, of kScratchBytes; each GPU
-// the library runs on holds its own copy until the process ends.  The call
+// sits in one file-scope device array, `scratch`, of kScratchBytes; a GPU holds
+// its own copy from the first call there (the runtime loads this file's code object
+// then: 82 MiB of free memory less) until the process ends.  The call
 // makes no hipMalloc / hipFree and creates no stream: it runs on the null
 // stream and returns when the results are on the host.  Every call on a GPU
 // shares that GPU's array, so calls that overlapped on one GPU would race: a

@@ -6,7 +6,7 @@
 // A step of a small box is a chain of latencies: at N = 400 its 80,000 pairs
 // are 0.05 us of the device's FP32 rate, an empty kernel in a chain of graph
 // nodes takes 1.8 us, and the force pass, kick and finaliser took 11.0 us.
-// Here the step is 4.3 us: the launch, one load of all coordinates, the pairs
+// Here the step is 4.6 us: the launch, one load of all coordinates, the pairs
 // of a lane, two passes through LDS and the stores.  From about N = 1500 on the
 // pair loop is visible, and at N = 4096 it is 9.4 us of the 14, which is the issue
 // time of its 22 slots per ordered pair.
