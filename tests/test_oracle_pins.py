@@ -84,6 +84,7 @@ def test_rdf_normalisation_matches_reference():
         R.close()
 
 
+@needs_ref
 def test_velocity_distribution_matches_reference():
     """initvelo / updatevelo of the reference (MDSystem.cpp:651-694) from the
     oracle's speed counts, bit for bit."""
